@@ -1,12 +1,12 @@
 // RTAMC2D transient solver on the GPU: one lane per particle history,
-// lanes refill from a global particle counter when their particle ends.
+// lanes refill from a particle counter when their particle ends.
 //
 // Reference: src/RTA_MC2D.cpp
-//   Init_generator (wall part)  272-533   -> init_particle()
+//   Init_generator (wall part)  272-533   -> rta_start()
 //   diffusive_bouncing::bounce  635-678   -> per-(side, mode) alias rows
 //   process_segment (transient) 699-769   -> tally_segment()
-//   evolparticle (transient)    990-1386  -> body of rta_history_kernel
-//   history loop                2228-2317 -> flight draw in the kernel
+//   evolparticle (transient)    990-1386  -> rta_fly(), rta_slow()
+//   history loop                2228-2317 -> rta_histories()
 //   post-processing             2326-2435 -> rta_postprocess()
 #include "runtime.hpp"
 #include <algorithm>
@@ -29,7 +29,7 @@ struct RtaGen {
 // box, generator and table indices are absolute in the batch's arrays.
 struct RtaRunDev {
     uint64_t first, count, seed;
-    int32_t gen0, ngen, gsel0, scat0;
+    int32_t gen0, ngen, gsel0, pad2;
     int32_t ballistic, gmask, pad0, pad1;  // gmask: sides whose specularity gets a gradient
     double wscale;                         // scattering-rate factor of the run
     float spec[4];                         // specular probability per side
@@ -43,11 +43,30 @@ struct RtaItem {
     int32_t lrows;       // the run's regular boxes
     int32_t lbins;       // leading time bins of each row held in LDS
     int32_t run;
+    int32_t box0, nbox, side0, nsides;  // the run's boxes and polygon sides
 };
 
+// One mode as the history kernels read it: 64 bytes in one cache line, so a
+// new mode costs one line (velocity, inverse velocity, rate and the range of
+// its diffuse-bounce table) instead of one line in each of three arrays.
+struct __align__(64) RtaMode {
+    double vx, vy, ivx, ivy, w;     // inverses are 0 where the component is 0
+    int32_t lo, len, base, pad[3];  // Lambert table: first partner, partners, offset
+};
+static_assert(sizeof(RtaMode) == 64, "one mode record is half a 128-byte line");
+
+// One box as the history kernels read it.
+struct __align__(16) RtaBox {
+    double xmin, xmax, ymin, ymax;
+    int32_t side_nbr[4];  // as DevBox
+    int32_t kind, lrow;  // lrow: LDS tally row of a regular box
+    int32_t s0, ns;      // polygon geometries: first side and sides
+};
+static_assert(sizeof(RtaBox) == 64, "box record");
+
 struct RtaParams {
-    const double4* modes;  // (vx, vy, w, omega)
-    const double2* ivel;   // (1/vx, 1/vy), 0 where the component is 0
+    const RtaMode* rmodes;
+    const RtaBox* rboxes;
     const int32_t* mirror; // [2][n]: partner with vx -> -vx (sides 0, 3), vy -> -vy (sides 1, 2)
     const uint2* scat;     // BE_derivative alias per run (n each)
     const DevBox* boxes;
@@ -61,11 +80,9 @@ struct RtaParams {
     const RtaGen* gens;
     const uint2* gen_sel;  // alias over each run's generators
     const uint2* gen_tab;  // per generator, n entries
-    const int4* lam_info;  // per mode: lo, len, base, 0
     const uint2* lam_tab;
     const int32_t* perm;   // omega-sorted position -> mode
     const double* timegrid;
-    const uint64_t* box_cell;  // first tally cell of each box (box-major, nt cells)
     const RtaRunDev* runs;
     double* gz;
     double* jx;
@@ -76,23 +93,24 @@ struct RtaParams {
     unsigned long long* counters;  // events, crossings, next id, stuck, bad mirror, bad translation
     uint64_t total;        // particles over all runs
     uint64_t cells;
-    unsigned long long max_iters;
     double maxtime;
     int32_t n, nt, nruns, pad;
-    // FP32 tallies in LDS (LT kernels): the LDS row (nt cells) of each box,
-    // ~0u for boxes that never tally; the global cell of each LDS row; per
-    // side the float offset of its score-weighted array, -1 for none. The
-    // LDS block holds 3 arrays (gz, jx, jy) of lrows * nt floats, then the
-    // gradient arrays.
-    const uint32_t* box_lrow;
+    // LDS tallies: the global cell of each LDS row (a regular box); the rows
+    // and their leading time bins held in LDS. Mode 1: lt_arrays FP32 arrays
+    // [lrows][lbins]: gz, jx, jy, then array lt_goff[s] of side s for each
+    // differentiated side (-1: none). Mode 2: FP64 gz, jx, jy; each workgroup
+    // writes its block to part[blockIdx.x] at the end.
     const uint64_t* lrow_cell;
-    int32_t lrows, pad1;
-    int32_t lt_goff[4];
-    // tally mode 2: the LDS holds FP64 gz, jx, jy of the first lbins time
-    // bins of every LDS row ([3][lrows][lbins]); each workgroup writes its
-    // block to part[blockIdx.x] at the end
-    int32_t lbins, pad2;
+    int32_t lrows, lbins;
+    int32_t lt_goff[4], lt_arrays;
     double* part;
+    // geometry in LDS (GL kernels): boxes and sides of the batch (modes 0 to
+    // 2), the byte offsets of the sides and the time grid after the boxes and
+    // of the tallies after both
+    int32_t nboxes, nsides, geo_side, geo_grid, geo_bytes;
+    int32_t lanes;  // lanes of a wave that follow histories
+    int32_t chunk;  // particle ids a wave takes at a time
+    int32_t mig, keep_waves;  // LDS offset of the mailbox (-1: none); waves that keep their histories
     double idt;  // nt / maxtime: time -> bin estimate on the uniform grid
     // tally mode 3: the work items, taken in order through counters[6]
     const RtaItem* items;
@@ -105,154 +123,239 @@ struct RtaParams {
 #define RTA_NCOPY 8
 // the XCD (XCC) this wave runs on, from the hardware register HW_REG_XCC_ID
 
-// get_bin_index (RTA_MC2D.cpp:140-148): lower_bound - 1 clamped to
-// [0, nt-1]. The grid is uniform (t_i = i maxtime / nt), so the bin is
-// estimated from target * nt / maxtime and corrected against the grid
-// values themselves, which keeps lower_bound's result exactly (a target
-// on a grid point t_j belongs to bin j - 1).
-__device__ inline int time_bin(const double* grid, int nt, double idt, double target) {
-    const double e = target * idt;
-    int k = e < 0. ? 0 : (e > (double)nt ? nt : (int)e);
-    while (k > 0 && grid[k] >= target) k--;
-    while (k < nt && grid[k + 1] < target) k++;
-    return k > nt - 1 ? nt - 1 : k;
+// Boxes, polygon sides and the time grid of the history kernels: in LDS (GL)
+// when they take at most RTA_GEO_LDS bytes, else in global memory. Every
+// lane of a wave reads its own box, side and time bin, and such a scattered
+// load occupies the vector memory pipe for one cycle per lane: with the
+// geometry, the grid and the mode record read from global memory for every
+// segment, 57 loads per wave and segment kept that pipe busy all the time
+// (16 runs of 3000 modes, 5.5e6 particles: 68 ms). LDS serves them 128 bytes a
+// cycle. A box takes 80 bytes of LDS: a stride of 20 banks starts 16
+// consecutive boxes at 16 different 16-byte groups, where 64 bytes would put
+// them on four.
+#define RTA_GEO_LDS 20480
+#define RTA_BOX_LDS 80
+template <bool GL>
+struct RtaGeo {
+    const unsigned char* box;
+    const DevSide* side;
+    const double* grid;
+    int32_t bo;      // tally mode 3: first box of the run (staged indices are local)
+    int32_t run;     // tally mode 3: the run of every lane, and its rate factor
+    double wscale;
+    __device__ inline RtaBox at(int i) const {
+        return *reinterpret_cast<const RtaBox*>(box + (size_t)i * (GL ? RTA_BOX_LDS : sizeof(RtaBox)));
+    }
+};
+
+// Copies nb boxes from bo on and ns sides from so on (with local indices) and
+// the time grid into LDS. The caller synchronises.
+template <bool POLY>
+__device__ inline void rta_stage_boxes(const RtaParams& P, unsigned char* lds, int bo, int nb, int so, int ns, int lrow0) {
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        RtaBox b = P.rboxes[bo + i];
+        for (int k = 0; k < 4; k++)
+            if (b.side_nbr[k] >= 0) b.side_nbr[k] -= bo;
+        b.lrow -= lrow0;
+        b.s0 -= so;
+        *reinterpret_cast<RtaBox*>(lds + (size_t)i * RTA_BOX_LDS) = b;
+    }
+    if constexpr (POLY) {
+        DevSide* S = reinterpret_cast<DevSide*>(lds + P.geo_side);
+        for (int i = threadIdx.x; i < ns; i += blockDim.x) {
+            DevSide s = P.sides[so + i];
+            if (s.nbr >= 0) s.nbr -= bo;
+            S[i] = s;
+        }
+    }
 }
+__device__ inline void rta_stage_grid(const RtaParams& P, unsigned char* lds) {
+    double* g = reinterpret_cast<double*>(lds + P.geo_grid);
+    for (int i = threadIdx.x; i <= P.nt; i += blockDim.x) g[i] = P.timegrid[i];
+}
+
+// get_bin_index (RTA_MC2D.cpp:140-148): lower_bound - 1 clamped to
+// [0, nt-1], of a time target >= 0. The grid is uniform (t_i = i maxtime /
+// nt), so the bin is estimated from target * nt / maxtime and corrected
+// against the grid values themselves, which keeps lower_bound's result
+// exactly (a target on a grid point t_j belongs to bin j - 1). upper: the
+// bin's upper grid value.
+__device__ inline int time_bin(const double* grid, int nt, double idt, double target, double& upper) {
+    int k = min((int)fmin(target * idt, 2.0e9), nt - 1);
+    double lower = grid[k];
+    upper = grid[k + 1];
+    while (k > 0 && lower >= target) {
+        k--;
+        upper = lower;
+        lower = grid[k];
+    }
+    while (k < nt - 1 && upper < target) {
+        k++;
+        upper = grid[k + 1];
+    }
+    return k;
+}
+
+// Where a workgroup's tallies go. Cells are numbered by one key: keys below
+// lc are cells of the LDS block (row * lbins + bin), the others lc + the
+// cell of the XCD's copy (box * nt + bin, boxes from the first box of the
+// tallied range on).
+struct RtaTally {
+    void* lds;           // FP64 [3][rows][lbins] (modes 2, 3) or FP32 arrays (mode 1)
+    uint32_t lbins, lc;  // time bins of a row held in LDS; rows * lbins
+    int32_t row0;        // box records' row of the block's first row
+    double* g;           // gz of the XCD's copy at cell 0 of the tallied range
+    double* dg;          // score-weighted gz of side 0 there (gradient runs)
+};
 
 // A lane's running sum of consecutive contributions to one tally cell
 // (box, time bin); it is added to the tallies when the lane's next
 // contribution falls in another cell and when the lane's histories end.
 // Successive segments of a history often share a cell (several flights in
 // one box within one time bin), and each cell update costs three adds.
+template <bool D>
 struct TallyAcc {
-    int box = -1, bin = 0;
+    uint32_t key = ~0u;
     double g = 0., x = 0., y = 0.;
+    double d[D ? 4 : 1] = {};  // score-weighted sums per side
 };
 
-// Adds the accumulator into the tallies: under tally mode 2 the first
-// lbins time bins of a box go to the workgroup's FP64 LDS block, later
-// bins (and every bin under mode 0) to the XCD's copy by device atomics.
-template <int TM>
-__device__ inline void acc_flush(const RtaParams& P, double* L, TallyAcc& a) {
-    if (a.box < 0) return;
-    // mode 3: the block holds [3][lrows][lbins] of the current item's run,
-    // after a header of ints (lrows, lbins, first global row)
-    const int* hd = reinterpret_cast<const int*>(L) - 4;
-    if (TM == 3 && a.bin < hd[1]) {
-        const uint32_t lc = (uint32_t)hd[0] * (uint32_t)hd[1];
-        const uint32_t i = (P.box_lrow[a.box] - (uint32_t)hd[2]) * (uint32_t)hd[1] + (uint32_t)a.bin;
-        atomicAdd(L + i, a.g);
-        atomicAdd(L + lc + i, a.x);
-        atomicAdd(L + 2 * lc + i, a.y);
-    } else if (TM == 2 && a.bin < P.lbins) {
-        const uint32_t lc = (uint32_t)P.lrows * (uint32_t)P.lbins;
-        const uint32_t i = P.box_lrow[a.box] * (uint32_t)P.lbins + (uint32_t)a.bin;
-        atomicAdd(L + i, a.g);
-        atomicAdd(L + lc + i, a.x);
-        atomicAdd(L + 2 * lc + i, a.y);
+// Adds the accumulator into the tallies: an LDS cell under modes 2 and 3,
+// else the XCD's copy by device atomics.
+template <int TM, bool D>
+__device__ inline void acc_flush(const RtaParams& P, const RtaTally& T, TallyAcc<D>& a) {
+    if (a.key == ~0u) return;
+    if ((TM == 2 || TM == 3) && a.key < T.lc) {
+        // an LDS pointer by type: with generic ones the compiler merges the
+        // tails of both branches into flat atomics
+        auto* L = (__attribute__((address_space(3))) double*)T.lds + a.key;
+        __builtin_amdgcn_ds_atomic_fadd_f64(L, a.g);
+        __builtin_amdgcn_ds_atomic_fadd_f64(L + T.lc, a.x);
+        __builtin_amdgcn_ds_atomic_fadd_f64(L + 2 * T.lc, a.y);
     } else {
-        const uint64_t k = P.box_cell[a.box] + (uint64_t)a.bin + (uint64_t)(xcd_id() % RTA_NCOPY) * 3 * P.cells;
-        atomicAdd(P.gz + k, a.g);
-        atomicAdd(P.jx + k, a.x);
-        atomicAdd(P.jy + k, a.y);
+        const uint64_t k = a.key - T.lc;
+        atomicAdd(T.g + k, a.g);
+        atomicAdd(T.g + P.cells + k, a.x);
+        atomicAdd(T.g + 2 * P.cells + k, a.y);
+        if constexpr (D) {
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                if (a.d[s] != 0.) atomicAdd(T.dg + (uint64_t)s * P.cells + k, a.d[s]);
+        }
     }
-    a.box = -1;
+    a.key = ~0u;
 }
 
-// process_segment (RTA_MC2D.cpp:699-769); gradient runs also add the
-// segment weighted by the particle's running score for each active side.
+// State of a lane. FRESH draws a flight and then flies; FLY continues one
+// across boxes; the pending states wait for rta_slow; DEAD waits for the
+// next particle id; DONE has none left.
+enum { RTA_DEAD = 0, RTA_FRESH = 1, RTA_FLY = 2, RTA_WALL = 3, RTA_MIXED = 4, RTA_TRANS = 5, RTA_DONE = 6 };
+
+// The state of one particle history between events.
+struct RtaState {
+    Pcg32 rng;
+    uint64_t look;             // generator state after the look-ahead draws
+    double x, y, t, dtrem;
+    double vx, vy, ivx, ivy;   // of the mode in flight
+    uint2 se;                  // look-ahead alias entry of the next scattering
+    uint32_t sk, su, budget;
+    int mode, box, still, bin, st, aux;  // aux: side (WALL) or side mask (MIXED)
+    int run;                   // modes 0 to 2: the lane's run and its rate factor
+    double wscale;
+    int sign, ballistic, gmask;
+    float score[4];
+};
+
+struct RtaCounts {
+    uint32_t events = 0, crossings = 0;
+};
+
+// Adds a segment's contribution c to time bin i of the lane's box (lrow: its
+// LDS row); gradient runs also add it weighted by the particle's running
+// score for each active side.
 // TM (tally mode) 0: FP64 device atomics. 1: the workgroup's FP32 partial
-// sums in LDS (lds), added into the FP64 tallies once at the end of the
-// kernel (lt_flush). 2: the workgroup's FP64 partial sums of gz, jx and jy
-// for the first lbins time bins in LDS, later bins by device atomics.
-// 3: as 2 with the LDS block holding only the rows of the run of the
-// workgroup's current work item. Modes 0 (without dT/dp), 2 and 3 merge
-// consecutive contributions to one cell in the lane's accumulator.
-template <bool GRAD, int TM>
-__device__ inline void tally_segment(const RtaParams& P, void* lds, TallyAcc& acc, int box, double t0, double t1,
-                                     int sign, double vx, double vy, int gmask, const float* score, int mode) {
-    int b0 = time_bin(P.timegrid, P.nt, P.idt, t0), b1 = time_bin(P.timegrid, P.nt, P.idt, t1);
-    double delta = t1 - t0;
-    if constexpr (TM == 2 || TM == 3 || (TM == 0 && !GRAD)) {
-        // spectral locations tally per mode; the Gamma-broadened spectra are
-        // one matrix product after the run (the reference adds the broadened
-        // weights of every segment, RTA_MC2D.cpp:718-766)
-        double* sp = nullptr;
-        if (TM == 0 && P.spec) {
-            const int l = P.box_loc[box];
-            if (l >= 0) sp = P.spec + (size_t)l * P.nt * P.n + mode;
-        }
-        for (int i = b0; i <= b1; i++) {
-            double lo = fmax(P.timegrid[i] - t0, 0.);
-            double hi = fmin(P.timegrid[i + 1] - t0, delta);
-            double c = sign * fmax(hi - lo, 0.);
-            if (c == 0.) continue;
-            if (TM == 0 && sp) atomicAdd(sp + (size_t)i * P.n, c);
-            if (box == acc.box && i == acc.bin) {
-                acc.g += c;
-                acc.x += vx * c;
-                acc.y += vy * c;
-            } else {
-                acc_flush<TM>(P, (double*)lds, acc);
-                acc.box = box;
-                acc.bin = i;
-                acc.g = c;
-                acc.x = vx * c;
-                acc.y = vy * c;
-            }
-        }
-        return;
-    }
+// sums in LDS for the leading lbins bins, later ones by device atomics. 2: the
+// same with FP64 partial sums. 3: as 2 with the LDS block holding only the
+// rows of the run of the workgroup's current work item. All modes but 1
+// merge consecutive contributions to one cell in the lane's accumulator.
+template <bool GRAD, int TM, bool D>
+__device__ inline void tally_bin(const RtaParams& P, const RtaTally& T, TallyAcc<D>& A, const RtaState& S, int lrow,
+                                 double* spec, int i, double c) {
+    if (c == 0.) return;
+    const uint32_t row0 = (uint32_t)(lrow - T.row0) * T.lbins, cell0 = (uint32_t)S.box * (uint32_t)P.nt;
     if constexpr (TM == 1) {
-        float* lt = (float*)lds;
-        const uint32_t lc = (uint32_t)P.lrows * (uint32_t)P.nt;
-        float* L = lt + P.box_lrow[box] * (uint32_t)P.nt;
-        for (int i = b0; i <= b1; i++) {
-            double lo = fmax(P.timegrid[i] - t0, 0.);
-            double hi = fmin(P.timegrid[i + 1] - t0, delta);
-            double c = sign * fmax(hi - lo, 0.);
-            if (c == 0.) continue;
-            atomicAdd(L + i, (float)c);
-            atomicAdd(L + lc + i, (float)(vx * c));
-            atomicAdd(L + 2 * lc + i, (float)(vy * c));
+        if ((uint32_t)i < T.lbins) {
+            float* L = (float*)T.lds + row0 + i;
+            atomicAdd(L, (float)c);
+            atomicAdd(L + T.lc, (float)(S.vx * c));
+            atomicAdd(L + 2 * T.lc, (float)(S.vy * c));
             if (GRAD) {
 #pragma unroll
                 for (int s = 0; s < 4; s++)
-                    if (P.lt_goff[s] >= 0 && ((gmask >> s) & 1) && score[s] != 0.f)
-                        atomicAdd(L + P.lt_goff[s] + i, (float)(c * (double)score[s]));
+                    if (P.lt_goff[s] >= 0 && ((S.gmask >> s) & 1) && S.score[s] != 0.f)
+                        atomicAdd(L + (uint32_t)P.lt_goff[s] * T.lc, (float)(c * (double)S.score[s]));
+            }
+        } else {
+            const uint64_t k = cell0 + (uint32_t)i;
+            atomicAdd(T.g + k, c);
+            atomicAdd(T.g + P.cells + k, S.vx * c);
+            atomicAdd(T.g + 2 * P.cells + k, S.vy * c);
+            if (GRAD) {
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    if (((S.gmask >> s) & 1) && S.score[s] != 0.f)
+                        atomicAdd(T.dg + (uint64_t)s * P.cells + k, c * (double)S.score[s]);
             }
         }
-        return;
-    }
-    // each XCD adds into its own copy of the tallies (RTA_NCOPY copies,
-    // summed after the kernel): the copy is picked by the hardware XCD id,
-    // so no two XCDs ever update one copy
-    const uint64_t xc = xcd_id() % RTA_NCOPY;
-    const uint64_t base = P.box_cell[box] + xc * 3 * P.cells;
-    // spectral locations tally per mode; the Gamma-broadened spectra are one
-    // matrix product after the run (the reference adds the broadened weights
-    // of every segment, RTA_MC2D.cpp:718-766)
-    double* sp = nullptr;
-    if (P.spec) {
-        const int l = P.box_loc[box];
-        if (l >= 0) sp = P.spec + (size_t)l * P.nt * P.n + mode;
-    }
-    for (int i = b0; i <= b1; i++) {
-        double lo = fmax(P.timegrid[i] - t0, 0.);
-        double hi = fmin(P.timegrid[i + 1] - t0, delta);
-        double c = sign * fmax(hi - lo, 0.);
-        if (c == 0.) continue;
-        const uint64_t k = base + i;
-        atomicAdd(P.gz + k, c);
-        atomicAdd(P.jx + k, vx * c);
-        atomicAdd(P.jy + k, vy * c);
-        if (sp) atomicAdd(sp + (size_t)i * P.n, c);
-        if (GRAD) {
+    } else {
+        if (TM == 0 && !GRAD && spec) atomicAdd(spec + (size_t)i * P.n, c);
+        const uint32_t key = (TM == 0 || (uint32_t)i >= T.lbins) ? T.lc + cell0 + (uint32_t)i : row0 + (uint32_t)i;
+        if (key != A.key) {
+            acc_flush<TM, D>(P, T, A);
+            A.key = key;
+            A.g = A.x = A.y = 0.;
+            if constexpr (D) A.d[0] = A.d[1] = A.d[2] = A.d[3] = 0.;
+        }
+        A.g += c;
+        A.x += S.vx * c;
+        A.y += S.vy * c;
+        if constexpr (D) {
+#pragma unroll
             for (int s = 0; s < 4; s++)
-                if (((gmask >> s) & 1) && score[s] != 0.f)
-                    atomicAdd(P.dgz + xc * 4 * P.cells + (size_t)s * P.cells + (k - xc * 3 * P.cells),
-                              c * (double)score[s]);
+                if ((S.gmask >> s) & 1) A.d[s] += c * (double)S.score[s];
         }
     }
+}
+
+// process_segment (RTA_MC2D.cpp:699-769) from the lane's time to t1, which
+// becomes the lane's time. The lane keeps its time bin: the bin of a
+// segment's start is that of the previous one's end. In bin i the segment
+// [t0, t1] covers [max(t_i - t0, 0), min(t_i+1 - t0, t1 - t0)], where only the
+// first bin's lower and the last bin's upper bound are not grid differences.
+template <bool GRAD, int TM, bool GL, bool D>
+__device__ inline void tally_segment(const RtaParams& P, const RtaGeo<GL>& G, const RtaTally& T, TallyAcc<D>& A,
+                                     RtaState& S, int lrow, double t1) {
+    const double t0 = S.t, delta = t1 - t0;
+    double upper;
+    const int b1 = time_bin(G.grid, P.nt, P.idt, t1, upper);
+    double* spec = nullptr;
+    if (TM == 0 && !GRAD && P.spec) {
+        // spectral locations tally per mode; the Gamma-broadened spectra are
+        // one matrix product after the run (the reference adds the broadened
+        // weights of every segment, RTA_MC2D.cpp:718-766)
+        const int l = P.box_loc[S.box];
+        if (l >= 0) spec = P.spec + (size_t)l * P.nt * P.n + S.mode;
+    }
+    double lo = 0.;
+    for (int i = S.bin; i < b1; i++) {
+        const double g = G.grid[i + 1] - t0;
+        tally_bin<GRAD, TM, D>(P, T, A, S, lrow, spec, i, S.sign * fmax(g - lo, 0.));
+        lo = g;
+    }
+    tally_bin<GRAD, TM, D>(P, T, A, S, lrow, spec, b1, S.sign * fmax(fmin(upper - t0, delta) - lo, 0.));
+    S.bin = b1;
+    S.still = t1 == t0 ? S.still + 1 : 0;
+    S.t = t1;
 }
 
 // the run holding global particle id pid (first ids ascending)
@@ -267,75 +370,70 @@ __device__ inline int find_run(const RtaParams& P, uint64_t pid) {
 
 // The workgroup's LDS partial sums into the FP64 tallies (the XCD's copy).
 template <bool GRAD>
-__device__ inline void lt_flush(const RtaParams& P, const float* lt) {
-    const uint32_t nt = (uint32_t)P.nt, lc = (uint32_t)P.lrows * nt;
-    const uint64_t xc = xcd_id() % RTA_NCOPY;
-    double* tz = P.gz + xc * 3 * P.cells;
-    for (uint32_t j = threadIdx.x; j < lc; j += blockDim.x) {
-        const uint32_t row = j / nt;
-        const uint64_t g = P.lrow_cell[row] + (j - row * nt);
+__device__ inline void lt_flush(const RtaParams& P, const RtaTally& T) {
+    const float* lt = (const float*)T.lds;
+    for (uint32_t j = threadIdx.x; j < T.lc; j += blockDim.x) {
+        const uint32_t row = j / T.lbins;
+        const uint64_t g = P.lrow_cell[row] + (j - row * T.lbins);
         for (int a = 0; a < 3; a++) {
-            const float v = lt[(size_t)a * lc + j];
-            if (v != 0.f) atomicAdd(tz + (uint64_t)a * P.cells + g, (double)v);
+            const float v = lt[(size_t)a * T.lc + j];
+            if (v != 0.f) atomicAdd(T.g + (uint64_t)a * P.cells + g, (double)v);
         }
         if (GRAD) {
             for (int s = 0; s < 4; s++) {
                 if (P.lt_goff[s] < 0) continue;
-                const float v = lt[(size_t)P.lt_goff[s] + j];
-                if (v != 0.f) atomicAdd(P.dgz + xc * 4 * P.cells + (uint64_t)s * P.cells + g, (double)v);
+                const float v = lt[(size_t)P.lt_goff[s] * T.lc + j];
+                if (v != 0.f) atomicAdd(T.dg + (uint64_t)s * P.cells + g, (double)v);
             }
         }
     }
 }
 
-// The LT kernels give the whole LDS to the tallies (up to 160 KB), so their
-// counters are summed through that block after the flush instead of
-// block_add_u64's static array.
-extern __shared__ __align__(16) float rta_lt[];
-__device__ inline void lt_counters(unsigned long long* cnt, unsigned long long v0, unsigned long long v1,
-                                   unsigned long long v3, unsigned long long v4, unsigned long long v5) {
-    unsigned long long* part = (unsigned long long*)rta_lt;
-    unsigned long long v[5] = {v0, v1, v3, v4, v5};
-    for (int k = 0; k < 5; k++)
-        for (int d = 32; d > 0; d >>= 1) v[k] += __shfl_down(v[k], d, 64);
-    __syncthreads();  // the flush has read every partial sum
-    if ((threadIdx.x & 63) == 0)
-        for (int k = 0; k < 5; k++) part[(threadIdx.x >> 6) * 5 + k] = v[k];
+// Event and crossing counts of the workgroup through LDS (16-byte aligned,
+// 16 waves at most), one global atomic per counter; every thread calls this.
+extern __shared__ __align__(16) unsigned char rta_lds[];
+__device__ inline void rta_add_counts(const RtaParams& P, const RtaCounts& C) {
+    unsigned long long* part = reinterpret_cast<unsigned long long*>(rta_lds);
+    unsigned long long ev = C.events, cr = C.crossings;
+    for (int d = 32; d > 0; d >>= 1) {
+        ev += __shfl_down(ev, d, 64);
+        cr += __shfl_down(cr, d, 64);
+    }
+    __syncthreads();  // the block's LDS has been read
+    if ((threadIdx.x & 63) == 0) {
+        part[2 * (threadIdx.x >> 6)] = ev;
+        part[2 * (threadIdx.x >> 6) + 1] = cr;
+    }
     __syncthreads();
-    if (threadIdx.x < 5) {
+    if (threadIdx.x < 2) {
         unsigned long long t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += part[w * 5 + threadIdx.x];
-        const int dst[5] = {0, 1, 3, 4, 5};
-        if (t) atomicAdd(cnt + dst[threadIdx.x], t);
+        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += part[2 * w + threadIdx.x];
+        if (t) atomicAdd(P.counters + threadIdx.x, t);
     }
 }
 
-// The state of one particle history between events.
-struct RtaState {
-    Pcg32 rng;
-    double x, y, t, dtrem, wscale, tlast;
-    unsigned long long budget;
-    int mode, box, sign, run, still, alive, need_flight, scat0;
-    int ballistic, pad0;
-    float score[4];
-};
+// The kernel's parameters for code off the main path: read from the kernel
+// argument segment where they are used. Kept in scalar registers over the
+// whole loop, the pointers of these paths would push those of the main path
+// into vector lanes (a lane read for each use).
+__device__ inline const RtaParams& rta_cold_params() {
+    auto* p = (const __attribute__((address_space(4))) RtaParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const RtaParams*)p;
+}
 
-struct RtaCounts {
-    unsigned long long events = 0, crossings = 0, stuck = 0, badmirror = 0, badtrans = 0;
-};
-
-// Init_generator (RTA_MC2D.cpp:436-484): particle pid of its run at t = 0
-template <bool GRAD, bool POLY>
-__device__ inline void rta_start(const RtaParams& P, RtaState& S, uint64_t pid) {
+// Init_generator (RTA_MC2D.cpp:436-484): particle pid of its run at t = 0.
+template <bool GRAD, int TM, bool POLY, bool GL>
+__device__ inline void rta_start(const RtaGeo<GL>& G, RtaState& S, uint64_t pid) {
+    const RtaParams& P = rta_cold_params();
     S.budget = 0;
-    S.still = 0;
-    S.tlast = -1.0;
-    S.run = find_run(P, pid);
-    const RtaRunDev& R = P.runs[S.run];
-    S.rng.seed(R.seed, pid - R.first);
+    S.still = -1;  // the first event of a history never counts as standing still
+    if (TM != 3) S.run = find_run(P, pid);
+    const RtaRunDev& R = P.runs[TM == 3 ? G.run : S.run];
     S.wscale = R.wscale;
-    S.scat0 = R.scat0;
+    S.rng.seed(R.seed, pid - R.first);
     S.ballistic = R.ballistic;
+    S.gmask = R.gmask;
     if (GRAD) S.score[0] = S.score[1] = S.score[2] = S.score[3] = 0.f;
     bool ng;
     int gi = R.gen0 + (int)alias_pick(P.gen_sel + R.gsel0, (uint32_t)R.ngen, S.rng, ng);
@@ -343,368 +441,643 @@ __device__ inline void rta_start(const RtaParams& P, RtaState& S, uint64_t pid) 
     double u = S.rng.uniform();
     S.x = g.p1x + u * g.ndx;
     S.y = g.p1y + u * g.ndy;
-    if constexpr (POLY) {
-        if (!poly_inside(P.sides, P.srange[g.idi], S.x, S.y)) {
-            const double2 c = P.center[g.idi];
-            double dx = c.x - S.x, dy = c.y - S.y;
-            double dn = sqrt(dx * dx + dy * dy);
-            S.x += 1.0e-6 * dx / dn;
-            S.y += 1.0e-6 * dy / dn;
-        }
-    } else {
-        const DevBox bi = P.boxes[g.idi];
-        if (!box_inside(bi, S.x, S.y)) {
-            double dx = 0.5 * (bi.xmin + bi.xmax) - S.x, dy = 0.5 * (bi.ymin + bi.ymax) - S.y;
-            double dn = sqrt(dx * dx + dy * dy);
-            S.x += 1.0e-6 * dx / dn;
-            S.y += 1.0e-6 * dy / dn;
-        }
+    S.box = g.idi - G.bo;
+    const RtaBox B = G.at(S.box);
+    const bool in = POLY ? poly_inside(G.side, make_int2(B.s0, B.ns), S.x, S.y)
+                         : S.x >= B.xmin && S.x <= B.xmax && S.y >= B.ymin && S.y <= B.ymax;
+    if (!in) {
+        const double ccx = POLY ? P.center[g.idi].x : 0.5 * (B.xmin + B.xmax);
+        const double ccy = POLY ? P.center[g.idi].y : 0.5 * (B.ymin + B.ymax);
+        double dx = ccx - S.x, dy = ccy - S.y;
+        double dn = sqrt(dx * dx + dy * dy);
+        S.x += 1.0e-6 * dx / dn;
+        S.y += 1.0e-6 * dy / dn;
     }
     S.mode = (int)alias_pick(P.gen_tab + (size_t)gi * P.n, (uint32_t)P.n, S.rng, ng);
     S.sign = g.sign;
-    S.box = g.idi;
     S.t = 0.;
-    S.alive = 1;
-    S.need_flight = 1;
+    S.bin = 0;
+    S.st = RTA_FRESH;
 }
 
-// Every history ends: a particle that exceeds the iteration budget or makes
-// 64 events in a row without advancing in time is dropped and counted.
-__device__ inline void rta_watch(const RtaParams& P, RtaState& S, RtaCounts& C) {
-    S.still = (S.t == S.tlast) ? S.still + 1 : 0;
-    S.tlast = S.t;
-    if (++S.budget > P.max_iters || S.still > 64) {
-        C.stuck++;
-        S.alive = 0;
+// The scattering that ends a flight inside the box draws the next two numbers
+// of the stream (alias_pick). They are taken ahead, once per flight, on a copy
+// of the generator, and the alias entry is loaded while the flight is
+// computed and flown; the copy replaces the generator only on that path, so
+// every stream is consumed as without the look-ahead.
+template <int TM, bool GL>
+__device__ inline void rta_look(const RtaParams& P, const RtaGeo<GL>& G, RtaState& S) {
+    Pcg32 r = S.rng;
+    S.sk = r.bounded((uint32_t)P.n);
+    S.su = r.next();
+    S.look = r.state;
+    S.se = P.scat[(size_t)(TM == 3 ? G.run : S.run) * (uint32_t)P.n + S.sk];
+}
+
+// Exit from a rectangle (box_exit) and the fast neighbour search (side_fast)
+// in one: time t, point (ex, ey), the side or, when the general search must
+// run, the mask of the sides. Returns the neighbour, SIDE_VOID or SIDE_MIXED.
+// Selects only: a lane's box and direction differ from its neighbours', so
+// branches would run one after the other.
+__device__ inline int rect_exit(const RtaBox& b, double x, double y, double vx, double vy, double ivx, double ivy,
+                                double& t, double& ex, double& ey, int& aux) {
+    const bool px = vx > 0., py = vy > 0.;
+    const double bx = px ? b.xmax : b.xmin, by = py ? b.ymax : b.ymin;
+    double tx = vx == 0. ? 1e300 : (bx - x) * ivx, ty = vy == 0. ? 1e300 : (by - y) * ivy;
+    tx = tx < 0. ? 0. : tx;
+    ty = ty < 0. ? 0. : ty;
+    const bool xfirst = tx < ty, yfirst = ty < tx;  // neither: both sides at once
+    t = yfirst ? ty : tx;
+    ex = yfirst ? x + t * vx : bx;
+    ey = xfirst ? y + t * vy : by;
+    if (almost_equal(t, 0.)) t = 0.;
+    const bool in_y = (ey > b.ymin) & (ey < b.ymax), in_x = (ex > b.xmin) & (ex < b.xmax);
+    const bool clear = (xfirst & in_y & !almost_equal(vx, 0.)) | (yfirst & in_x & !almost_equal(vy, 0.));
+    const int nx = px ? b.side_nbr[3] : b.side_nbr[0], ny = py ? b.side_nbr[2] : b.side_nbr[1];
+    if (clear) {
+        aux = xfirst ? (px ? 3 : 0) : (py ? 2 : 1);
+        return xfirst ? nx : ny;
     }
+    const int sx = px ? 3 : (vx < 0. ? 0 : 31), sy = py ? 2 : (vy < 0. ? 1 : 31);
+    aux = (yfirst ? 0 : 1 << sx) | (xfirst ? 0 : 1 << sy);
+    return SIDE_MIXED;
 }
 
-// One step of evolparticle (RTA_MC2D.cpp:990-1386) after the flight draw of
-// the history loop (2262-2288).
-// POLY: the geometry has convex polygon boxes (diffuse sides only)
-template <bool GRAD, int TM, bool POLY>
-__device__ inline void rta_event(const RtaParams& P, void* lds, TallyAcc& A, RtaState& S, RtaCounts& C) {
-    const double4 md = P.modes[S.mode];
-    const DevBox B = P.boxes[S.box];
-    double u = 0.;
-    if (S.need_flight) {
+// One event of evolparticle (RTA_MC2D.cpp:990-1386) for lanes in FRESH or FLY:
+// the flight draw of the history loop (2262-2288), the segment to the next
+// scattering or box side and its tally, the scattering or the crossing into
+// the one box that shares the side. What few lanes meet at a time (void
+// sides, corners and partly shared sides, periodic boxes) is left to
+// rta_slow.
+template <bool GRAD, int TM, bool POLY, bool GL, bool D>
+__device__ inline void rta_fly(const RtaParams& P, const RtaGeo<GL>& G, const RtaTally& T, TallyAcc<D>& A,
+                               RtaState& S, RtaCounts& C) {
+    // every history ends: a particle that exceeds the iteration budget or
+    // makes 64 events in a row without advancing in time is dropped
+    if (++S.budget > (1u << 26) || S.still > 64) {
+        atomicAdd(P.counters + 3, 1ULL);
+        S.st = RTA_DEAD;
+        return;
+    }
+    if (S.st == RTA_FRESH) {
         // exponential flight, truncated at maxtime
         if (!(S.t < P.maxtime)) {
-            S.alive = 0;
+            S.st = RTA_DEAD;
             return;
         }
-        u = 1.0 - S.rng.uniform();
-    }
-    // The scattering that ends a flight inside the box draws the next two
-    // numbers of the stream (alias_pick); they are taken here on a copy of
-    // the generator and the alias entry is loaded while the flight and the
-    // exit test are computed. The copy replaces the generator only on that
-    // path, so every stream is consumed as without the look-ahead.
-    Pcg32 r2 = S.rng;
-    const uint32_t sk = r2.bounded((uint32_t)P.n);
-    const uint32_t su = r2.next();
-    const uint2 se = P.scat[(size_t)S.scat0 + sk];
-    if (S.need_flight) {
-        S.dtrem = -log(u) / (md.z * S.wscale);
+        const RtaMode* M = P.rmodes + S.mode;
+        const double2 v = make_double2(M->vx, M->vy), iv = make_double2(M->ivx, M->ivy);
+        const double w = M->w;
+        const double u = 1.0 - S.rng.uniform();
+        rta_look<TM>(P, G, S);
+        S.vx = v.x;
+        S.vy = v.y;
+        S.ivx = iv.x;
+        S.ivy = iv.y;
+        S.dtrem = -log(u) / (w * (TM == 3 ? G.wscale : S.wscale));
         if (S.t + S.dtrem > P.maxtime) S.dtrem = P.maxtime - S.t + 1.0e-8;
-        if (almost_equal(S.dtrem, 0.)) return;
-        S.need_flight = 0;
-    }
-    if (B.kind == 2) {
-        // periodic box: translate, keep the remaining flight (RTA_MC2D.cpp:1034-1043)
-        const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, S.box, S.x, S.y,
-                                             md.x, md.y, S.rng)
-                            : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, S.box, S.x, S.y, md.x, md.y, S.rng);
-        if (nb < 0) {
-            C.badtrans++;
-            S.alive = 0;
+        if (almost_equal(S.dtrem, 0.)) {
+            S.still++;
             return;
         }
-        S.box = nb;
+        S.st = RTA_FLY;
+    }
+    const RtaBox B = G.at(S.box);
+    if (B.kind != 0) {
+        S.still++;
+        if (B.kind == 2) {
+            S.st = RTA_TRANS;
+        } else {  // reservoir: absorbed (RTA_MC2D.cpp:1046-1053)
+            C.events++;
+            S.st = RTA_DEAD;
+        }
         return;
     }
-    if (B.kind == 1) {  // reservoir: absorbed (RTA_MC2D.cpp:1046-1053)
-        C.events++;
-        S.alive = 0;
-        return;
-    }
-    const int gmask = GRAD ? P.runs[S.run].gmask : 0;
-    const double vx = md.x, vy = md.y;
-    double nx = S.x + S.dtrem * vx, ny = S.y + S.dtrem * vy;
-    int2 sr = make_int2(0, 0);
-    if constexpr (POLY) sr = P.srange[S.box];
-    const bool inside = POLY ? poly_inside(P.sides, sr, nx, ny) : box_inside(B, nx, ny);
-    int mask = 0;
-    double ex = 0., ey = 0., tf = 0.;
+    const double vx = S.vx, vy = S.vy;
+    double nx = S.x + S.dtrem * vx, ny = S.y + S.dtrem * vy, step = S.dtrem;
+    const int2 sr = make_int2(B.s0, B.ns);
+    const bool inside = POLY ? poly_inside(G.side, sr, nx, ny)
+                             : (nx >= B.xmin) & (nx <= B.xmax) & (ny >= B.ymin) & (ny <= B.ymax);
+    int fast = SIDE_MIXED;
     if (!inside) {
         if constexpr (POLY) {
-            tf = poly_exit(P.sides, sr, S.x, S.y, vx, vy, mask, ex, ey);
+            int mask;
+            step = poly_exit(G.side, sr, S.x, S.y, vx, vy, mask, nx, ny);
+            fast = poly_side_fast(G.side, sr, mask, nx, ny, vx, vy, S.aux);
+            if (fast == SIDE_MIXED) S.aux = mask;
         } else {
-            const double2 iv = P.ivel[S.mode];
-            tf = box_exit(B, S.x, S.y, vx, vy, iv.x, iv.y, mask, ex, ey);
+            fast = rect_exit(B, S.x, S.y, vx, vy, S.ivx, S.ivy, step, nx, ny, S.aux);
         }
     }
+    tally_segment<GRAD, TM, GL, D>(P, G, T, A, S, B.lrow, S.t + step);
+    S.x = nx;
+    S.y = ny;
     if (inside) {
-        tally_segment<GRAD, TM>(P, lds, A, S.box, S.t, S.t + S.dtrem, S.sign, vx, vy, gmask, S.score, S.mode);
-        S.x = nx;
-        S.y = ny;
-        S.t += S.dtrem;
         if (!S.ballistic) {
             // alias_pick with the draws taken ahead
-            S.mode = su < se.x ? (int)sk : (int)(se.y & 0x3fffffffu);
-            S.rng = r2;
+            S.mode = S.su < S.se.x ? (int)S.sk : (int)(S.se.y & 0x3fffffffu);
+            S.rng.state = S.look;
         }
         C.events++;
-        S.need_flight = 1;
+        S.st = RTA_FRESH;
         return;
     }
-    double left = S.dtrem - tf;
+    double left = S.dtrem - step;
     if (almost_equal(left, 0.)) left = 0.;
-    tally_segment<GRAD, TM>(P, lds, A, S.box, S.t, S.t + tf, S.sign, vx, vy, gmask, S.score, S.mode);
-    S.t += tf;
-    int side = 0;
-    const int fast = POLY ? poly_side_fast(P.sides, sr, mask, ex, ey, vx, vy, side)
-                          : side_fast(B, mask, ex, ey, vx, vy, side);
-    Ids4 pb{};
-    int npb;
-    if (fast >= 0) {
-        pb.a = fast;
-        npb = 1;
-    } else if (fast == SIDE_VOID) {
-        npb = 0;
-    } else {
-        npb = POLY ? poly_find_pboxes(P.sides, P.srange, P.cts, B, ex, ey, vx, vy, pb)
-                   : find_pboxes(P.boxes, P.cts, B, ex, ey, vx, vy, pb);
-    }
-    if (npb == 0) {
-        int s = fast == SIDE_VOID ? side
-              : (__popc(mask) == 1 ? __ffs(mask) - 1
-                 : (POLY ? poly_pick_void_side(P.sides, P.srange, P.cts, B, sr, mask, ex, ey, S.rng.next())
-                         : pick_void_side(P.boxes, P.cts, B, mask, ex, ey, S.rng.next())));
-        // specular with probability p (mirror partner of the mode), else
-        // diffuse; a draw is made only when 0 < p < 1 (polygon runs: diffuse)
-        const float p = POLY ? 0.f : P.runs[S.run].spec[s];
-        bool specular = p >= 1.f;
-        if (p > 0.f && p < 1.f) {
-            specular = S.rng.uniform() < (double)p;
-            if (GRAD && ((gmask >> s) & 1)) {
-                // d/dp log P(outcome): 1/p for specular, -1/(1-p) for diffuse
-                const float d = specular ? 1.f / p : -1.f / (1.f - p);
-                if (s == 0) S.score[0] += d;
-                else if (s == 1) S.score[1] += d;
-                else if (s == 2) S.score[2] += d;
-                else S.score[3] += d;
-            }
-        }
-        if (specular) {
-            const int partner = P.mirror[(s == 0 || s == 3 ? 0 : (size_t)P.n) + S.mode];
-            if (partner < 0) {
-                C.badmirror++;
-                S.alive = 0;
-                return;
-            }
-            S.mode = partner;
-        } else {
-            // Lambert re-emission (RTA_MC2D.cpp:635-678)
-            const int4 li = P.lam_info[S.mode];
-            const int tabk = POLY ? P.sides[sr.x + s].nid : s;
-            bool ng;
-            int k = (int)alias_pick(P.lam_tab + li.z + (size_t)tabk * li.y, (uint32_t)li.y, S.rng, ng);
-            S.mode = P.perm[li.x + k];
-        }
-        // the remaining flight is discarded (RTA_MC2D.cpp:1259)
-        S.x = ex;
-        S.y = ey;
-        C.events++;
-        S.need_flight = 1;
-        return;
-    }
-    S.x = ex;
-    S.y = ey;
-    if (npb == 1) {
-        S.box = pb.a;
-    } else {
-        // several candidate boxes at a corner (RTA_MC2D.cpp:1316-1380)
-        Ids4 cand{};
-        int nc = 0;
-        double cx = ex + 1.0e-6 * vx, cy = ey + 1.0e-6 * vy;
-        for (int k = 0; k < npb && k < 4; k++) {
-            const bool in = POLY ? poly_inside(P.sides, P.srange[pb.get(k)], cx, cy)
-                                 : box_inside(P.boxes[pb.get(k)], cx, cy);
-            if (in) cand.set(nc++, pb.get(k));
-        }
-        if (nc > 0) {
-            S.box = cand.get((int)S.rng.bounded((uint32_t)nc));
-        } else {
-            S.box = pb.get((int)S.rng.bounded((uint32_t)(npb < 4 ? npb : 4)));
-            double ccx, ccy;
-            if constexpr (POLY) {
-                ccx = P.center[S.box].x;
-                ccy = P.center[S.box].y;
-            } else {
-                const DevBox nb = P.boxes[S.box];
-                ccx = 0.5 * (nb.xmin + nb.xmax);
-                ccy = 0.5 * (nb.ymin + nb.ymax);
-            }
-            double dx = ccx - S.x, dy = ccy - S.y;
-            double dn = sqrt(dx * dx + dy * dy);
-            S.x += 1.0e-6 * dx / dn;
-            S.y += 1.0e-6 * dy / dn;
-        }
-    }
-    C.crossings++;
     S.dtrem = left;
-    if (S.dtrem == 0.) S.need_flight = 1;
-    return;
+    if (fast >= 0) {
+        S.box = fast;
+        C.crossings++;
+        S.st = left == 0. ? RTA_FRESH : RTA_FLY;
+    } else {
+        S.st = fast == SIDE_VOID ? RTA_WALL : RTA_MIXED;
+    }
 }
 
-// One lane follows one particle history at a time and takes the next id
-// from a per-wave pool when it ends; ids of all runs form one range, so a
-// batch of runs of any sizes fills the GPU in one launch.
-template <bool GRAD, int TMK, bool POLY = false>
-__global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams P) {
-    float* lt = nullptr;
-    if constexpr (TMK == 1) {
-        lt = rta_lt;
-        int narr = 3;
-        for (int s = 0; s < 4; s++) narr += P.lt_goff[s] >= 0 ? 1 : 0;
-        const uint32_t nf = (uint32_t)narr * (uint32_t)P.lrows * (uint32_t)P.nt;
-        for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) lt[j] = 0.f;
-        __syncthreads();
-    } else if constexpr (TMK == 2) {
-        lt = rta_lt;
-        double* g = (double*)rta_lt;
-        const uint32_t nf = 3u * (uint32_t)P.lrows * (uint32_t)P.lbins;
-        for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) g[j] = 0.;
-        __syncthreads();
+// The rest of an event for lanes in WALL (a void side reached), MIXED (an exit
+// that the general neighbour search decides) or TRANS (a periodic box).
+template <bool GRAD, int TM, bool POLY, bool GL>
+__device__ inline void rta_slow(const RtaGeo<GL>& G, RtaState& S, RtaCounts& C) {
+    const RtaParams& P = rta_cold_params();
+    const int abox = S.box + G.bo;  // the box in the batch's arrays
+    const double vx = S.vx, vy = S.vy;
+    if (S.st == RTA_TRANS) {
+        // periodic box: translate, keep the remaining flight (RTA_MC2D.cpp:1034-1043)
+        const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, abox, S.x, S.y,
+                                             vx, vy, S.rng)
+                            : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, abox, S.x, S.y, vx, vy, S.rng);
+        if (nb < 0) {
+            atomicAdd(P.counters + 5, 1ULL);
+            S.st = RTA_DEAD;
+            return;
+        }
+        S.box = nb - G.bo;
+        S.st = RTA_FLY;
+        rta_look<TM>(P, G, S);  // the translation may have drawn
+        return;
     }
-    TallyAcc A;
-    RtaState S;
-    S.alive = 0;
-    RtaCounts C;
-    // particle ids come from a per-wave pool refilled 64 at a time, so the
-    // global id counter sees one atomic per 64 histories
-    unsigned long long pool_lo = 0, pool_hi = 0;
-    for (;;) {
-        if (S.alive) rta_watch(P, S, C);
-        unsigned long long pid = ~0ULL;
-        unsigned long long want = __ballot(!S.alive);
-        while (want) {
-            if (pool_lo == pool_hi) {
-                unsigned long long base = 0;
-                const int leader = __ffsll((long long)want) - 1;
-                if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(P.counters + 2, 64ULL);
-                base = __shfl(base, leader, 64);
-                pool_lo = base;
-                pool_hi = base + 64;
+    int s = S.aux;
+    if (S.st == RTA_MIXED) {
+        const int mask = S.aux;
+        const DevBox B = P.boxes[abox];
+        const int2 sr = POLY ? P.srange[abox] : make_int2(0, 0);
+        Ids4 pb{};
+        const int npb = POLY ? poly_find_pboxes(P.sides, P.srange, P.cts, B, S.x, S.y, vx, vy, pb)
+                             : find_pboxes(P.boxes, P.cts, B, S.x, S.y, vx, vy, pb);
+        if (npb > 0) {
+            int nbox;
+            if (npb == 1) {
+                nbox = pb.a;
+            } else {
+                // several candidate boxes at a corner (RTA_MC2D.cpp:1316-1380)
+                Ids4 cand{};
+                int nc = 0;
+                const double cx = S.x + 1.0e-6 * vx, cy = S.y + 1.0e-6 * vy;
+                for (int k = 0; k < npb && k < 4; k++) {
+                    const bool in = POLY ? poly_inside(P.sides, P.srange[pb.get(k)], cx, cy)
+                                         : box_inside(P.boxes[pb.get(k)], cx, cy);
+                    if (in) cand.set(nc++, pb.get(k));
+                }
+                if (nc > 0) {
+                    nbox = cand.get((int)S.rng.bounded((uint32_t)nc));
+                } else {
+                    nbox = pb.get((int)S.rng.bounded((uint32_t)(npb < 4 ? npb : 4)));
+                    double ccx, ccy;
+                    if constexpr (POLY) {
+                        ccx = P.center[nbox].x;
+                        ccy = P.center[nbox].y;
+                    } else {
+                        const DevBox nb = P.boxes[nbox];
+                        ccx = 0.5 * (nb.xmin + nb.xmax);
+                        ccy = 0.5 * (nb.ymin + nb.ymax);
+                    }
+                    double dx = ccx - S.x, dy = ccy - S.y;
+                    double dn = sqrt(dx * dx + dy * dy);
+                    S.x += 1.0e-6 * dx / dn;
+                    S.y += 1.0e-6 * dy / dn;
+                }
+                rta_look<TM>(P, G, S);  // the choice has drawn
             }
-            const unsigned long long below = want & ((1ULL << (threadIdx.x & 63)) - 1ULL);
-            const unsigned long long rank = (unsigned long long)__popcll(below);
-            const unsigned long long take = min((unsigned long long)__popcll(want), pool_hi - pool_lo);
-            const bool mine = (want >> (threadIdx.x & 63)) & 1ULL;
-            if (mine && rank < take) pid = pool_lo + rank;
-            pool_lo += take;
-            want = __ballot(!S.alive && pid == ~0ULL);
+            S.box = nbox - G.bo;
+            C.crossings++;
+            S.st = S.dtrem == 0. ? RTA_FRESH : RTA_FLY;
+            return;
         }
-        if (!S.alive) {
-            if (pid >= P.total) break;
-            rta_start<GRAD, POLY>(P, S, pid);
-        }
-        rta_event<GRAD, TMK, POLY>(P, lt, A, S, C);
+        s = __popc(mask) == 1 ? __ffs(mask) - 1
+            : (POLY ? poly_pick_void_side(P.sides, P.srange, P.cts, B, sr, mask, S.x, S.y, S.rng.next())
+                    : pick_void_side(P.boxes, P.cts, B, mask, S.x, S.y, S.rng.next()));
     }
+    // specular with probability p (mirror partner of the mode), else
+    // diffuse; a draw is made only when 0 < p < 1 (polygon runs: diffuse)
+    const float p = POLY ? 0.f : P.runs[TM == 3 ? G.run : S.run].spec[s];
+    bool specular = p >= 1.f;
+    if (p > 0.f && p < 1.f) {
+        specular = S.rng.uniform() < (double)p;
+        if (GRAD && ((S.gmask >> s) & 1)) {
+            // d/dp log P(outcome): 1/p for specular, -1/(1-p) for diffuse
+            const float d = specular ? 1.f / p : -1.f / (1.f - p);
+            // selects keep the scores in registers
+#pragma unroll
+            for (int k = 0; k < 4; k++) S.score[k] = s == k ? S.score[k] + d : S.score[k];
+        }
+    }
+    if (specular) {
+        const int partner = P.mirror[(s == 0 || s == 3 ? 0 : (size_t)P.n) + S.mode];
+        if (partner < 0) {
+            atomicAdd(P.counters + 4, 1ULL);
+            S.st = RTA_DEAD;
+            return;
+        }
+        S.mode = partner;
+    } else {
+        // Lambert re-emission (RTA_MC2D.cpp:635-678)
+        const RtaMode* M = P.rmodes + S.mode;
+        const int lo = M->lo, len = M->len, base = M->base;
+        const int tabk = POLY ? P.sides[P.srange[abox].x + s].nid : s;
+        bool ng;
+        const int k = (int)alias_pick(P.lam_tab + base + (size_t)tabk * len, (uint32_t)len, S.rng, ng);
+        S.mode = P.perm[lo + k];
+    }
+    // the remaining flight is discarded (RTA_MC2D.cpp:1259)
+    C.events++;
+    S.st = RTA_FRESH;
+}
+
+// Histories change waves within a workgroup once the particle ids have run
+// out. History lengths are heavy-tailed (a ribbon of 1 um over 5 ns: 160
+// events on average, 2900 for a particle that stays to the end), so the waves
+// would run on with a few lanes each: 19 of 64 on average over a run of 1e6
+// particles, and a pass costs a wave the same with 5 lanes as with 64. A wave
+// donates its idle lanes to RtaMig::free. A wave whose live histories fit in
+// lanes that other waves donated reserves them, writes the histories to the
+// mailbox and ends; waves with idle lanes take them from there. The first
+// keep_waves waves of a workgroup (one per SIMD of the CU) never give theirs
+// away. A wave leaves with idle lanes only after withdrawing its donation, so
+// reserved lanes always exist and every wait ends.
+struct RtaMig {
+    int32_t free;   // donated idle lanes not reserved
+    int32_t lock;   // the mailbox is in use
+    int32_t n;      // histories in the mailbox not yet claimed
+    int32_t total, read;  // its size and the histories read
+    int32_t pad[3];
+};
+#define RTA_MAIL_WORDS 12
+#define RTA_MIG_BYTES (sizeof(RtaMig) + 64 * RTA_MAIL_WORDS * sizeof(uint64_t))
+// between barriers; the caller synchronises
+__device__ inline void rta_mig_init(const RtaParams& P) {
+    if (P.mig >= 0 && threadIdx.x < sizeof(RtaMig) / sizeof(int32_t))
+        reinterpret_cast<int32_t*>(rta_lds + P.mig)[threadIdx.x] = 0;
+}
+__device__ inline int wg_load(const int32_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline bool wg_cas(int32_t* p, int& expect, int v) {
+    return __hip_atomic_compare_exchange_strong(p, &expect, v, __ATOMIC_ACQ_REL, __ATOMIC_ACQUIRE,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline int wg_add(int32_t* p, int v) {
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// takes n from *p unless less than n is there (one lane of a wave calls it)
+__device__ inline bool wg_take(int32_t* p, int need, int n) {
+    int f = wg_load(p);
+    while (f >= need)
+        if (wg_cas(p, f, f - n)) return true;
+    return false;
+}
+
+template <bool GRAD>
+__device__ inline void rta_mail_write(uint64_t* w, const RtaState& S) {
+    auto pair = [](int a, int b) { return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32; };
+    w[0 * 64] = S.rng.state;
+    w[1 * 64] = S.rng.inc;
+    w[2 * 64] = (uint64_t)__double_as_longlong(S.x);
+    w[3 * 64] = (uint64_t)__double_as_longlong(S.y);
+    w[4 * 64] = (uint64_t)__double_as_longlong(S.t);
+    w[5 * 64] = (uint64_t)__double_as_longlong(S.dtrem);
+    w[6 * 64] = pair(S.mode, S.box);
+    w[7 * 64] = pair(S.still, S.st | S.aux << 8);
+    w[8 * 64] = pair(S.bin, S.run);
+    w[9 * 64] = pair((int)S.budget, (S.sign < 0 ? 1 : 0) | (S.ballistic ? 2 : 0) | S.gmask << 2);
+    if (GRAD) {
+        w[10 * 64] = pair(__float_as_int(S.score[0]), __float_as_int(S.score[1]));
+        w[11 * 64] = pair(__float_as_int(S.score[2]), __float_as_int(S.score[3]));
+    }
+}
+template <bool GRAD, int TM, bool GL>
+__device__ inline void rta_mail_read(const RtaParams& P, const RtaGeo<GL>& G, const uint64_t* w, RtaState& S) {
+    auto lo = [](uint64_t v) { return (int)(uint32_t)v; };
+    auto hi = [](uint64_t v) { return (int)(uint32_t)(v >> 32); };
+    S.rng.state = w[0 * 64];
+    S.rng.inc = w[1 * 64];
+    S.x = __longlong_as_double((long long)w[2 * 64]);
+    S.y = __longlong_as_double((long long)w[3 * 64]);
+    S.t = __longlong_as_double((long long)w[4 * 64]);
+    S.dtrem = __longlong_as_double((long long)w[5 * 64]);
+    S.mode = lo(w[6 * 64]);
+    S.box = hi(w[6 * 64]);
+    S.still = lo(w[7 * 64]);
+    S.st = hi(w[7 * 64]) & 255;
+    S.aux = hi(w[7 * 64]) >> 8;
+    S.bin = lo(w[8 * 64]);
+    S.run = hi(w[8 * 64]);
+    S.budget = (uint32_t)lo(w[9 * 64]);
+    const int f = hi(w[9 * 64]);
+    S.sign = (f & 1) ? -1 : 1;
+    S.ballistic = (f >> 1) & 1;
+    S.gmask = f >> 2;
+    if (GRAD) {
+        S.score[0] = __int_as_float(lo(w[10 * 64]));
+        S.score[1] = __int_as_float(hi(w[10 * 64]));
+        S.score[2] = __int_as_float(lo(w[11 * 64]));
+        S.score[3] = __int_as_float(hi(w[11 * 64]));
+    }
+    if (TM != 3) S.wscale = P.runs[S.run].wscale;
+    // of the flight under way: the mode's velocity and the look-ahead
+    const RtaMode* M = P.rmodes + S.mode;
+    S.vx = M->vx;
+    S.vy = M->vy;
+    S.ivx = M->ivx;
+    S.ivy = M->ivy;
+    rta_look<TM>(P, G, S);
+}
+
+// Follows histories until the ids run out: one particle history per lane at a
+// time. Per pass the lanes in FRESH or FLY make one event; the lanes that
+// wait (pending sides, ended histories) are served together once an eighth of
+// the live lanes wait for a side or RTA_REFILL_MIN for an id, or no lane of the
+// wave can fly, so the code of those paths, which a few lanes per pass would
+// run with the rest of the wave idle, runs every few passes with more lanes
+// in it. take(want, lo, hi) hands the wave a range of at least one id (ids at
+// or past `end` mean that there is none left). Streams are keyed by the
+// particle id and kept with the history, so the order of ids and of events
+// between lanes changes nothing in any history.
+#define RTA_REFILL_MIN 8
+template <bool GRAD, int TM, bool POLY, bool GL, bool D, class Take>
+__device__ inline void rta_histories(const RtaParams& P, const RtaGeo<GL>& G, const RtaTally& T, RtaCounts& C,
+                                     unsigned long long end, Take take) {
+    TallyAcc<D> A;
+    RtaState S;
+    const int lane = threadIdx.x & 63;
+    const unsigned long long below = (1ULL << lane) - 1ULL;
+    S.st = lane < P.lanes ? RTA_DEAD : RTA_DONE;
+    const auto can_fly = [&S] { return S.st == RTA_FRESH || S.st == RTA_FLY; };
+    unsigned long long pool_lo = 0, pool_hi = 0;
+    bool exhausted = false;  // no id left
+    RtaMig* M = reinterpret_cast<RtaMig*>(rta_lds + P.mig);
+    uint64_t* mail = reinterpret_cast<uint64_t*>(rta_lds + P.mig + sizeof(RtaMig));
+    const bool may_give = (int)(threadIdx.x >> 6) >= P.keep_waves;
+    int donated = 0;
+    uint32_t tick = 0;
+    for (;;) {
+        unsigned long long flying = __ballot(can_fly());
+        const unsigned long long pend = __ballot(S.st >= RTA_WALL && S.st <= RTA_TRANS);
+        if (pend && 8 * __popcll(pend) >= __popcll(flying | pend)) {
+            if ((pend >> lane) & 1ULL) rta_slow<GRAD, TM, POLY, GL>(G, S, C);
+            flying = __ballot(can_fly());
+        }
+        unsigned long long dead = __ballot(S.st == RTA_DEAD);
+        if (dead && (!flying || exhausted || __popcll(dead) >= RTA_REFILL_MIN)) {
+            unsigned long long pid = ~0ULL;
+            while (dead && !exhausted) {
+                if (pool_lo == pool_hi) {
+                    take(__popcll(dead), pool_lo, pool_hi);
+                    exhausted = pool_lo >= end;
+                }
+                const unsigned long long rank = (unsigned long long)__popcll(dead & below);
+                const unsigned long long n = min((unsigned long long)__popcll(dead), pool_hi - pool_lo);
+                const bool mine = (dead >> lane) & 1ULL;
+                if (mine && rank < n) pid = pool_lo + rank;
+                pool_lo += n;
+                dead = __ballot(S.st == RTA_DEAD && pid == ~0ULL);
+            }
+            if (S.st == RTA_DEAD) {
+                if (pid >= end) {
+                    S.st = RTA_DONE;
+                } else {
+                    rta_start<GRAD, TM, POLY, GL>(G, S, pid);
+                    // the lane's 32-bit counts: far from wrapping between two particles
+                    if ((C.events | C.crossings) & 0x80000000u) {
+                        atomicAdd(P.counters + 0, (unsigned long long)C.events);
+                        atomicAdd(P.counters + 1, (unsigned long long)C.crossings);
+                        C.events = C.crossings = 0;
+                    }
+                }
+            }
+            flying = __ballot(can_fly());
+        }
+        if (exhausted && (!flying || (++tick & 7) == 0)) {
+            unsigned long long idle = __ballot(S.st == RTA_DONE);
+            if (P.mig < 0) {
+                if (idle == ~0ULL) break;
+            } else {
+                const int nidle = __popcll(idle);
+                if (nidle > donated) {
+                    if (lane == 0) wg_add(&M->free, nidle - donated);
+                    donated = nidle;
+                }
+                // take histories from the mailbox into idle lanes
+                int got = 0, at = 0;
+                if (lane == 0 && nidle > 0) {
+                    int n = wg_load(&M->n);
+                    while (n > 0) {
+                        got = min(nidle, n);
+                        at = n - got;
+                        if (wg_cas(&M->n, n, at)) break;
+                        got = 0;
+                    }
+                }
+                got = __builtin_amdgcn_readfirstlane(got);
+                if (got > 0) {
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    const int rank = __popcll(idle & below);
+                    if (S.st == RTA_DONE && rank < got)
+                        rta_mail_read<GRAD, TM, GL>(P, G, mail + at + rank, S);
+                    donated -= got;
+                    if (lane == 0) {
+                        const int total = M->total;
+                        if (wg_add(&M->read, got) + got == total) {
+                            M->read = 0;
+                            __hip_atomic_store(&M->lock, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                    }
+                    idle = __ballot(S.st == RTA_DONE);
+                    flying = __ballot(can_fly());
+                }
+                const int alive = 64 - __popcll(idle);
+                if (alive == 0) {
+                    int ok = 0;
+                    if (lane == 0) ok = wg_take(&M->free, donated, donated);
+                    if (__builtin_amdgcn_readfirstlane(ok)) break;
+                    __builtin_amdgcn_s_sleep(8);  // reserved lanes: their histories are on the way
+                    continue;
+                }
+                // hand the wave's histories over
+                if (may_give) {
+                    int ok = 0;
+                    if (lane == 0) {
+                        ok = wg_take(&M->free, donated + alive, donated + alive);
+                        int z = 0;
+                        if (ok && !wg_cas(&M->lock, z, 1)) {
+                            wg_add(&M->free, donated + alive);
+                            ok = 0;
+                        }
+                    }
+                    if (__builtin_amdgcn_readfirstlane(ok)) {
+                        if (S.st != RTA_DONE) rta_mail_write<GRAD>(mail + __popcll(~idle & below), S);
+                        if (lane == 0) {
+                            M->total = alive;
+                            __hip_atomic_store(&M->n, alive, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                        break;
+                    }
+                }
+            }
+        }
+        if (!flying) {
+            if (!exhausted && __ballot(S.st != RTA_DONE) == 0ULL) exhausted = true;  // no lane follows histories
+            continue;  // lanes that wait are served in the next pass
+        }
+        if ((flying >> lane) & 1ULL) rta_fly<GRAD, TM, POLY, GL, D>(P, G, T, A, S, C);
+    }
+    if constexpr (TM != 1) acc_flush<TM, D>(P, T, A);
+}
+
+// ids of the whole batch from the global counter, P.chunk at a time
+struct RtaTakeGlobal {
+    unsigned long long* next;
+    int chunk;
+    __device__ inline void operator()(int, unsigned long long& lo, unsigned long long& hi) const {
+        unsigned long long b = 0;
+        if ((threadIdx.x & 63) == 0) b = atomicAdd(next, (unsigned long long)chunk);
+        lo = __shfl(b, 0, 64);
+        hi = lo + chunk;
+    }
+};
+// ids of a work item from the workgroup's LDS counter, as many as lanes wait
+struct RtaTakeItem {
+    unsigned long long* next;
+    __device__ inline void operator()(int want, unsigned long long& lo, unsigned long long& hi) const {
+        unsigned long long b = 0;
+        if ((threadIdx.x & 63) == 0) b = atomicAdd(next, (unsigned long long)want);
+        lo = __shfl(b, 0, 64);
+        hi = lo + want;
+    }
+};
+
+// One launch follows the histories of all runs of a batch; ids of all runs
+// form one range, so a batch of runs of any sizes fills the GPU.
+// Bound by VALU issue while ids last (a pass is about 400 vector
+// instructions, three waves per SIMD) and by the latency of a pass times the
+// passes of the longest history after that. 1 um x 200 nm, 100 bins, 200 time
+// bins, 3000 modes, 1e6 particles: 16.2 ms with geometry, grid and mode
+// arrays read from global memory for every segment (57 scattered loads per
+// wave and segment; 15 of 64 lanes active), 10.7 ms with the geometry in LDS,
+// the mode in registers and the rare paths deferred, 7.0 ms with histories
+// changing waves, 6.2 ms with the exit test in selects, the segment's bins
+// found once and the rare paths' parameters read where they are used.
+template <bool GRAD, int TMK, bool POLY, bool GL>
+__global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams P) {
+    constexpr bool D = GRAD && TMK == 0;
+    const uint64_t xc = xcd_id() % RTA_NCOPY;
+    RtaGeo<GL> G;
+    G.bo = 0;
+    if constexpr (GL) {
+        rta_stage_boxes<POLY>(P, rta_lds, 0, P.nboxes, 0, P.nsides, 0);
+        rta_stage_grid(P, rta_lds);
+        G.box = rta_lds;
+        G.side = reinterpret_cast<const DevSide*>(rta_lds + P.geo_side);
+        G.grid = reinterpret_cast<const double*>(rta_lds + P.geo_grid);
+    } else {
+        G.box = reinterpret_cast<const unsigned char*>(P.rboxes);
+        G.side = P.sides;
+        G.grid = P.timegrid;
+    }
+    RtaTally T;
+    T.lds = rta_lds + P.geo_bytes;
+    T.row0 = 0;
+    T.lbins = (uint32_t)P.lbins;
+    T.lc = (TMK == 1 || TMK == 2) ? (uint32_t)P.lrows * (uint32_t)P.lbins : 0u;
+    T.g = P.gz + xc * 3 * P.cells;
+    T.dg = GRAD ? P.dgz + xc * 4 * P.cells : nullptr;
+    uint32_t words = 0;  // 8-byte words of the LDS tallies
+    if constexpr (TMK == 1) words = (P.lt_arrays * T.lc + 1) / 2;
+    if constexpr (TMK == 2) words = 3 * T.lc;
+    for (uint32_t j = threadIdx.x; j < words; j += blockDim.x) ((double*)T.lds)[j] = 0.;
+    rta_mig_init(P);
+    __syncthreads();
+    RtaCounts C;
+    rta_histories<GRAD, TMK, POLY, GL, D>(P, G, T, C, P.total, RtaTakeGlobal{P.counters + 2, P.chunk});
     if constexpr (TMK == 1) {
         __syncthreads();  // every history of the workgroup has ended
-        lt_flush<GRAD>(P, lt);
-        lt_counters(P.counters, C.events, C.crossings, C.stuck, C.badmirror, C.badtrans);
+        lt_flush<GRAD>(P, T);
     } else if constexpr (TMK == 2) {
-        acc_flush<2>(P, (double*)lt, A);
         __syncthreads();  // every lane has added its last cell
         // the workgroup's block, stored whole (rta_sum_parts_kernel adds the
         // blocks of all workgroups)
-        const uint32_t nf = 3u * (uint32_t)P.lrows * (uint32_t)P.lbins;
-        const double* g = (const double*)lt;
-        double* dst = P.part + (size_t)blockIdx.x * nf;
-        for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) dst[j] = g[j];
-        lt_counters(P.counters, C.events, C.crossings, C.stuck, C.badmirror, C.badtrans);
-    } else {
-        if constexpr (!GRAD) acc_flush<0>(P, nullptr, A);
-        block_add_u64(P.counters + 0, C.events);
-        block_add_u64(P.counters + 1, C.crossings);
-        block_add_u64(P.counters + 3, C.stuck);
-        block_add_u64(P.counters + 4, C.badmirror);
-        block_add_u64(P.counters + 5, C.badtrans);
+        const double* g = (const double*)T.lds;
+        double* dst = P.part + (size_t)blockIdx.x * words;
+        for (uint32_t j = threadIdx.x; j < words; j += blockDim.x) dst[j] = g[j];
     }
+    rta_add_counts(P, C);
 }
 
 // Tally mode 3: persistent workgroups (768 threads, one per CU) take work
 // items in order; the histories of an item (ids of one run) run with the
-// run's rows, as many leading time bins as fit, in an FP64 LDS block, which
-// is added into the XCD's tally copy once the item's last history has
-// ended. Later bins go to the copies by device atomics, as under mode 2. A
-// batch whose runs each fit a block of their own thus gets LDS sums where
-// one block for all runs would not hold a single time bin.
-template <bool POLY>
+// run's boxes, time grid and rows (as many leading time bins as fit) in an
+// FP64 LDS block, which is added into the XCD's tally copy once the item's
+// last history has ended. Later bins go to the copies by device atomics, as
+// under mode 2. A batch whose runs each fit a block of their own thus gets LDS
+// sums where one block for all runs would not hold a single time bin.
+template <bool POLY, bool GL>
 __global__ __launch_bounds__(768) void rta_history_items_kernel(RtaParams P) {
-    int* hd = reinterpret_cast<int*>(rta_lt);  // lrows, lbins, first row, item
-    double* L = reinterpret_cast<double*>(rta_lt) + 2;
     __shared__ unsigned long long next_id;
-    TallyAcc A;
-    RtaState S;
-    S.alive = 0;
-    RtaCounts C;
+    __shared__ int item;
     const uint64_t xc = xcd_id() % RTA_NCOPY;
+    if constexpr (GL) rta_stage_grid(P, rta_lds);
+    double* L = reinterpret_cast<double*>(rta_lds + P.geo_bytes);
+    RtaCounts C;
     for (;;) {
         __syncthreads();  // the previous item's block has been read
         if (threadIdx.x == 0) {
             const unsigned long long it = atomicAdd(P.counters + 6, 1ULL);
-            hd[3] = it < (unsigned long long)P.nitems ? (int)it : P.nitems;
-            if (it < (unsigned long long)P.nitems) {
-                const RtaItem I = P.items[it];
-                hd[0] = I.lrows;
-                hd[1] = I.lbins;
-                hd[2] = I.lrow0;
-                next_id = I.lo;
-            }
+            item = it < (unsigned long long)P.nitems ? (int)it : P.nitems;
+            if (it < (unsigned long long)P.nitems) next_id = P.items[it].lo;
         }
         __syncthreads();
-        const int it = __builtin_amdgcn_readfirstlane(hd[3]);
+        const int it = __builtin_amdgcn_readfirstlane(item);
         if (it >= P.nitems) break;
         // the item's fields as uniform scalars
-        const uint64_t ihi = P.items[it].hi;
-        const uint32_t lbins = (uint32_t)P.items[it].lbins, lrow0 = (uint32_t)P.items[it].lrow0;
-        const uint32_t lc = (uint32_t)P.items[it].lrows * lbins, nf = 3u * lc;
-        for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) L[j] = 0.;
-        __syncthreads();
-        // ids of the item from per-wave pools of 64, taken from next_id
-        unsigned long long pool_lo = 0, pool_hi = 0;
-        for (;;) {
-            if (S.alive) rta_watch(P, S, C);
-            unsigned long long pid = ~0ULL;
-            unsigned long long want = __ballot(!S.alive);
-            while (want) {
-                if (pool_lo == pool_hi) {
-                    unsigned long long base = 0;
-                    const int leader = __ffsll((long long)want) - 1;
-                    if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(&next_id, 64ULL);
-                    base = __shfl(base, leader, 64);
-                    pool_lo = base;
-                    pool_hi = base + 64;
-                }
-                const unsigned long long below = want & ((1ULL << (threadIdx.x & 63)) - 1ULL);
-                const unsigned long long rank = (unsigned long long)__popcll(below);
-                const unsigned long long take = min((unsigned long long)__popcll(want), pool_hi - pool_lo);
-                const bool mine = (want >> (threadIdx.x & 63)) & 1ULL;
-                if (mine && rank < take) pid = pool_lo + rank;
-                pool_lo += take;
-                want = __ballot(!S.alive && pid == ~0ULL);
-            }
-            if (!S.alive) {
-                if (pid >= ihi) break;
-                rta_start<false, POLY>(P, S, pid);
-            }
-            rta_event<false, 3, POLY>(P, L, A, S, C);
+        const RtaItem& I = P.items[it];
+        const uint32_t lbins = (uint32_t)I.lbins, lrow0 = (uint32_t)I.lrow0;
+        const uint32_t lc = (uint32_t)I.lrows * lbins, nf = 3u * lc;
+        RtaGeo<GL> G;
+        G.bo = I.box0;
+        G.run = I.run;
+        G.wscale = P.runs[I.run].wscale;
+        if constexpr (GL) {
+            rta_stage_boxes<POLY>(P, rta_lds, I.box0, I.nbox, I.side0, I.nsides, (int)lrow0);
+            G.box = rta_lds;
+            G.side = reinterpret_cast<const DevSide*>(rta_lds + P.geo_side);
+            G.grid = reinterpret_cast<const double*>(rta_lds + P.geo_grid);
+        } else {
+            // global boxes keep the batch's indices
+            G.bo = 0;
+            G.box = reinterpret_cast<const unsigned char*>(P.rboxes);
+            G.side = P.sides;
+            G.grid = P.timegrid;
         }
-        acc_flush<3>(P, L, A);
+        RtaTally T;
+        T.lds = L;
+        T.row0 = GL ? 0 : (int32_t)lrow0;  // staged records hold the run's own rows
+        T.lbins = lbins;
+        T.lc = lc;
+        T.g = P.gz + xc * 3 * P.cells + (GL ? (uint64_t)I.box0 * (uint64_t)P.nt : 0);
+        T.dg = nullptr;
+        for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) L[j] = 0.;
+        rta_mig_init(P);
+        __syncthreads();
+        rta_histories<false, 3, POLY, GL, false>(P, G, T, C, I.hi, RtaTakeItem{&next_id});
         __syncthreads();  // every history of the item has ended and added its last cell
         for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) {
             const double v = L[j];
@@ -714,11 +1087,7 @@ __global__ __launch_bounds__(768) void rta_history_items_kernel(RtaParams P) {
             atomicAdd(P.gz + xc * 3 * P.cells + (uint64_t)a * P.cells + cell, v);
         }
     }
-    block_add_u64(P.counters + 0, C.events);
-    block_add_u64(P.counters + 1, C.crossings);
-    block_add_u64(P.counters + 3, C.stuck);
-    block_add_u64(P.counters + 4, C.badmirror);
-    block_add_u64(P.counters + 5, C.badtrans);
+    rta_add_counts(P, C);
 }
 
 // clears the tallies and counters (a kernel rather than a memset so that the
@@ -785,18 +1154,16 @@ struct RtaBatch {
     DevBuf<DevSide> d_sides;
     DevBuf<int2> d_srange;
     DevBuf<double2> d_center;
-    DevBuf<double4> d_modes;
-    DevBuf<double2> d_ivel;
+    DevBuf<RtaMode> d_rmodes;
+    DevBuf<RtaBox> d_rboxes;
     DevBuf<int32_t> d_mirror, d_perm;
     DevBuf<uint2> d_scat, d_gen_sel, d_gen_tab, d_lam_tab;
     DevBuf<RtaGen> d_gens;
-    DevBuf<int4> d_lam_info;
     DevBuf<DevBox> d_boxes;
     DevBuf<DevContact> d_cts;
     DevBuf<double4> d_cseg;
     DevBuf<double2> d_ptrans;
     DevBuf<double> d_timegrid, d_tally, d_dgz;
-    DevBuf<uint64_t> d_box_cell;
     DevBuf<RtaRunDev> d_runs, d_trial_runs;
     DevBuf<unsigned long long> d_counters;
     // spectral decomposition (one run): locations, per-mode tallies, the
@@ -812,9 +1179,10 @@ struct RtaBatch {
     // 2 FP64 per-workgroup partial sums of the first lbins time bins in LDS
     // (one 768-thread workgroup per CU), later bins by device atomics
     int tally = 0, lt_goff[4] = {-1, -1, -1, -1};
-    uint32_t lrows = 0, lbins = 0;
-    size_t lt_bytes = 0, lg_bytes = 0;  // LDS of modes 1 and 2
-    DevBuf<uint32_t> d_box_lrow;
+    uint32_t lrows = 0;
+    int lt_arrays = 3;            // mode 1: FP32 arrays
+    int nboxes = 0, nsides = 0;   // over all runs
+    std::vector<int> side0, nside;  // per run: first polygon side and sides
     DevBuf<uint64_t> d_lrow_cell;
     DevBuf<double> d_part;  // mode 2: [blocks][3][lrows][lbins]
     // 3: per run, the first LDS row and the rows of its regular boxes; the
@@ -823,6 +1191,8 @@ struct RtaBatch {
     std::vector<RtaItem> items;
     DevBuf<RtaItem> d_items;
     size_t l3_bytes = 0;
+    int l3_nbox = 0, l3_nside = 0;  // boxes and sides of the largest run
+    bool l3_mail = true;
     bool use_graph = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -934,8 +1304,8 @@ static void build_mirrors(const Modes& m, std::vector<int32_t>& mir) {
 
 static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total) {
     RtaParams P{};
-    P.modes = b->d_modes.p;
-    P.ivel = b->d_ivel.p;
+    P.rmodes = b->d_rmodes.p;
+    P.rboxes = b->d_rboxes.p;
     P.mirror = b->d_mirror.p;
     P.scat = b->d_scat.p;
     P.boxes = b->d_boxes.p;
@@ -948,11 +1318,9 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
     P.gens = b->d_gens.p;
     P.gen_sel = b->d_gen_sel.p;
     P.gen_tab = b->d_gen_tab.p;
-    P.lam_info = b->d_lam_info.p;
     P.lam_tab = b->d_lam_tab.p;
     P.perm = b->d_perm.p;
     P.timegrid = b->d_timegrid.p;
-    P.box_cell = b->d_box_cell.p;
     P.runs = runs;
     P.gz = b->d_tally.p;
     P.jx = b->d_tally.p + b->cells;
@@ -963,16 +1331,16 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
     P.counters = b->d_counters.p;
     P.total = total;
     P.cells = b->cells;
-    P.max_iters = 1ULL << 26;
     P.maxtime = b->maxtime;
     P.n = b->m->n;
     P.nt = b->ntime - 1;
     P.nruns = b->nruns;
-    P.box_lrow = b->d_box_lrow.p;
     P.lrow_cell = b->d_lrow_cell.p;
     P.lrows = (int32_t)b->lrows;
     for (int k = 0; k < 4; k++) P.lt_goff[k] = b->lt_goff[k];
-    P.lbins = (int32_t)b->lbins;
+    P.lt_arrays = b->lt_arrays;
+    P.nboxes = b->nboxes;
+    P.nsides = b->nsides;
     P.part = b->d_part.p;
     P.idt = (double)(b->ntime - 1) / b->maxtime;
     P.items = b->d_items.p;
@@ -980,7 +1348,99 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
     return P;
 }
 
-static void launch_batch(RtaBatch* b, const RtaParams& P, int block, int blocks, hipStream_t s) {
+// LDS of a workgroup of the history kernels: the geometry and the time grid
+// when they take at most RTA_GEO_LDS bytes (see RtaGeo), then the tallies.
+struct RtaLds {
+    bool gl = false;
+    int32_t side = 0, grid = 0, geo = 0;  // byte offsets: sides, grid, tallies
+    int32_t mig = -1;                     // of the mailbox, before the tallies
+    uint32_t lbins = 0;                   // leading time bins of a tally row
+    size_t bytes = 0;
+};
+static RtaLds rta_lds_layout(int nboxes, int nsides, int nt) {
+    RtaLds L;
+    auto up16 = [](size_t v) { return (v + 15) & ~(size_t)15; };
+    const size_t side = (size_t)RTA_BOX_LDS * nboxes, grid = up16(side + sizeof(DevSide) * (size_t)nsides);
+    const size_t geo = up16(grid + sizeof(double) * ((size_t)nt + 1));
+    L.gl = geo <= RTA_GEO_LDS;
+    if (L.gl) {
+        L.side = (int32_t)side;
+        L.grid = (int32_t)grid;
+        L.geo = (int32_t)geo;
+    }
+    L.mig = L.geo;
+    L.geo += (int32_t)RTA_MIG_BYTES;
+    L.bytes = std::max<size_t>((size_t)L.geo, 16 * 2 * sizeof(uint64_t));  // rta_add_counts' space
+    return L;
+}
+// without the mailbox, where it would leave no room for one time bin
+static void drop_mail(RtaLds& L) {
+    L.geo = L.mig;
+    L.mig = -1;
+}
+// layout of tally modes 0, 1 and 2: rows of `arrays` tallies of `width`
+// bytes per bin, as many leading time bins as the workgroup's LDS holds (the
+// early bins carry most of the segments: particles enter at t = 0 and leave
+// through the reservoirs)
+static RtaLds rta_lds_of(const RtaBatch* b, int tally) {
+    const int nt = b->ntime - 1;
+    RtaLds L = rta_lds_layout(b->nboxes, b->nsides, nt);
+    if ((tally == 1 || tally == 2) && b->lrows) {
+        const size_t arrays = tally == 1 ? (size_t)b->lt_arrays : 3, width = tally == 1 ? sizeof(float) : sizeof(double);
+        const size_t per_bin = arrays * b->lrows * width;
+        if ((size_t)L.geo + per_bin > b->ctx->lds_per_block) drop_mail(L);
+        L.lbins = (uint32_t)std::min<size_t>((size_t)nt, (b->ctx->lds_per_block - (size_t)L.geo) / per_bin);
+        L.bytes = std::max<size_t>(L.bytes, ((size_t)L.geo + per_bin * L.lbins + 7) & ~(size_t)7);
+    }
+    return L;
+}
+static void set_lds(RtaParams& P, const RtaLds& L) {
+    P.geo_side = L.side;
+    P.geo_grid = L.grid;
+    P.geo_bytes = L.geo;
+    P.mig = L.mig;
+    P.lbins = (int32_t)L.lbins;
+}
+// Lanes of a wave that follow histories and ids a wave takes at a time. With
+// fewer particles than lanes they are spread over all waves (a wave with few
+// lanes skips the paths none of them takes, and all SIMDs work); ids are
+// handed out in pieces of at most a quarter of a wave's share, so that no
+// wave is left with a piece when the others have finished.
+static void set_shares(RtaParams& P, int block, int blocks, int cus) {
+    // a CU holds 12 waves of these kernels (at most 168 registers)
+    const uint64_t waves = (uint64_t)std::min(blocks * (block / 64), 12 * cus);
+    P.lanes = (int32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (P.total + waves - 1) / waves));
+    P.chunk = (int32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, P.total / (4 * waves)));
+    // histories stay where they are when every wave has only a few
+    if (P.lanes < 16) P.keep_waves = block / 64;
+    else P.keep_waves = std::max(1, block / 64 / 3);
+}
+
+using RtaKernel = void (*)(RtaParams);
+// the history kernel of a tally mode (0, 1 or 2) by [polygons][geometry in LDS]
+static RtaKernel rta_kernel(int tally, bool grad, bool poly, bool gl) {
+    static const RtaKernel plain[3][2][2] = {
+        {{rta_history_kernel<false, 0, false, false>, rta_history_kernel<false, 0, false, true>},
+         {rta_history_kernel<false, 0, true, false>, rta_history_kernel<false, 0, true, true>}},
+        {{rta_history_kernel<false, 1, false, false>, rta_history_kernel<false, 1, false, true>},
+         {rta_history_kernel<false, 1, true, false>, rta_history_kernel<false, 1, true, true>}},
+        {{rta_history_kernel<false, 2, false, false>, rta_history_kernel<false, 2, false, true>},
+         {rta_history_kernel<false, 2, true, false>, rta_history_kernel<false, 2, true, true>}}};
+    // rectangles only (specular sides)
+    static const RtaKernel with_grad[2][2] = {
+        {rta_history_kernel<true, 0, false, false>, rta_history_kernel<true, 0, false, true>},
+        {rta_history_kernel<true, 1, false, false>, rta_history_kernel<true, 1, false, true>}};
+    return grad ? with_grad[tally][gl] : plain[tally][poly][gl];
+}
+static RtaKernel rta_items_kernel(bool poly, bool gl) {
+    return poly ? (gl ? rta_history_items_kernel<true, true> : rta_history_items_kernel<true, false>)
+                : (gl ? rta_history_items_kernel<false, true> : rta_history_items_kernel<false, false>);
+}
+static void allow_lds(RtaKernel k, size_t bytes) {
+    HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+}
+
+static void launch_batch(RtaBatch* b, RtaParams P, int block, int blocks, hipStream_t s) {
     hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, b->d_tally.p, RTA_NCOPY * 3 * b->cells,
                        b->d_counters.p);
     if (b->any_grad)
@@ -989,32 +1449,23 @@ static void launch_batch(RtaBatch* b, const RtaParams& P, int block, int blocks,
     if (b->nloc)
         hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, b->d_spec.p,
                            (uint64_t)b->nloc * (b->ntime - 1) * b->m->n, b->d_counters.p);
+    set_shares(P, block, blocks, b->ctx->cu_count);
     if (b->tally == 3) {
-        if (b->poly)
-            hipLaunchKernelGGL(rta_history_items_kernel<true>, dim3(blocks), dim3(block), b->l3_bytes, s, P);
-        else
-            hipLaunchKernelGGL(rta_history_items_kernel<false>, dim3(blocks), dim3(block), b->l3_bytes, s, P);
-    } else if (b->tally == 2) {
-        if (b->poly)
-            hipLaunchKernelGGL((rta_history_kernel<false, 2, true>), dim3(blocks), dim3(block), b->lg_bytes, s, P);
-        else
-            hipLaunchKernelGGL((rta_history_kernel<false, 2>), dim3(blocks), dim3(block), b->lg_bytes, s, P);
-        const uint32_t nf = 3u * b->lrows * b->lbins;
-        hipLaunchKernelGGL(rta_sum_parts_kernel, dim3(std::min<uint32_t>((nf + 255) / 256, 4096u)), dim3(256), 0, s,
-                           b->d_tally.p, b->d_part.p, blocks, b->lrows, b->lbins, b->d_lrow_cell.p, b->cells);
-    } else if (b->tally == 1) {
-        if (b->any_grad)
-            hipLaunchKernelGGL((rta_history_kernel<true, 1>), dim3(blocks), dim3(block), b->lt_bytes, s, P);
-        else if (b->poly)
-            hipLaunchKernelGGL((rta_history_kernel<false, 1, true>), dim3(blocks), dim3(block), b->lt_bytes, s, P);
-        else
-            hipLaunchKernelGGL((rta_history_kernel<false, 1>), dim3(blocks), dim3(block), b->lt_bytes, s, P);
-    } else if (b->poly) {
-        hipLaunchKernelGGL((rta_history_kernel<false, 0, true>), dim3(blocks), dim3(block), 0, s, P);
-    } else if (b->any_grad) {
-        hipLaunchKernelGGL((rta_history_kernel<true, 0>), dim3(blocks), dim3(block), 0, s, P);
+        RtaLds L = rta_lds_layout(b->l3_nbox, b->l3_nside, b->ntime - 1);
+        if (!b->l3_mail) drop_mail(L);
+        set_lds(P, L);
+        P.lanes = 64;
+        P.keep_waves = std::max(1, block / 64 / 3);
+        hipLaunchKernelGGL(rta_items_kernel(b->poly, L.gl), dim3(blocks), dim3(block), b->l3_bytes, s, P);
     } else {
-        hipLaunchKernelGGL((rta_history_kernel<false, 0>), dim3(blocks), dim3(block), 0, s, P);
+        const RtaLds L = rta_lds_of(b, b->tally);
+        set_lds(P, L);
+        hipLaunchKernelGGL(rta_kernel(b->tally, b->any_grad, b->poly, L.gl), dim3(blocks), dim3(block), L.bytes, s, P);
+        if (b->tally == 2) {
+            const uint32_t nf = 3u * b->lrows * L.lbins;
+            hipLaunchKernelGGL(rta_sum_parts_kernel, dim3(std::min<uint32_t>((nf + 255) / 256, 4096u)), dim3(256), 0, s,
+                               b->d_tally.p, b->d_part.p, blocks, b->lrows, L.lbins, b->d_lrow_cell.p, b->cells);
+        }
     }
     // the per-XCD copies into copy 0
     hipLaunchKernelGGL(rta_sum_copies_kernel, dim3(1024), dim3(256), 0, s, b->d_tally.p, 3 * b->cells);
@@ -1037,13 +1488,6 @@ static void batch_create(RtaBatch* b) {
     b->timegrid.resize(b->ntime);
     for (int i = 0; i < b->ntime; i++) b->timegrid[i] = (double)i * b->maxtime / (b->ntime - 1);
     const int nt = b->ntime - 1;
-    std::vector<double4> md(n);
-    for (int i = 0; i < n; i++) md[i] = make_double4(m->vx[i], m->vy[i], m->w[i], m->omega[i]);
-    b->d_modes.upload(md, s);
-    std::vector<double2> iv(n);
-    for (int i = 0; i < n; i++)
-        iv[i] = make_double2(m->vx[i] != 0. ? 1.0 / m->vx[i] : 0., m->vy[i] != 0. ? 1.0 / m->vy[i] : 0.);
-    b->d_ivel.upload(iv, s);
     std::vector<int32_t> mir;
     build_mirrors(*m, mir);
     b->d_mirror.upload(mir, s);
@@ -1052,8 +1496,8 @@ static void batch_create(RtaBatch* b) {
     std::vector<DevContact> cts;
     std::vector<double4> cseg;
     std::vector<double2> ptrans;
-    std::vector<uint64_t> box_cell, lrow_cell;
-    std::vector<uint32_t> box_lrow;
+    std::vector<uint64_t> lrow_cell;
+    std::vector<RtaBox> rboxes;
     std::vector<RtaGen> gens;
     std::vector<uint2> gsel, gtab, scat;
     std::vector<double> pmf(n);
@@ -1106,6 +1550,7 @@ static void batch_create(RtaBatch* b) {
         b->nbox.push_back(nb);
         b->cell0.push_back(b->cells);
         b->run_lrow0.push_back((int32_t)b->lrows);
+        b->side0.push_back((int)sides.size());
         for (int i = 0; i < nb; i++) {
             DevBox d = g->dboxes[i];
             if (d.kind == 2 && d.tgt < 0)
@@ -1117,6 +1562,8 @@ static void batch_create(RtaBatch* b) {
             for (int k = 0; k < 4; k++)
                 if (d.side_nbr[k] >= 0) d.side_nbr[k] += bo;
             boxes.push_back(d);
+            RtaBox rb{d.xmin, d.xmax, d.ymin, d.ymax, {d.side_nbr[0], d.side_nbr[1], d.side_nbr[2], d.side_nbr[3]},
+                      d.kind, 0, (int)sides.size(), b->poly ? g->srange[i].y : 0};
             if (b->poly) {
                 const int2 sr = g->srange[i];
                 srange.push_back(make_int2((int)sides.size(), sr.y));
@@ -1135,11 +1582,15 @@ static void batch_create(RtaBatch* b) {
                 }
                 center.push_back(make_double2(g->boxes[i].cx(), g->boxes[i].cy()));
             }
-            box_cell.push_back(b->cells + (uint64_t)i * nt);
-            // only regular boxes tally (reservoirs absorb, periodic boxes translate)
-            box_lrow.push_back(d.kind == 0 ? b->lrows++ : ~0u);
-            if (d.kind == 0) lrow_cell.push_back(b->cells + (uint64_t)i * nt);
+            // only regular boxes tally (reservoirs absorb, periodic boxes
+            // translate); box i of the batch has the cells i nt ... i nt + nt - 1
+            if (d.kind == 0) {
+                rb.lrow = (int32_t)b->lrows++;
+                lrow_cell.push_back(b->cells + (uint64_t)i * nt);
+            }
+            rboxes.push_back(rb);
         }
+        b->nside.push_back((int)sides.size() - b->side0.back());
         for (auto ct : g->dcontacts) {
             ct.box += bo;
             cts.push_back(ct);
@@ -1150,7 +1601,6 @@ static void batch_create(RtaBatch* b) {
         // BE_derivative sampler at the run temperature (sampling.cpp:47-68)
         for (int i = 0; i < n; i++) pmf[i] = m->omega[i] <= 0. ? 0. : h_be_kernel(m->omega[i], D.T0) * m->w[i];
         if (!build_alias(pmf.data(), n, th.data(), al.data())) throw Error(BTE_EINVAL, "empty scattering pmf");
-        R.scat0 = (int32_t)scat.size();
         for (int i = 0; i < n; i++) scat.push_back(make_uint2(th[i], al[i]));
         // isothermal wall generators (RTA_MC2D.cpp:296-347, 366-397)
         std::vector<double> gw;
@@ -1185,6 +1635,9 @@ static void batch_create(RtaBatch* b) {
         b->total += D.nparticles;
     }
     b->d_boxes.upload(boxes, s);
+    b->d_rboxes.upload(rboxes, s);
+    b->nboxes = (int)boxes.size();
+    b->nsides = (int)sides.size();
     if (b->poly) {
         b->d_sides.upload(sides, s);
         b->d_srange.upload(srange, s);
@@ -1193,22 +1646,14 @@ static void batch_create(RtaBatch* b) {
     b->d_cts.upload(cts.empty() ? std::vector<DevContact>(1) : cts, s);
     b->d_cseg.upload(cseg.empty() ? std::vector<double4>(1) : cseg, s);
     b->d_ptrans.upload(ptrans, s);
-    b->d_box_cell.upload(box_cell, s);
-    b->d_box_lrow.upload(box_lrow, s);
     b->d_lrow_cell.upload(lrow_cell.empty() ? std::vector<uint64_t>(1) : lrow_cell, s);
-    // LDS block of the FP32 tallies: gz, jx, jy, then one array per side that
-    // some run differentiates; at least the counters' reduction space
+    // arrays of the FP32 tallies: gz, jx, jy, then one per side that some run
+    // differentiates
     int gunion = 0;
     for (auto& R : b->runs) gunion |= R.gmask;
-    int narr = 3;
+    b->lt_arrays = 3;
     for (int k = 0; k < 4; k++)
-        if ((gunion >> k) & 1) b->lt_goff[k] = narr++ * (int)(b->lrows * (uint32_t)nt);
-    b->lt_bytes = std::max<size_t>((size_t)narr * b->lrows * nt * sizeof(float), 16 * 5 * sizeof(uint64_t));
-    // mode 2: as many leading time bins of every LDS row as the workgroup's
-    // LDS holds in FP64 for gz, jx and jy (the early bins carry most of the
-    // segments: particles enter at t = 0 and leave through the reservoirs)
-    b->lbins = b->lrows ? (uint32_t)std::min<size_t>((size_t)nt, c->lds_per_block / (3 * sizeof(double) * b->lrows)) : 0;
-    b->lg_bytes = std::max<size_t>((size_t)3 * b->lrows * b->lbins * sizeof(double), 16 * 5 * sizeof(uint64_t));
+        if ((gunion >> k) & 1) b->lt_goff[k] = b->lt_arrays++;
     b->d_gens.upload(gens, s);
     b->d_gen_sel.upload(gsel, s);
     b->d_gen_tab.upload(gtab, s);
@@ -1219,7 +1664,11 @@ static void batch_create(RtaBatch* b) {
     std::vector<uint2> ltab;
     std::vector<int32_t> perm;
     build_lambert(*m, b->sigma > 0 ? b->sigma : 0.25, normals, info, ltab, perm);
-    b->d_lam_info.upload(info, s);
+    std::vector<RtaMode> rm(n);
+    for (int i = 0; i < n; i++)
+        rm[i] = RtaMode{m->vx[i], m->vy[i], m->vx[i] != 0. ? 1.0 / m->vx[i] : 0., m->vy[i] != 0. ? 1.0 / m->vy[i] : 0.,
+                        m->w[i], info[i].x, info[i].y, info[i].z, {0, 0, 0}};
+    b->d_rmodes.upload(rm, s);
     b->d_lam_tab.upload(ltab, s);
     b->d_perm.upload(perm, s);
     b->d_timegrid.upload(b->timegrid, s);
@@ -1352,25 +1801,29 @@ static void batch_set_tally(RtaBatch* b, int mode) {
         if (b->nloc) throw Error(BTE_EINVAL, "LDS tallies do not cover spectral locations");
         if (b->any_grad) throw Error(BTE_EINVAL, "tally mode 3 does not carry dT/dp; use mode 1 or 0");
         const int nt = b->ntime - 1;
-        // the block: a 16-byte header, then [3][rows][bins] doubles; a margin
-        // for the kernel's static LDS
-        const size_t avail = b->ctx->lds_per_block - 1024;
-        b->l3_bytes = 16 * 5 * sizeof(uint64_t);
+        // the block: the largest run's geometry and the time grid (see RtaGeo),
+        // then [3][rows][bins] doubles; a margin for the kernel's static LDS
+        b->l3_nbox = *std::max_element(b->nbox.begin(), b->nbox.end());
+        b->l3_nside = *std::max_element(b->nside.begin(), b->nside.end());
+        RtaLds L = rta_lds_layout(b->l3_nbox, b->l3_nside, nt);
+        const int32_t max_rows = *std::max_element(b->run_lrows.begin(), b->run_lrows.end());
+        b->l3_mail = (size_t)L.geo + 3 * sizeof(double) * (size_t)max_rows <= b->ctx->lds_per_block - 1024;
+        if (!b->l3_mail) drop_mail(L);
+        const size_t avail = b->ctx->lds_per_block - 1024 - (size_t)L.geo;
+        b->l3_bytes = L.bytes;
         std::vector<int32_t> lb(b->nruns, 0);
         for (int r = 0; r < b->nruns; r++) {
             const size_t rows = (size_t)b->run_lrows[r];
             if (rows == 0) continue;
-            if (16 + 3 * sizeof(double) * rows > avail)
+            if (16 + 3 * sizeof(double) * rows > b->ctx->lds_per_block - 1024)
                 throw Error(BTE_EINVAL, "run " + std::to_string(r) + ": FP64 LDS tallies need " +
                                             std::to_string(16 + 3 * sizeof(double) * rows) +
                                             " bytes of LDS for one time bin, the device has " +
-                                            std::to_string(avail) + " per workgroup");
-            lb[r] = (int32_t)std::min<size_t>((size_t)nt, (avail - 16) / (3 * sizeof(double) * rows));
-            b->l3_bytes = std::max(b->l3_bytes, 16 + 3 * sizeof(double) * rows * (size_t)lb[r]);
+                                            std::to_string(b->ctx->lds_per_block - 1024) + " per workgroup");
+            lb[r] = (int32_t)std::min<size_t>((size_t)nt, avail / (3 * sizeof(double) * rows));
+            b->l3_bytes = std::max(b->l3_bytes, (size_t)L.geo + 3 * sizeof(double) * rows * (size_t)lb[r]);
         }
-        HIPCHECK(hipFuncSetAttribute(b->poly ? reinterpret_cast<const void*>(&rta_history_items_kernel<true>)
-                                             : reinterpret_cast<const void*>(&rta_history_items_kernel<false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->l3_bytes));
+        allow_lds(rta_items_kernel(b->poly, L.gl), b->l3_bytes);
         b->block = 768;
         b->blocks = b->ctx->cu_count;
         // about eight items per workgroup (configuration 3 without the
@@ -1396,6 +1849,10 @@ static void batch_set_tally(RtaBatch* b, int mode) {
                 I.lrows = b->run_lrows[r];
                 I.lbins = lb[r];
                 I.run = r;
+                I.box0 = b->box0[r];
+                I.nbox = b->nbox[r];
+                I.side0 = b->side0[r];
+                I.nsides = b->nside[r];
                 b->items.push_back(I);
             }
         }
@@ -1404,28 +1861,28 @@ static void batch_set_tally(RtaBatch* b, int mode) {
     } else if (mode == 2) {
         if (b->nloc) throw Error(BTE_EINVAL, "LDS tallies do not cover spectral locations");
         if (b->any_grad) throw Error(BTE_EINVAL, "tally mode 2 does not carry dT/dp; use mode 1 or 0");
-        if (b->lbins == 0)
+        const RtaLds L = rta_lds_of(b, 2);
+        if (L.lbins == 0)
             throw Error(BTE_EINVAL, "FP64 LDS tallies need " + std::to_string(3 * sizeof(double) * b->lrows) +
                                         " bytes of LDS for one time bin, the device has " +
                                         std::to_string(b->ctx->lds_per_block) + " per workgroup");
-        HIPCHECK(hipFuncSetAttribute(b->poly ? reinterpret_cast<const void*>(&rta_history_kernel<false, 2, true>)
-                                             : reinterpret_cast<const void*>(&rta_history_kernel<false, 2>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->ctx->lds_per_block));
+        allow_lds(rta_kernel(2, false, b->poly, L.gl), b->ctx->lds_per_block);
         // two 768-thread workgroups per CU when two blocks fit its LDS (small
         // geometries), else one
         b->block = 768;
-        b->blocks = b->ctx->cu_count * (2 * b->lg_bytes <= b->ctx->lds_per_block ? 2 : 1);
-        const size_t np = (size_t)b->blocks * 3 * b->lrows * b->lbins;
+        b->blocks = b->ctx->cu_count * (2 * L.bytes <= b->ctx->lds_per_block ? 2 : 1);
+        const size_t np = (size_t)b->blocks * 3 * b->lrows * L.lbins;
         if (b->d_part.n < np) b->d_part.alloc(np);  // kept: a captured graph holds its address
     } else if (mode == 1) {
         if (b->nloc) throw Error(BTE_EINVAL, "FP32 LDS tallies do not cover spectral locations");
-        if (b->lt_bytes > b->ctx->lds_per_block)
-            throw Error(BTE_EINVAL, "FP32 LDS tallies need " + std::to_string(b->lt_bytes) + " bytes of LDS, the device has " +
+        // every time bin of every array has to fit next to nothing else: what
+        // the geometry displaces goes to device atomics
+        const size_t need = std::max<size_t>((size_t)b->lt_arrays * b->lrows * (size_t)(b->ntime - 1) * sizeof(float),
+                                             16 * 5 * sizeof(uint64_t));
+        if (need > b->ctx->lds_per_block)
+            throw Error(BTE_EINVAL, "FP32 LDS tallies need " + std::to_string(need) + " bytes of LDS, the device has " +
                                         std::to_string(b->ctx->lds_per_block) + " per workgroup");
-        const void* k = b->any_grad ? reinterpret_cast<const void*>(&rta_history_kernel<true, 1>)
-                        : b->poly   ? reinterpret_cast<const void*>(&rta_history_kernel<false, 1, true>)
-                                    : reinterpret_cast<const void*>(&rta_history_kernel<false, 1>);
-        HIPCHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->ctx->lds_per_block));
+        allow_lds(rta_kernel(1, b->any_grad, b->poly, rta_lds_of(b, 1).gl), b->ctx->lds_per_block);
         b->block = 768;
         b->blocks = b->ctx->cu_count;
     } else if (b->tally != 0) {
@@ -1551,11 +2008,16 @@ static void rta_execute_noalloc(RtaBatch* b, double* d_T, double* d_jx, double* 
     HIPCHECK(hipSetDevice(c->device));
     double* base = (double*)scratch_address(c->device);
     // the tally mode bte_rta_execute picks, without touching the handle's
-    const int mode = b->lbins > 0 ? 2 : 0;
+    const RtaLds L2 = rta_lds_of(b, 2);
+    const int mode = L2.lbins > 0 ? 2 : 0;
+    const RtaLds L = mode == 2 ? L2 : rta_lds_of(b, 0);
     const int block = mode == 2 ? 768 : 256, blocks = mode == 2 ? c->cu_count : c->cu_count * 8;
     const size_t ncopy = (size_t)RTA_NCOPY * 3 * b->cells;
     const size_t ncnt = 8;  // the counters, as unsigned 64-bit words
-    const size_t npart = mode == 2 ? (size_t)blocks * 3 * b->lrows * b->lbins : 0;
+    // the limit counts the time bins that a workgroup's whole LDS holds
+    const size_t full_bins = mode == 2 ? std::min<size_t>((size_t)(b->ntime - 1),
+                                                          c->lds_per_block / (3 * sizeof(double) * b->lrows)) : 0;
+    const size_t npart = mode == 2 ? (size_t)blocks * 3 * b->lrows * full_bins : 0;
     const size_t need = (ncopy + ncnt + npart) * sizeof(double);
     if (need > RTA_SCRATCH_BYTES)
         throw Error(BTE_EINVAL, "bte_rta_execute_noalloc needs " + std::to_string(need) +
@@ -1573,15 +2035,15 @@ static void rta_execute_noalloc(RtaBatch* b, double* d_T, double* d_jx, double* 
     // the counters start at zero (a kernel, not a memset, so that a graph
     // capture records no memset node); the partial blocks are overwritten
     hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, base, (uint64_t)ncopy, P.counters);
+    set_lds(P, L);
+    set_shares(P, block, blocks, c->cu_count);
+    const RtaKernel k = rta_kernel(mode, false, false, L.gl);
+    if (mode == 2) allow_lds(k, c->lds_per_block);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(block), L.bytes, s, P);
     if (mode == 2) {
-        HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&rta_history_kernel<false, 2>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_per_block));
-        hipLaunchKernelGGL((rta_history_kernel<false, 2>), dim3(blocks), dim3(block), b->lg_bytes, s, P);
-        const uint32_t nf = 3u * b->lrows * b->lbins;
+        const uint32_t nf = 3u * b->lrows * L.lbins;
         hipLaunchKernelGGL(rta_sum_parts_kernel, dim3(std::min<uint32_t>((nf + 255) / 256, 4096u)), dim3(256), 0, s,
-                           base, P.part, blocks, b->lrows, b->lbins, b->d_lrow_cell.p, b->cells);
-    } else {
-        hipLaunchKernelGGL((rta_history_kernel<false, 0>), dim3(blocks), dim3(block), 0, s, P);
+                           base, P.part, blocks, b->lrows, L.lbins, b->d_lrow_cell.p, b->cells);
     }
     hipLaunchKernelGGL(rta_sum_copies_kernel, dim3(1024), dim3(256), 0, s, base, 3 * b->cells);
     const int nb = b->nbox[0], nt = b->ntime - 1;
@@ -1685,7 +2147,7 @@ int bte_rta_execute(bte_rta* rr, double* T_out, double* jx_out, double* jy_out, 
     // FP64 LDS partial sums of the leading time bins (tally mode 2: the same
     // histories and FP64 sums) whenever one time bin of every box fits;
     // device atomics with spectral locations
-    const int want = (!b->nloc && !b->any_grad && b->lbins > 0) ? 2 : 0;
+    const int want = (!b->nloc && !b->any_grad && rta_lds_of(b, 2).lbins > 0) ? 2 : 0;
     if (b->tally != want) batch_set_tally(b, want);
     bte_rta_batch_report br{};
     double E = 0;

@@ -241,8 +241,9 @@ int bte_rta_batch_create(bte_ctx* ctx, const bte_modes* m, int nruns, const bte_
  * thread-local arrays, RTA_MC2D.cpp:699-769 and 2326-2335). mode 0 (default):
  * FP64 device atomics. mode 1: every workgroup sums its segments in FP32
  * arrays in LDS (T, jx, jy and each differentiated side over the regular
- * boxes' cells) and adds them into the FP64 tallies once at the end; one
- * 768-thread workgroup per CU. BTE_EINVAL when those arrays exceed the
+ * boxes' cells; the last time bins go to the FP64 tallies by device atomics
+ * where the workgroup's geometry takes their room) and adds them into the
+ * FP64 tallies once at the end; one 768-thread workgroup per CU. BTE_EINVAL when those arrays exceed the
  * device's LDS per workgroup. mode 2: FP64 sums of T, jx and jy in LDS for
  * as many leading time bins of all regular boxes as fit, later bins by FP64
  * device atomics. mode 3: as mode 2 with each workgroup working through

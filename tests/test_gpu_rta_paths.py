@@ -1,0 +1,107 @@
+"""The history kernels' routes: boxes, polygon sides and time grid in LDS or,
+past 20 KB, in global memory; waves with one lane up to full waves; histories
+that change waves once the ids have run out. A run's histories depend on its
+seed and particle ids only, so every route gives the same event and crossing
+counts and, up to the order of the FP64 sums, the same T, jx and jy (1e-10 of
+the largest magnitude, as in the tally-mode tests)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+KW = dict(thickness=1.0, dt=10.0, maxtime=400.0, sigma_bounce=2.0)
+
+
+def _modes(pkg, ctx, n=300, mirror=True):
+    m = pkg.workloads.material(n, seed=3, mirror=mirror)
+    return pkg.ModeTable(ctx, m["omega"], m["vx"], m["vy"], m["w"], m["V"], m["lattz"])
+
+
+def _ribbon(pkg, ctx, nb, width=40.0, dx=10.0, poly=False):
+    rect, kind, teq, _ = pkg.workloads.ribbon(nb * dx, width, nb, 300.0, reservoirs=(300.5, 299.5))
+    polys = None
+    if poly:
+        # slanted shared sides: neighbours meet along x = k dx +- 2 (bottom to top)
+        polys = [np.array([[r[0], r[2]], [r[1], r[2]], [r[1], r[3]], [r[0], r[3]]]) for r in rect]
+        for k in range(nb):
+            if k > 0:
+                polys[k][3, 0] += 2.0
+            if k < nb - 1:
+                polys[k][2, 0] += 2.0
+    return pkg.Geometry(ctx, rect, kind, teq, polys=polys)
+
+
+def _same(a, b):
+    for key, off in (("T", 300.0), ("jx", 0.0), ("jy", 0.0)):
+        scale = np.abs(b[key] - off).max()
+        np.testing.assert_allclose(a[key] - off, b[key] - off, rtol=0, atol=1e-10 * scale)
+
+
+# in LDS: 80 B a box, 56 B a polygon side, 8 B a time step, at most 20480 B;
+# 250 rectangles or 70 quadrilaterals are the last that fit next to 41 steps
+@pytest.mark.parametrize("tally", ["fp64", "fp64-lds", "fp64-lds-runs", "fp32-lds"])
+@pytest.mark.parametrize("poly,nb", [(False, 8), (False, 249), (False, 251), (True, 9), (True, 75)])
+def test_geometry_in_lds_and_in_global_memory(pkg, ctx, tally, poly, nb):
+    """One ribbon alone (its geometry in LDS while it fits) and beside a second
+    ribbon that takes the batch past the LDS limit."""
+    modes = _modes(pkg, ctx)
+    geom, other = _ribbon(pkg, ctx, nb, poly=poly), _ribbon(pkg, ctx, 260, poly=poly)
+    run = dict(geom=geom, T0=300.0, nparticles=30000, seed=5)
+    kw = dict(KW)
+    if tally == "fp32-lds":
+        kw.update(dt=80.0)  # every time bin of every box has to fit in LDS
+    tol = 1e-4 if tally == "fp32-lds" else 1e-10
+    ref_b = pkg.RtaBatch(ctx, modes, [run], **kw)
+    (ref,), rep = ref_b.execute()
+    ref_b.close()
+    one = pkg.RtaBatch(ctx, modes, [run], tally=tally, **kw)
+    (got,), grep = one.execute()
+    one.close()
+    assert (grep["events"], grep["crossings"]) == (rep["events"], rep["crossings"])
+    both = [got]
+    if tally != "fp32-lds" or not poly:
+        two = pkg.RtaBatch(ctx, modes, [run, dict(geom=other, T0=300.0, nparticles=100, seed=6)], tally=tally, **kw)
+        res, _ = two.execute()
+        two.close()
+        both.append(res[0])
+    for g in both:
+        for key, off in (("T", 300.0), ("jx", 0.0), ("jy", 0.0)):
+            scale = np.abs(ref[key] - off).max()
+            assert scale > 0
+            np.testing.assert_allclose(g[key] - off, ref[key] - off, rtol=0, atol=tol * scale)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 3071, 3073, 50000, 200001])
+def test_particle_counts_around_the_lanes_of_the_gpu(pkg, ctx, n):
+    """From one history to more than one per lane: waves with a single lane,
+    partly filled waves and refills, under every tally mode."""
+    modes = _modes(pkg, ctx)
+    run = dict(geom=_ribbon(pkg, ctx, 12), T0=300.0, nparticles=n, seed=9, specularity=(0.0, 0.5, 1.0, 0.0))
+    out = {}
+    for tally in ("fp64", "fp64-lds", "fp64-lds-runs", "fp32-lds"):
+        b = pkg.RtaBatch(ctx, modes, [run], tally=tally, **KW)
+        (out[tally],), rep = b.execute()
+        b.close()
+        out[tally]["counts"] = (rep["events"], rep["crossings"])
+    for tally in ("fp64-lds", "fp64-lds-runs"):
+        assert out[tally]["counts"] == out["fp64"]["counts"]
+        _same(out[tally], out["fp64"])
+    assert out["fp32-lds"]["counts"] == out["fp64"]["counts"]
+
+
+def test_scores_move_with_their_histories(pkg, ctx):
+    """dT/dp in FP64 tallies: the ribbon alone (LDS geometry) and in a batch
+    past the LDS limit (global geometry)."""
+    modes = _modes(pkg, ctx)
+    run = dict(geom=_ribbon(pkg, ctx, 20), T0=300.0, nparticles=60000, seed=11, specularity=(0.0, 0.4, 0.6, 0.0),
+               grad=True)
+    a = pkg.RtaBatch(ctx, modes, [run], **KW)
+    (ra,), rep_a = a.execute(grad=True)
+    a.close()
+    b = pkg.RtaBatch(ctx, modes, [run, dict(geom=_ribbon(pkg, ctx, 260), T0=300.0, nparticles=100, seed=6)], **KW)
+    rb, _ = b.execute(grad=True)
+    b.close()
+    _same(rb[0], ra)
+    scale = np.abs(ra["dTdp"]).max()
+    assert scale > 0
+    np.testing.assert_allclose(rb[0]["dTdp"], ra["dTdp"], rtol=0, atol=1e-10 * scale)
