@@ -267,9 +267,9 @@ class RtaBatch(_Handle):
     when the regular boxes' cells do not fit in LDS), "fp64-lds" (FP64
     per-workgroup sums of T, jx and jy in LDS for the leading time bins that
     fit, later bins by device atomics; no dT/dp) or "fp64-lds-runs" (the same
-    with each workgroup's LDS holding the rows of one run at a time: work
-    items of one run's particles, so batches of many runs keep as many time
-    bins in LDS as a single run; no dT/dp)."""
+    with each workgroup's LDS holding the rows of the one run it follows
+    at a time, so batches of many runs keep as many time bins in LDS as a
+    single run; no dT/dp)."""
     _destroy = "bte_rta_batch_destroy"
 
     def __init__(self, ctx, modes, runs, thickness, dt, maxtime, sigma_bounce=0.25, use_graph=False,

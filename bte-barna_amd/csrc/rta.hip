@@ -35,14 +35,13 @@ struct RtaRunDev {
     float spec[4];                         // specular probability per side
 };
 
-// Tally mode 3: a contiguous range of one run's particle ids, taken whole by
-// one workgroup, and the run's rows in the workgroup's FP64 LDS block.
-struct RtaItem {
-    uint64_t lo, hi;     // particle ids [lo, hi)
+// Tally mode 3: one run of the batch and its rows in the FP64 LDS block of a
+// workgroup that follows its histories.
+struct RtaRunRows {
     int32_t lrow0;       // global LDS row of the run's first regular box
     int32_t lrows;       // the run's regular boxes
     int32_t lbins;       // leading time bins of each row held in LDS
-    int32_t run;
+    int32_t wgs;         // workgroups that begin with this run
     int32_t box0, nbox, side0, nsides;  // the run's boxes and polygon sides
 };
 
@@ -108,13 +107,15 @@ struct RtaParams {
     // 2), the byte offsets of the sides and the time grid after the boxes and
     // of the tallies after both
     int32_t nboxes, nsides, geo_side, geo_grid, geo_bytes;
-    int32_t lanes;  // lanes of a wave that follow histories
-    int32_t chunk;  // particle ids a wave takes at a time
-    int32_t mig, keep_waves;  // LDS offset of the mailbox (-1: none); waves that keep their histories
+    int32_t mig;    // byte offset of the mailbox (-1: none)
+    int32_t waves;  // waves that share the particles (modes 0 to 2)
     double idt;  // nt / maxtime: time -> bin estimate on the uniform grid
-    // tally mode 3: the work items, taken in order through counters[6]
-    const RtaItem* items;
-    int32_t nitems, pad3;
+    // tally mode 3: the runs' rows, the run each workgroup begins with (-1:
+    // none), and per run the next particle (from 0) and the workgroups on it
+    const RtaRunRows* rows;
+    const int32_t* first_run;
+    unsigned long long* run_next;
+    unsigned long long* run_wgs;
 };
 
 // Per-XCD copies of the f64 tallies. Device-wide f64 atomics to a few
@@ -276,7 +277,7 @@ struct RtaCounts {
 // TM (tally mode) 0: FP64 device atomics. 1: the workgroup's FP32 partial
 // sums in LDS for the leading lbins bins, later ones by device atomics. 2: the
 // same with FP64 partial sums. 3: as 2 with the LDS block holding only the
-// rows of the run of the workgroup's current work item. All modes but 1
+// rows of the run that the workgroup follows. All modes but 1
 // merge consecutive contributions to one cell in the lane's accumulator.
 template <bool GRAD, int TM, bool D>
 __device__ inline void tally_bin(const RtaParams& P, const RtaTally& T, TallyAcc<D>& A, const RtaState& S, int lrow,
@@ -802,31 +803,51 @@ __device__ inline void rta_mail_read(const RtaParams& P, const RtaGeo<GL>& G, co
     rta_look<TM>(P, G, S);
 }
 
+// How a wave shares `total` particles with `waves` waves. With fewer particles
+// than lanes they are spread over all waves (a wave with few lanes skips the
+// paths none of them takes, and all SIMDs work); ids are handed out in pieces
+// of at most a quarter of a wave's share, so that no wave is left with a
+// piece when the others have finished. Histories stay where they are when
+// every wave has only a few.
+struct RtaShare {
+    int lanes;       // lanes that follow histories
+    int chunk;       // particle ids taken at a time
+    int keep_waves;  // leading waves of the workgroup that keep their histories
+};
+__device__ inline RtaShare rta_share(unsigned long long total, unsigned waves, int threads) {
+    const unsigned long long per = (total + waves - 1) / waves;
+    RtaShare W;
+    W.lanes = (int)min(64ULL, max(1ULL, per));
+    W.chunk = (int)min(64ULL, max(1ULL, per / 4));
+    W.keep_waves = W.lanes < 16 ? threads / 64 : max(1, threads / 64 / 3);
+    return W;
+}
+
 // Follows histories until the ids run out: one particle history per lane at a
 // time. Per pass the lanes in FRESH or FLY make one event; the lanes that
 // wait (pending sides, ended histories) are served together once an eighth of
 // the live lanes wait for a side or RTA_REFILL_MIN for an id, or no lane of the
 // wave can fly, so the code of those paths, which a few lanes per pass would
 // run with the rest of the wave idle, runs every few passes with more lanes
-// in it. take(want, lo, hi) hands the wave a range of at least one id (ids at
-// or past `end` mean that there is none left). Streams are keyed by the
+// in it. take(lo, hi) hands the wave a range of at least one id (ids at or
+// past `end` mean that there is none left). Streams are keyed by the
 // particle id and kept with the history, so the order of ids and of events
 // between lanes changes nothing in any history.
 #define RTA_REFILL_MIN 8
 template <bool GRAD, int TM, bool POLY, bool GL, bool D, class Take>
 __device__ inline void rta_histories(const RtaParams& P, const RtaGeo<GL>& G, const RtaTally& T, RtaCounts& C,
-                                     unsigned long long end, Take take) {
+                                     unsigned long long end, RtaShare W, Take take) {
     TallyAcc<D> A;
     RtaState S;
     const int lane = threadIdx.x & 63;
     const unsigned long long below = (1ULL << lane) - 1ULL;
-    S.st = lane < P.lanes ? RTA_DEAD : RTA_DONE;
+    S.st = lane < W.lanes ? RTA_DEAD : RTA_DONE;
     const auto can_fly = [&S] { return S.st == RTA_FRESH || S.st == RTA_FLY; };
     unsigned long long pool_lo = 0, pool_hi = 0;
     bool exhausted = false;  // no id left
     RtaMig* M = reinterpret_cast<RtaMig*>(rta_lds + P.mig);
     uint64_t* mail = reinterpret_cast<uint64_t*>(rta_lds + P.mig + sizeof(RtaMig));
-    const bool may_give = (int)(threadIdx.x >> 6) >= P.keep_waves;
+    const bool may_give = (int)(threadIdx.x >> 6) >= W.keep_waves;
     int donated = 0;
     uint32_t tick = 0;
     for (;;) {
@@ -841,7 +862,7 @@ __device__ inline void rta_histories(const RtaParams& P, const RtaGeo<GL>& G, co
             unsigned long long pid = ~0ULL;
             while (dead && !exhausted) {
                 if (pool_lo == pool_hi) {
-                    take(__popcll(dead), pool_lo, pool_hi);
+                    take(pool_lo, pool_hi);
                     exhausted = pool_lo >= end;
                 }
                 const unsigned long long rank = (unsigned long long)__popcll(dead & below);
@@ -943,25 +964,16 @@ __device__ inline void rta_histories(const RtaParams& P, const RtaGeo<GL>& G, co
     if constexpr (TM != 1) acc_flush<TM, D>(P, T, A);
 }
 
-// ids of the whole batch from the global counter, P.chunk at a time
-struct RtaTakeGlobal {
+// Particle ids base + 0, 1, ... from a counter in global memory, `chunk` at a time.
+struct RtaTake {
     unsigned long long* next;
+    unsigned long long base;
     int chunk;
-    __device__ inline void operator()(int, unsigned long long& lo, unsigned long long& hi) const {
+    __device__ inline void operator()(unsigned long long& lo, unsigned long long& hi) const {
         unsigned long long b = 0;
         if ((threadIdx.x & 63) == 0) b = atomicAdd(next, (unsigned long long)chunk);
-        lo = __shfl(b, 0, 64);
+        lo = base + __shfl(b, 0, 64);
         hi = lo + chunk;
-    }
-};
-// ids of a work item from the workgroup's LDS counter, as many as lanes wait
-struct RtaTakeItem {
-    unsigned long long* next;
-    __device__ inline void operator()(int want, unsigned long long& lo, unsigned long long& hi) const {
-        unsigned long long b = 0;
-        if ((threadIdx.x & 63) == 0) b = atomicAdd(next, (unsigned long long)want);
-        lo = __shfl(b, 0, 64);
-        hi = lo + want;
     }
 };
 
@@ -1007,7 +1019,9 @@ __global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams 
     rta_mig_init(P);
     __syncthreads();
     RtaCounts C;
-    rta_histories<GRAD, TMK, POLY, GL, D>(P, G, T, C, P.total, RtaTakeGlobal{P.counters + 2, P.chunk});
+    const RtaShare W = rta_share(P.total, (unsigned)P.waves, (int)blockDim.x);
+    rta_histories<GRAD, TMK, POLY, GL, D>(P, G, T, C, P.total, W,
+                                             RtaTake{P.counters + 2, 0, W.chunk});
     if constexpr (TMK == 1) {
         __syncthreads();  // every history of the workgroup has ended
         lt_flush<GRAD>(P, T);
@@ -1022,39 +1036,77 @@ __global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams 
     rta_add_counts(P, C);
 }
 
-// Tally mode 3: persistent workgroups (768 threads, one per CU) take work
-// items in order; the histories of an item (ids of one run) run with the
-// run's boxes, time grid and rows (as many leading time bins as fit) in an
-// FP64 LDS block, which is added into the XCD's tally copy once the item's
-// last history has ended. Later bins go to the copies by device atomics, as
-// under mode 2. A batch whose runs each fit a block of their own thus gets LDS
-// sums where one block for all runs would not hold a single time bin.
+// Tally mode 3: persistent workgroups (768 threads, one per CU) follow one run's
+// histories at a time, with the run's boxes, time grid and rows (as many
+// leading time bins as fit) in an FP64 LDS block. Ids come from the run's
+// counter, so a workgroup stays on its run until every id is taken; once its
+// last history has ended, the block is added into the XCD's tally copy and the
+// workgroup joins the run with the most particles left per workgroup. Later
+// bins go to the copies by device atomics, as under mode 2. A batch whose runs
+// each fit a block of their own thus gets LDS sums where one block for all
+// runs would not hold a single time bin.
+// The wait for the longest history (2900 passes against 160 on average for
+// 1 um over 5 ns) is paid once per run that a workgroup follows: 16 runs of
+// 3e4 to 1e6 particles take 17.3 ms, against 28.6 ms with the ids in items of
+// 4096 or more, each of which ended with that wait.
+
+// The run a workgroup turns to, by its first wave: the first_run entry, then
+// the run with the most particles left per workgroup on it, where those fill
+// the lanes of one more (or nobody follows it). -1: none is left.
+__device__ inline int rta_pick_run(const RtaParams& P, bool first) {
+    const int lane = threadIdx.x & 63;
+    int run = first ? P.first_run[blockIdx.x] : -1;
+    if (run < 0) {
+        unsigned long long best = 0;
+        for (int r = lane; r < P.nruns; r += 64) {
+            const unsigned long long n = P.runs[r].count;
+            const unsigned long long at = __hip_atomic_load(P.run_next + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long w = __hip_atomic_load(P.run_wgs + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (at >= n || (w > 0 && n - at < (w + 1) * blockDim.x)) continue;
+            const unsigned long long share = (n - at) / (w + 1) + 1;
+            if (share > best) {
+                best = share;
+                run = r;
+            }
+        }
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long b = __shfl_xor(best, d, 64);
+            const int r = __shfl_xor(run, d, 64);
+            if (b > best || (b == best && r > run)) {
+                best = b;
+                run = r;
+            }
+        }
+    }
+    if (run >= 0 && lane == 0) atomicAdd(P.run_wgs + run, 1ULL);
+    return run;
+}
+
 template <bool POLY, bool GL>
-__global__ __launch_bounds__(768) void rta_history_items_kernel(RtaParams P) {
-    __shared__ unsigned long long next_id;
-    __shared__ int item;
+__global__ __launch_bounds__(768) void rta_history_runs_kernel(RtaParams P) {
+    __shared__ int picked;
     const uint64_t xc = xcd_id() % RTA_NCOPY;
     if constexpr (GL) rta_stage_grid(P, rta_lds);
     double* L = reinterpret_cast<double*>(rta_lds + P.geo_bytes);
     RtaCounts C;
-    for (;;) {
-        __syncthreads();  // the previous item's block has been read
-        if (threadIdx.x == 0) {
-            const unsigned long long it = atomicAdd(P.counters + 6, 1ULL);
-            item = it < (unsigned long long)P.nitems ? (int)it : P.nitems;
-            if (it < (unsigned long long)P.nitems) next_id = P.items[it].lo;
+    for (bool first = true;; first = false) {
+        __syncthreads();  // the previous run's block has been read
+        if (threadIdx.x < 64) {
+            const int r = rta_pick_run(P, first);
+            if (threadIdx.x == 0) picked = r;
         }
         __syncthreads();
-        const int it = __builtin_amdgcn_readfirstlane(item);
-        if (it >= P.nitems) break;
-        // the item's fields as uniform scalars
-        const RtaItem& I = P.items[it];
+        const int run = __builtin_amdgcn_readfirstlane(picked);
+        if (run < 0) break;
+        // the run's fields as uniform scalars
+        const RtaRunRows& I = P.rows[run];
         const uint32_t lbins = (uint32_t)I.lbins, lrow0 = (uint32_t)I.lrow0;
         const uint32_t lc = (uint32_t)I.lrows * lbins, nf = 3u * lc;
+        const unsigned long long count = P.runs[run].count, first_id = P.runs[run].first;
         RtaGeo<GL> G;
         G.bo = I.box0;
-        G.run = I.run;
-        G.wscale = P.runs[I.run].wscale;
+        G.run = run;
+        G.wscale = P.runs[run].wscale;
         if constexpr (GL) {
             rta_stage_boxes<POLY>(P, rta_lds, I.box0, I.nbox, I.side0, I.nsides, (int)lrow0);
             G.box = rta_lds;
@@ -1077,8 +1129,12 @@ __global__ __launch_bounds__(768) void rta_history_items_kernel(RtaParams P) {
         for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) L[j] = 0.;
         rta_mig_init(P);
         __syncthreads();
-        rta_histories<false, 3, POLY, GL, false>(P, G, T, C, I.hi, RtaTakeItem{&next_id});
-        __syncthreads();  // every history of the item has ended and added its last cell
+        // a workgroup that begins with the run takes its share of the
+        // particles, one that joins fills its lanes
+        const RtaShare W = rta_share(count, first ? (unsigned)I.wgs * (blockDim.x / 64) : 1u, (int)blockDim.x);
+        rta_histories<false, 3, POLY, GL, false>(P, G, T, C, first_id + count, W,
+                                                 RtaTake{P.run_next + run, first_id, W.chunk});
+        __syncthreads();  // every history of the run has ended and added its last cell
         for (uint32_t j = threadIdx.x; j < nf; j += blockDim.x) {
             const double v = L[j];
             if (v == 0.) continue;
@@ -1086,16 +1142,19 @@ __global__ __launch_bounds__(768) void rta_history_items_kernel(RtaParams P) {
             const uint64_t cell = P.lrow_cell[lrow0 + row] + (r - row * lbins);
             atomicAdd(P.gz + xc * 3 * P.cells + (uint64_t)a * P.cells + cell, v);
         }
+        if (threadIdx.x == 0) atomicAdd(P.run_wgs + run, ~0ULL);  // - 1
     }
     rta_add_counts(P, C);
 }
 
 // clears the tallies and counters (a kernel rather than a memset so that the
 // launch sequence can be captured in a graph)
-__global__ __launch_bounds__(256) void rta_clear_kernel(double* a, uint64_t n, unsigned long long* cnt) {
+__global__ __launch_bounds__(256) void rta_clear_kernel(double* a, uint64_t n, unsigned long long* cnt,
+                                                       int ncnt) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         a[i] = 0.;
-    if (blockIdx.x == 0 && threadIdx.x < 8) cnt[threadIdx.x] = 0ULL;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < ncnt; i += blockDim.x) cnt[i] = 0ULL;
 }
 
 // running sum over the time bins of every (location, mode) column: the step
@@ -1185,11 +1244,11 @@ struct RtaBatch {
     std::vector<int> side0, nside;  // per run: first polygon side and sides
     DevBuf<uint64_t> d_lrow_cell;
     DevBuf<double> d_part;  // mode 2: [blocks][3][lrows][lbins]
-    // 3: per run, the first LDS row and the rows of its regular boxes; the
-    // work items and the LDS bytes of the largest run block (with header)
+    // 3: per run, the first LDS row and the rows of its regular boxes; their
+    // device records, the run each workgroup begins with and the LDS bytes
     std::vector<int32_t> run_lrow0, run_lrows;
-    std::vector<RtaItem> items;
-    DevBuf<RtaItem> d_items;
+    DevBuf<RtaRunRows> d_rows;
+    DevBuf<int32_t> d_first_run;
     size_t l3_bytes = 0;
     int l3_nbox = 0, l3_nside = 0;  // boxes and sides of the largest run
     bool l3_mail = true;
@@ -1343,8 +1402,10 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
     P.nsides = b->nsides;
     P.part = b->d_part.p;
     P.idt = (double)(b->ntime - 1) / b->maxtime;
-    P.items = b->d_items.p;
-    P.nitems = (int32_t)b->items.size();
+    P.rows = b->d_rows.p;
+    P.first_run = b->d_first_run.p;
+    P.run_next = b->d_counters.p + 8;
+    P.run_wgs = P.run_next + b->nruns;
     return P;
 }
 
@@ -1401,20 +1462,8 @@ static void set_lds(RtaParams& P, const RtaLds& L) {
     P.mig = L.mig;
     P.lbins = (int32_t)L.lbins;
 }
-// Lanes of a wave that follow histories and ids a wave takes at a time. With
-// fewer particles than lanes they are spread over all waves (a wave with few
-// lanes skips the paths none of them takes, and all SIMDs work); ids are
-// handed out in pieces of at most a quarter of a wave's share, so that no
-// wave is left with a piece when the others have finished.
-static void set_shares(RtaParams& P, int block, int blocks, int cus) {
-    // a CU holds 12 waves of these kernels (at most 168 registers)
-    const uint64_t waves = (uint64_t)std::min(blocks * (block / 64), 12 * cus);
-    P.lanes = (int32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (P.total + waves - 1) / waves));
-    P.chunk = (int32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, P.total / (4 * waves)));
-    // histories stay where they are when every wave has only a few
-    if (P.lanes < 16) P.keep_waves = block / 64;
-    else P.keep_waves = std::max(1, block / 64 / 3);
-}
+// waves that run at a time: a CU holds 12 of these kernels (at most 168 registers)
+static int32_t share_waves(int block, int blocks, int cus) { return std::min(blocks * (block / 64), 12 * cus); }
 
 using RtaKernel = void (*)(RtaParams);
 // the history kernel of a tally mode (0, 1 or 2) by [polygons][geometry in LDS]
@@ -1432,9 +1481,9 @@ static RtaKernel rta_kernel(int tally, bool grad, bool poly, bool gl) {
         {rta_history_kernel<true, 1, false, false>, rta_history_kernel<true, 1, false, true>}};
     return grad ? with_grad[tally][gl] : plain[tally][poly][gl];
 }
-static RtaKernel rta_items_kernel(bool poly, bool gl) {
-    return poly ? (gl ? rta_history_items_kernel<true, true> : rta_history_items_kernel<true, false>)
-                : (gl ? rta_history_items_kernel<false, true> : rta_history_items_kernel<false, false>);
+static RtaKernel rta_runs_kernel(bool poly, bool gl) {
+    return poly ? (gl ? rta_history_runs_kernel<true, true> : rta_history_runs_kernel<true, false>)
+                : (gl ? rta_history_runs_kernel<false, true> : rta_history_runs_kernel<false, false>);
 }
 static void allow_lds(RtaKernel k, size_t bytes) {
     HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
@@ -1442,21 +1491,19 @@ static void allow_lds(RtaKernel k, size_t bytes) {
 
 static void launch_batch(RtaBatch* b, RtaParams P, int block, int blocks, hipStream_t s) {
     hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, b->d_tally.p, RTA_NCOPY * 3 * b->cells,
-                       b->d_counters.p);
+                       b->d_counters.p, 8 + 2 * b->nruns);
     if (b->any_grad)
         hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, b->d_dgz.p, RTA_NCOPY * 4 * b->cells,
-                           b->d_counters.p);
+                           b->d_counters.p, 0);
     if (b->nloc)
         hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, b->d_spec.p,
-                           (uint64_t)b->nloc * (b->ntime - 1) * b->m->n, b->d_counters.p);
-    set_shares(P, block, blocks, b->ctx->cu_count);
+                           (uint64_t)b->nloc * (b->ntime - 1) * b->m->n, b->d_counters.p, 0);
+    P.waves = share_waves(block, blocks, b->ctx->cu_count);
     if (b->tally == 3) {
         RtaLds L = rta_lds_layout(b->l3_nbox, b->l3_nside, b->ntime - 1);
         if (!b->l3_mail) drop_mail(L);
         set_lds(P, L);
-        P.lanes = 64;
-        P.keep_waves = std::max(1, block / 64 / 3);
-        hipLaunchKernelGGL(rta_items_kernel(b->poly, L.gl), dim3(blocks), dim3(block), b->l3_bytes, s, P);
+        hipLaunchKernelGGL(rta_runs_kernel(b->poly, L.gl), dim3(blocks), dim3(block), b->l3_bytes, s, P);
     } else {
         const RtaLds L = rta_lds_of(b, b->tally);
         set_lds(P, L);
@@ -1674,7 +1721,7 @@ static void batch_create(RtaBatch* b) {
     b->d_timegrid.upload(b->timegrid, s);
     b->d_tally.alloc((size_t)RTA_NCOPY * 3 * b->cells);
     if (b->any_grad) b->d_dgz.alloc((size_t)RTA_NCOPY * 4 * b->cells);
-    b->d_counters.alloc(8);
+    b->d_counters.alloc(8 + 2 * (size_t)b->nruns);  // and tally mode 3's counters per run
     b->blocks = c->cu_count * 8;
     HIPCHECK(hipEventCreate(&b->ev0));
     HIPCHECK(hipEventCreate(&b->ev1));
@@ -1823,41 +1870,45 @@ static void batch_set_tally(RtaBatch* b, int mode) {
             lb[r] = (int32_t)std::min<size_t>((size_t)nt, avail / (3 * sizeof(double) * rows));
             b->l3_bytes = std::max(b->l3_bytes, (size_t)L.geo + 3 * sizeof(double) * rows * (size_t)lb[r]);
         }
-        allow_lds(rta_items_kernel(b->poly, L.gl), b->l3_bytes);
+        allow_lds(rta_runs_kernel(b->poly, L.gl), b->l3_bytes);
         b->block = 768;
         b->blocks = b->ctx->cu_count;
-        // about eight items per workgroup (configuration 3 without the
-        // scattering look-ahead: 1.24 s, against 1.33 s with four, 1.54 s
-        // with two and 1.24 s with sixteen), at
-        // least 4096 ids each; the runs with most particles first, so that
-        // the last items taken are short
-        const uint64_t isz = std::max<uint64_t>(4096, (b->total + 8 * (uint64_t)b->blocks - 1) / (8 * (uint64_t)b->blocks));
-        std::vector<int> order(b->nruns);
+        // workgroups per run in proportion to its particles (largest remainder),
+        // one at least while there are as many workgroups as runs; with more
+        // runs the largest begin and the others are picked as workgroups end
+        std::vector<int> order(b->nruns), wgs(b->nruns, 0);
         for (int r = 0; r < b->nruns; r++) order[r] = r;
         std::stable_sort(order.begin(), order.end(),
                          [&](int x, int y) { return b->runs[x].count > b->runs[y].count; });
-        b->items.clear();
-        for (int r : order) {
-            const RtaRunDev& R = b->runs[r];
-            if (R.count == 0) continue;
-            const uint64_t k = (R.count + isz - 1) / isz;
-            for (uint64_t q = 0; q < k; q++) {
-                RtaItem I{};
-                I.lo = R.first + R.count * q / k;
-                I.hi = R.first + R.count * (q + 1) / k;
-                I.lrow0 = b->run_lrow0[r];
-                I.lrows = b->run_lrows[r];
-                I.lbins = lb[r];
-                I.run = r;
-                I.box0 = b->box0[r];
-                I.nbox = b->nbox[r];
-                I.side0 = b->side0[r];
-                I.nsides = b->nside[r];
-                b->items.push_back(I);
+        int left = b->blocks;
+        for (int r : order)
+            if (left > 0) {
+                wgs[r] = 1;
+                left--;
             }
+        if (left > 0) {
+            std::vector<std::pair<double, int>> rest;
+            const int spare = left;
+            for (int r = 0; r < b->nruns; r++) {
+                const double share = (double)spare * (double)b->runs[r].count / (double)b->total;
+                wgs[r] += (int)share;
+                left -= (int)share;
+                rest.push_back({share - std::floor(share), r});
+            }
+            std::stable_sort(rest.begin(), rest.end(), [](auto& x, auto& y) { return x.first > y.first; });
+            for (int k = 0; k < left; k++) wgs[rest[k % rest.size()].second]++;
         }
-        // the same buffer while the list does not grow: a captured graph holds its address
-        if (!b->items.empty()) b->d_items.upload(b->items.data(), b->items.size(), b->ctx->stream);
+        std::vector<int32_t> first;
+        for (int r : order) first.insert(first.end(), wgs[r], r);
+        first.resize(b->blocks, -1);
+        std::vector<RtaRunRows> rows(b->nruns);
+        for (int r = 0; r < b->nruns; r++)
+            rows[r] = RtaRunRows{b->run_lrow0[r], b->run_lrows[r], lb[r], wgs[r],
+                                 b->box0[r], b->nbox[r], b->side0[r], b->nside[r]};
+        // the same buffers when the mode is set again: a captured graph holds their addresses
+        b->d_rows.upload(rows.data(), rows.size(), b->ctx->stream);
+        b->d_first_run.upload(first.data(), first.size(), b->ctx->stream);
+        HIPCHECK(hipStreamSynchronize(b->ctx->stream));  // the host arrays end here
     } else if (mode == 2) {
         if (b->nloc) throw Error(BTE_EINVAL, "LDS tallies do not cover spectral locations");
         if (b->any_grad) throw Error(BTE_EINVAL, "tally mode 2 does not carry dT/dp; use mode 1 or 0");
@@ -2034,9 +2085,9 @@ static void rta_execute_noalloc(RtaBatch* b, double* d_T, double* d_jx, double* 
     // the scratch keeps the previous call's contents: the tally copies and
     // the counters start at zero (a kernel, not a memset, so that a graph
     // capture records no memset node); the partial blocks are overwritten
-    hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, base, (uint64_t)ncopy, P.counters);
+    hipLaunchKernelGGL(rta_clear_kernel, dim3(1024), dim3(256), 0, s, base, (uint64_t)ncopy, P.counters, 8);
     set_lds(P, L);
-    set_shares(P, block, blocks, c->cu_count);
+    P.waves = share_waves(block, blocks, c->cu_count);
     const RtaKernel k = rta_kernel(mode, false, false, L.gl);
     if (mode == 2) allow_lds(k, c->lds_per_block);
     hipLaunchKernelGGL(k, dim3(blocks), dim3(block), L.bytes, s, P);

@@ -246,10 +246,10 @@ int bte_rta_batch_create(bte_ctx* ctx, const bte_modes* m, int nruns, const bte_
  * FP64 tallies once at the end; one 768-thread workgroup per CU. BTE_EINVAL when those arrays exceed the
  * device's LDS per workgroup. mode 2: FP64 sums of T, jx and jy in LDS for
  * as many leading time bins of all regular boxes as fit, later bins by FP64
- * device atomics. mode 3: as mode 2 with each workgroup working through
- * items of one run's particles at a time and its LDS holding only that
- * run's boxes (added into the tallies after each item), so a batch of many
- * runs keeps as many bins in LDS as one run. Modes 2 and 3: FP64 sums
+ * device atomics. mode 3: as mode 2 with each workgroup following one
+ * run's particles at a time and its LDS holding only that run's boxes (added
+ * into the tallies when the run's particles are taken and their histories
+ * have ended), so a batch of many runs keeps as many bins in LDS as one run. Modes 2 and 3: FP64 sums
  * throughout; not with dT/dp or spectral locations (BTE_EINVAL). */
 int bte_rta_batch_set_tally(bte_rta_batch* b, int mode);
 /* Times the batch scaled to `fraction` of each run's particles over a set of

@@ -105,3 +105,24 @@ def test_scores_move_with_their_histories(pkg, ctx):
     scale = np.abs(ra["dTdp"]).max()
     assert scale > 0
     np.testing.assert_allclose(rb[0]["dTdp"], ra["dTdp"], rtol=0, atol=1e-10 * scale)
+
+
+@pytest.mark.parametrize("nruns", [1, 3, 300])
+def test_runs_shared_among_workgroups(pkg, ctx, nruns):
+    """Tally mode 3 with one run for all workgroups, a few uneven ones, and
+    more runs than workgroups (those without one are picked up later)."""
+    modes = _modes(pkg, ctx, n=100)
+    geom = _ribbon(pkg, ctx, 6)
+    counts = [int(c) for c in (np.geomspace(60000, 900, nruns) if nruns < 10 else 20 + 37 * (np.arange(nruns) % 11))]
+    runs = [dict(geom=geom, T0=300.0, nparticles=c, seed=40 + k, wscale=0.5 + k / nruns)
+            for k, c in enumerate(counts)]
+    ref_b = pkg.RtaBatch(ctx, modes, runs, **KW)
+    ref, rep = ref_b.execute()
+    ref_b.close()
+    b = pkg.RtaBatch(ctx, modes, runs, tally="fp64-lds-runs", **KW)
+    for _ in range(2):
+        got, grep = b.execute()
+        assert (grep["events"], grep["crossings"]) == (rep["events"], rep["crossings"])
+        for g, r in zip(got, ref):
+            _same(g, r)
+    b.close()
