@@ -1172,17 +1172,31 @@ __global__ __launch_bounds__(256) void rta_spec_cumsum_kernel(double* S, int nlo
 
 // Tally mode 2: the LDS blocks of all workgroups, part[blk][3][lrows][lbins],
 // summed per cell and added into copy 0 of the tallies (cells of the first
-// lbins time bins receive no device atomics, so the add is a plain store)
-__global__ __launch_bounds__(256) void rta_sum_parts_kernel(double* tally, const double* part, int nblk,
+// lbins time bins receive no device atomics, so the add is a plain store).
+// Each workgroup sums 32 neighbouring cells (256 bytes of every block) with 16
+// threads per cell: one thread per cell left most CUs idle behind a chain of
+// 256 to 512 loads (3000 cells of 512 blocks: 123 us, now 5.1 us; 19200
+// cells of 256: 77 us, now 9.8 us).
+#define RTA_SUM_CELLS 32
+__global__ __launch_bounds__(512) void rta_sum_parts_kernel(double* tally, const double* part, int nblk,
                                                             uint32_t lrows, uint32_t lbins,
                                                             const uint64_t* lrow_cell, uint64_t cells) {
+    constexpr int NG = 512 / RTA_SUM_CELLS;
+    __shared__ double sum[NG][RTA_SUM_CELLS];
     const uint32_t lc = lrows * lbins, nf = 3u * lc;
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nf; j += gridDim.x * blockDim.x) {
-        double v = 0.;
-        for (int b = 0; b < nblk; b++) v += part[(size_t)b * nf + j];
+    const uint32_t q = threadIdx.x % RTA_SUM_CELLS, g = threadIdx.x / RTA_SUM_CELLS;
+    const uint32_t j = blockIdx.x * RTA_SUM_CELLS + q;
+    double v = 0.;
+    if (j < nf) {
+#pragma unroll 8
+        for (int b = (int)g; b < nblk; b += NG) v += part[(size_t)b * nf + j];
+    }
+    sum[g][q] = v;
+    __syncthreads();
+    if (g == 0 && j < nf) {
+        for (int k = 1; k < NG; k++) v += sum[k][q];
         const uint32_t a = j / lc, r = j - a * lc, row = r / lbins;
-        double* dst = tally + (uint64_t)a * cells + lrow_cell[row] + (r - row * lbins);
-        *dst += v;
+        tally[(uint64_t)a * cells + lrow_cell[row] + (r - row * lbins)] += v;
     }
 }
 
@@ -1510,7 +1524,7 @@ static void launch_batch(RtaBatch* b, RtaParams P, int block, int blocks, hipStr
         hipLaunchKernelGGL(rta_kernel(b->tally, b->any_grad, b->poly, L.gl), dim3(blocks), dim3(block), L.bytes, s, P);
         if (b->tally == 2) {
             const uint32_t nf = 3u * b->lrows * L.lbins;
-            hipLaunchKernelGGL(rta_sum_parts_kernel, dim3(std::min<uint32_t>((nf + 255) / 256, 4096u)), dim3(256), 0, s,
+            hipLaunchKernelGGL(rta_sum_parts_kernel, dim3((nf + RTA_SUM_CELLS - 1) / RTA_SUM_CELLS), dim3(512), 0, s,
                                b->d_tally.p, b->d_part.p, blocks, b->lrows, L.lbins, b->d_lrow_cell.p, b->cells);
         }
     }
@@ -2093,7 +2107,7 @@ static void rta_execute_noalloc(RtaBatch* b, double* d_T, double* d_jx, double* 
     hipLaunchKernelGGL(k, dim3(blocks), dim3(block), L.bytes, s, P);
     if (mode == 2) {
         const uint32_t nf = 3u * b->lrows * L.lbins;
-        hipLaunchKernelGGL(rta_sum_parts_kernel, dim3(std::min<uint32_t>((nf + 255) / 256, 4096u)), dim3(256), 0, s,
+        hipLaunchKernelGGL(rta_sum_parts_kernel, dim3((nf + RTA_SUM_CELLS - 1) / RTA_SUM_CELLS), dim3(512), 0, s,
                            base, P.part, blocks, b->lrows, L.lbins, b->d_lrow_cell.p, b->cells);
     }
     hipLaunchKernelGGL(rta_sum_copies_kernel, dim3(1024), dim3(256), 0, s, base, 3 * b->cells);
