@@ -84,7 +84,6 @@ struct BertParams {
     uint32_t segcap;         // capacity of one segment (cap / nsegs)
     int32_t nsegs;           // step + emit + source workgroups
     int32_t seg_emit0, seg_src0;  // first emit and first source segment
-    int32_t ncts;
     uint64_t seed;
     double dt, Eeff, thickness;
     int32_t n, ngamma, ncol, nbox, nseg;
@@ -93,8 +92,7 @@ struct BertParams {
     int32_t nslots;          // propagator slots (box temperatures)
     int32_t lds_props;       // properties from per-workgroup box sums (nbox <= BERT_LDS_BOXES)
     // dynamic LDS layout of the particle kernels (byte offsets)
-    int32_t lds_pre, lds_eb, lds_sbox, lds_boxes, lds_cts, lds_vel;
-    int32_t cts_lds;         // contacts staged in LDS too (GL instantiations)
+    int32_t lds_pre, lds_eb, lds_sbox, lds_boxes, lds_vel;
     int32_t eb_lds;          // wall counters in LDS (nsd <= BERT_EB_LDS)
 };
 
@@ -110,129 +108,185 @@ __device__ inline void seed_stream(Pcg32& r, uint64_t key, uint64_t pid) {
 
 // The particle kernels share one dynamic LDS block: segment prefix sums,
 // wall counters, box sums and, when small enough (GL instantiations), the
-// geometry tables. Offsets are set on the host.
+// boxes. Offsets are set on the host.
 #define BERT_LDS_BOXES 512
 #define BERT_GEO_LDS_BYTES 49152
 extern __shared__ __align__(16) unsigned char bert_dyn[];
+
+// The boxes of the crossing loop: in LDS (GL) 80 bytes apart, else the global
+// records. Every lane reads its own box, and a stride of 20 banks starts 16
+// consecutive boxes at 16 different 16-byte groups, where the records' 64
+// bytes put them on four.
+#define BERT_BOX_LDS 80
 template <bool GL>
-__device__ inline void geo_stage(const BertParams& P, const DevBox*& boxes, const DevContact*& cts) {
-    if (GL) {
-        DevBox* gb = (DevBox*)(bert_dyn + P.lds_boxes);
-        DevContact* gc = (DevContact*)(bert_dyn + P.lds_cts);
-        for (int i = threadIdx.x; i < P.nbox; i += blockDim.x) gb[i] = P.boxes[i];
-        boxes = gb;
-        cts = P.cts;
-        if (P.cts_lds) {
-            for (int i = threadIdx.x; i < P.ncts; i += blockDim.x) gc[i] = P.cts[i];
-            cts = gc;
-        }
-    } else {
-        boxes = P.boxes;
-        cts = P.cts;
+struct BertBoxes {
+    const unsigned char* p;
+    __device__ inline const DevBox& operator[](int i) const {
+        return *reinterpret_cast<const DevBox*>(p + (size_t)i * (GL ? BERT_BOX_LDS : sizeof(DevBox)));
     }
+};
+template <bool GL>
+__device__ inline BertBoxes<GL> geo_stage(const BertParams& P) {
+    if (!GL) return BertBoxes<GL>{reinterpret_cast<const unsigned char*>(P.boxes)};
+    unsigned char* gb = bert_dyn + P.lds_boxes;
+    for (int i = threadIdx.x; i < P.nbox; i += blockDim.x)
+        *reinterpret_cast<DevBox*>(gb + (size_t)i * BERT_BOX_LDS) = P.boxes[i];
+    return BertBoxes<GL>{gb};
+}
+
+// The kernel's parameters (its first argument) for code off the main path,
+// read from the kernel argument segment where they are used: kept in scalar
+// registers over the whole particle loop, the pointers of these paths push
+// those of the main path into vector lanes (a lane read for each use).
+__device__ inline const BertParams& bert_cold_params() {
+    auto* p = (const __attribute__((address_space(4))) BertParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const BertParams*)p;
+}
+
+// One hit of side i (Eborder): the workgroup's LDS counters, or the global
+// ones where those do not fit (or the kernel has none: lds false)
+__device__ inline void wall_hit(const BertParams& P, bool lds, int32_t* Eg, int i, int sign) {
+    if (lds) {
+        auto* L = (__attribute__((address_space(3))) int32_t*)(bert_dyn + P.lds_eb) + i;
+        __hip_atomic_fetch_add(L, sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else {
+        atomicAdd(Eg + i, sign);
+    }
+}
+
+// What advect meets rarely, for the lanes that met it: a periodic box
+// (mask 0), or an exit through the sides of mask that needs the general
+// neighbour search. Returns 1 to fly on for dt, 0 when the particle has ended.
+template <bool PER, bool POLY>
+__device__ inline int advect_slow(bool eb_lds, int32_t* Eg, double& x, double& y, int& box, int sign, double vx,
+                                  double vy, int mask, Pcg32& rng) {
+    const BertParams& P = bert_cold_params();
+    if (mask == 0) {
+        if (!PER) {  // the host launches PER whenever a box is periodic
+            atomicOr(P.flags + 3, 1u);
+            return 0;
+        }
+        // translate and continue the flight (beyondRTA_MC2d.cpp:729-737)
+        const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng)
+                            : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng);
+        if (nb < 0) {
+            atomicOr(P.flags + 3, 1u);
+            return 0;
+        }
+        box = nb;
+        return 1;
+    }
+    const DevBox B = P.boxes[box];
+    const int2 sr = POLY ? P.srange[box] : make_int2(4 * box, 4);
+    Ids4 pb{};
+    const int npb = POLY ? poly_find_pboxes(P.sides, P.srange, P.cts, B, x, y, vx, vy, pb)
+                         : find_pboxes(P.boxes, P.cts, B, x, y, vx, vy, pb);
+    if (npb == 0) {
+        const int s = __popc(mask) == 1 ? __ffs(mask) - 1
+                      : (POLY ? poly_pick_void_side(P.sides, P.srange, P.cts, B, sr, mask, x, y, rng.next())
+                              : pick_void_side(P.boxes, P.cts, B, mask, x, y, rng.next()));
+        wall_hit(P, eb_lds, Eg, sr.x + s, sign);
+        return 0;
+    }
+    if (npb == 1) {
+        box = pb.a;
+        return 1;
+    }
+    Ids4 cand{};
+    int nc = 0;
+    double tau = 1.0e-6;
+    while (nc == 0 && tau >= 1.0e-15) {
+        for (int k = 0; k < npb && k < 4; k++) {
+            const double tx = x + tau * vx, ty = y + tau * vy;
+            const bool in = POLY ? poly_inside(P.sides, P.srange[pb.get(k)], tx, ty)
+                                 : box_inside(P.boxes[pb.get(k)], tx, ty);
+            if (in) cand.set(nc++, pb.get(k));
+        }
+        tau /= 10.0;
+    }
+    if (nc == 0) {
+        const double ccx = POLY ? P.center[box].x : 0.5 * (B.xmin + B.xmax);
+        const double ccy = POLY ? P.center[box].y : 0.5 * (B.ymin + B.ymax);
+        const double dx = ccx - x, dy = ccy - y;
+        const double dn = sqrt(dx * dx + dy * dy);
+        x += 1.0e-6 * dx / dn;
+        y += 1.0e-6 * dy / dn;
+    } else {
+        box = cand.get((int)rng.bounded((uint32_t)nc));
+    }
+    return 1;
 }
 
 // evolparticle (beyondRTA_MC2d.cpp:708-970): ballistic advection by dt
 // through box crossings; a void side adds the particle sign to that side's
 // Eborder and ends the particle. Returns false if the particle ended.
+// The inner loop crosses sides shared with one box; a lane that meets a
+// periodic box or an exit that needs the general search waits at its end, so
+// that the long code of those cases runs once for all of them.
+// With the exit test in selects, the boxes at a conflict-free stride and the
+// rare cases' parameters out of the loop's scalar registers (95 instead of 165
+// lane reads of spilled ones in the kernel) the step kernel takes 144.6 us
+// instead of 152 at 3.3e6 particle-steps.
 // PER compiles in the periodic translation; without periodic boxes the
-// kernels use the instantiation without it, which needs about 50 fewer
-// registers per lane (4 resident waves per SIMD instead of 3). POLY: convex
-// polygon boxes (the geometry from the side tables).
-template <bool PER, bool POLY>
-__device__ inline bool advect(const BertParams& P, const DevBox* boxes, const DevContact* cts, double& x,
+// kernels use the instantiation without it, which needs fewer registers per
+// lane. POLY: convex polygon boxes (the geometry from the side tables).
+template <bool PER, bool POLY, bool GL>
+__device__ inline bool advect(const BertParams& P, const BertBoxes<GL>& boxes, bool eb_lds, int32_t* Eg, double& x,
                               double& y, int& box, int sign, double vx, double vy, double ivx, double ivy,
-                              double dt, Pcg32& rng, int32_t* Eb) {
-    for (int it = 0; it < 4096; it++) {
-        const DevBox B = boxes[box];
-        if (B.kind == 1) return false;  // reservoir: deleted
-        if (B.kind == 2) {
-            if (!PER) {  // the host launches PER whenever a box is periodic
-                atomicOr(P.flags + 3, 1u);
+                              double dt, Pcg32& rng) {
+    for (int it = 0;;) {
+        int mask = -1;
+        for (;; it++) {
+            if (it >= 4096) {
+                atomicOr(P.flags + 2, 1u);
                 return false;
             }
-            // periodic box: translate and continue the flight (beyondRTA_MC2d.cpp:729-737)
-            const int nb = POLY ? translate_poly(boxes, P.sides, P.srange, cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng)
-                                : translate_rect(boxes, cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng);
-            if (nb < 0) {
-                atomicOr(P.flags + 3, 1u);
+            const DevBox B = boxes[box];
+            if (B.kind != 0) {
+                if (B.kind == 1) return false;  // reservoir: deleted
+                mask = 0;
+                break;
+            }
+            double nx = x + dt * vx, ny = y + dt * vy;
+            int2 sr = make_int2(4 * box, 4);
+            if constexpr (POLY) sr = P.srange[box];
+            const bool inside = POLY ? poly_inside(P.sides, sr, nx, ny)
+                                     : (nx >= B.xmin) & (nx <= B.xmax) & (ny >= B.ymin) & (ny <= B.ymax);
+            if (inside) {
+                x = nx;
+                y = ny;
+                return true;
+            }
+            double tf;
+            int aux, fast;
+            if constexpr (POLY) {
+                int m;
+                tf = poly_exit(P.sides, sr, x, y, vx, vy, m, nx, ny);
+                fast = poly_side_fast(P.sides, sr, m, nx, ny, vx, vy, aux);
+                if (fast == SIDE_MIXED) aux = m;
+            } else {
+                fast = rect_exit(B, x, y, vx, vy, ivx, ivy, tf, nx, ny, aux);
+            }
+            dt -= tf;
+            if (almost_equal(dt, 0.)) dt = 0.;
+            if (fast == SIDE_VOID) {
+                wall_hit(P, eb_lds, Eg, sr.x + aux, sign);
                 return false;
             }
-            box = nb;
-            continue;
-        }
-        double nx = x + dt * vx, ny = y + dt * vy;
-        int2 sr = make_int2(4 * box, 4);
-        if constexpr (POLY) sr = P.srange[box];
-        if (POLY ? poly_inside(P.sides, sr, nx, ny) : box_inside(B, nx, ny)) {
             x = nx;
             y = ny;
-            return true;
-        }
-        int mask;
-        double ex, ey;
-        double tf = POLY ? poly_exit(P.sides, sr, x, y, vx, vy, mask, ex, ey)
-                         : box_exit(B, x, y, vx, vy, ivx, ivy, mask, ex, ey);
-        double left = dt - tf;
-        if (almost_equal(left, 0.)) left = 0.;
-        int side = 0;
-        const int fast = POLY ? poly_side_fast(P.sides, sr, mask, ex, ey, vx, vy, side)
-                              : side_fast(B, mask, ex, ey, vx, vy, side);
-        if (fast == SIDE_VOID) {
-            atomicAdd(Eb + sr.x + side, sign);
-            return false;
-        }
-        if (fast >= 0) {
-            x = ex;
-            y = ey;
+            if (fast < 0) {
+                mask = aux;
+                break;
+            }
             box = fast;
-            dt = left;
             if (dt == 0.) return true;
-            continue;
         }
-        Ids4 pb{};
-        int npb = POLY ? poly_find_pboxes(P.sides, P.srange, cts, B, ex, ey, vx, vy, pb)
-                       : find_pboxes(boxes, cts, B, ex, ey, vx, vy, pb);
-        if (npb == 0) {
-            int s = __popc(mask) == 1 ? __ffs(mask) - 1
-                    : (POLY ? poly_pick_void_side(P.sides, P.srange, cts, B, sr, mask, ex, ey, rng.next())
-                            : pick_void_side(boxes, cts, B, mask, ex, ey, rng.next()));
-            atomicAdd(Eb + sr.x + s, sign);
-            return false;
-        }
-        x = ex;
-        y = ey;
-        if (npb == 1) {
-            box = pb.a;
-        } else {
-            Ids4 cand{};
-            int nc = 0;
-            double tau = 1.0e-6;
-            while (nc == 0 && tau >= 1.0e-15) {
-                for (int k = 0; k < npb && k < 4; k++) {
-                    const double tx = ex + tau * vx, ty = ey + tau * vy;
-                    const bool in = POLY ? poly_inside(P.sides, P.srange[pb.get(k)], tx, ty)
-                                         : box_inside(boxes[pb.get(k)], tx, ty);
-                    if (in) cand.set(nc++, pb.get(k));
-                }
-                tau /= 10.0;
-            }
-            if (nc == 0) {
-                const double ccx = POLY ? P.center[box].x : 0.5 * (B.xmin + B.xmax);
-                const double ccy = POLY ? P.center[box].y : 0.5 * (B.ymin + B.ymax);
-                double dx = ccx - ex, dy = ccy - ey;
-                double dn = sqrt(dx * dx + dy * dy);
-                x = ex + 1.0e-6 * dx / dn;
-                y = ey + 1.0e-6 * dy / dn;
-            } else {
-                box = cand.get((int)rng.bounded((uint32_t)nc));
-            }
-        }
-        dt = left;
-        if (dt == 0.) return true;
+        if (!advect_slow<PER, POLY>(eb_lds, Eg, x, y, box, sign, vx, vy, mask, rng)) return false;
+        if (mask != 0 && dt == 0.) return true;
+        it++;
     }
-    atomicOr(P.flags + 2, 1u);
-    return false;
 }
 
 // The propagator of the box a particle scatters in (one slot per box
@@ -515,11 +569,10 @@ __device__ inline uint32_t permute_index(uint32_t t, uint32_t c, uint64_t key) {
 // Wall counters are accumulated per workgroup in LDS and flushed with one
 // global atomic per touched side (the walls of a few boxes take most hits).
 #define BERT_EB_LDS 2048
-__device__ inline int32_t* eb_lds_begin(const BertParams& P, int32_t* Eb, int nb4) {
-    if (!P.eb_lds) return Eb;
+__device__ inline void eb_lds_begin(const BertParams& P, int nb4) {
+    if (!P.eb_lds) return;
     int32_t* sEb = (int32_t*)(bert_dyn + P.lds_eb);
     for (int i = threadIdx.x; i < nb4; i += blockDim.x) sEb[i] = 0;
-    return sEb;
 }
 __device__ inline void eb_lds_flush(const BertParams& P, int32_t* Eb, int nb4) {
     if (!P.eb_lds) return;
@@ -561,9 +614,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) v
     __shared__ uint32_t tsum[16];
     __shared__ uint32_t lcount;
     uint32_t* pre = (uint32_t*)(bert_dyn + P.lds_pre);
-    const DevBox* boxes;
-    const DevContact* cts;
-    geo_stage<GL>(P, boxes, cts);
+    const BertBoxes<GL> boxes = geo_stage<GL>(P);
     const double2* vtab = P.vel;
     const double2* ivtab = P.ivel;
     if constexpr (VL) {
@@ -578,7 +629,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) v
     }
     const int nb4 = P.nsd;
     int32_t* Eg = P.Eb + (size_t)(step & 1) * nb4;
-    int32_t* Eb = eb_lds_begin(P, Eg, nb4);
+    eb_lds_begin(P, nb4);
     if (threadIdx.x == 0) lcount = 0;
     double* sbox = box_lds_begin(P);
     const uint32_t* segin = P.seg + (size_t)cur * P.nsegs;
@@ -640,7 +691,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) v
                 if (nslots_of<P1>(P) == 1) f0 = first_pick<P1>(P, rng, mode, 0);
                 const double2 v = vtab[mode];
                 const double2 iv = ivtab[mode];
-                alive = advect<PER, POLY>(P, boxes, cts, p.x, p.y, box, sign, v.x, v.y, iv.x, iv.y, P.dt, rng, Eb);
+                alive = advect<PER, POLY, GL>(P, boxes, P.eb_lds != 0, Eg, p.x, p.y, box, sign, v.x, v.y, iv.x, iv.y, P.dt, rng);
                 if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, box);
             }
         }
@@ -915,9 +966,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
     const int myseg = P.seg_emit0 + blockIdx.x;
     uint32_t* segout = P.seg + (size_t)(cur ^ 1) * P.nsegs;
     if (threadIdx.x == 0) lcount = 0;
-    const DevBox* boxes;
-    const DevContact* cts;
-    geo_stage<GL>(P, boxes, cts);
+    const BertBoxes<GL> boxes = geo_stage<GL>(P);
     const double2* vtab = P.vel;
     const double2* ivtab = P.ivel;
     if constexpr (VL) {
@@ -931,7 +980,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
         ivtab = sv + P.n;
     }
     int32_t* Eg = P.Eb + (size_t)((step + 1) & 1) * nb4;
-    int32_t* Ebn = eb_lds_begin(P, Eg, nb4);
+    eb_lds_begin(P, nb4);
     double* sbox = box_lds_begin(P);
     const uint32_t total = seg_prefix(P.wcount, nb4, 0xffffffffu, pre, tsum);  // ends with a barrier
     const uint32_t lo = (uint32_t)((uint64_t)total * blockIdx.x / gridDim.x);
@@ -996,7 +1045,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
             const double2 iv = ivtab[mode];
             double rdt = P.dt * rng.uniform();
             if (nslots_of<P1>(P) == 1) f0 = first_pick<P1>(P, rng, mode, 0);
-            alive = advect<PER, POLY>(P, boxes, cts, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng, Ebn);
+            alive = advect<PER, POLY, GL>(P, boxes, P.eb_lds != 0, Eg, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
             if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, bx);
         }
         scatter_out<P1>(P, H, sbox, vtab, rng, f0, alive, mode, sign, bx, x, y, pid, step, &lcount, myseg);
@@ -1037,6 +1086,7 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
     __syncthreads();
     int32_t* Eb = P.Eb + (size_t)(step & 1) * P.nsd;
     unsigned long long* H = hist ? P.H + (size_t)cur * P.nbox * P.n : nullptr;
+    const BertBoxes<false> boxes{reinterpret_cast<const unsigned char*>(P.boxes)};
     unsigned long long done = 0;
     const int j0 = (int)((int64_t)nparts_all * blockIdx.x / gridDim.x);
     const int j1 = (int)((int64_t)nparts_all * (blockIdx.x + 1) / gridDim.x);
@@ -1103,7 +1153,7 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
                 const double2 iv = P.ivel[mode];
                 double rdt = P.dt * rng.uniform();
                 if (nslots_of<false>(P) == 1) f0 = first_pick<false>(P, rng, mode, 0);
-                alive = advect<PER, POLY>(P, P.boxes, P.cts, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng, Eb);
+                alive = advect<PER, POLY, false>(P, boxes, false, Eb, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
                 if (nslots_of<false>(P) > 1 && alive) f0 = first_pick<false>(P, rng, mode, bx);
             }
             scatter_out<false>(P, H, sbox, P.vel, rng, f0, alive, mode, sign, bx, x, y, pid, step, &lcount, myseg);
@@ -1505,7 +1555,6 @@ static BertParams make_params(Bert* b) {
     P.segcap = (uint32_t)(b->cap / b->nsegs);
     P.seg_emit0 = b->step_blocks;
     P.seg_src0 = b->step_blocks + b->emit_blocks;
-    P.ncts = (int)b->g->dcontacts.size();
     P.seed = b->cfg.seed;
     P.dt = b->cfg.dt;
     P.Eeff = b->Eeff;
@@ -1532,25 +1581,8 @@ static BertParams make_params(Bert* b) {
     if (P.eb_lds) off = up16(off + sizeof(int32_t) * (size_t)nb4);
     P.lds_sbox = (int32_t)off;
     if (P.lds_props) off = up16(off + sizeof(double) * 3 * (size_t)P.nbox);
-    const size_t geo = sizeof(DevBox) * (size_t)P.nbox + sizeof(DevContact) * (size_t)P.ncts;
-    b->geo_lds = geo <= BERT_GEO_LDS_BYTES && !b->g->poly;  // polygon kernels read the geometry globally
     P.lds_boxes = (int32_t)off;
-    P.lds_cts = (int32_t)up16(off + sizeof(DevBox) * (size_t)P.nbox);
-    P.cts_lds = 1;
-    if (b->geo_lds) {
-        off = up16(P.lds_cts + sizeof(DevContact) * (size_t)P.ncts);
-        // the step workgroups share the CU's LDS: five 256-thread ones, or
-        // one VL workgroup with the velocity tables after the layout. When
-        // the layout does not fit that share, the contacts (read only for
-        // sides that several boxes share and for periodic translations) stay
-        // in global memory
-        const long long per_wg = b->vl ? (long long)b->ctx->lds_per_block - 1024 - 32 * (long long)P.n
-                                       : (long long)(b->ctx->lds_per_block / 5);
-        if ((b->vl || b->p1) && !b->periodic && (long long)off + 256 > per_wg && (long long)P.lds_cts + 256 <= per_wg) {
-            P.cts_lds = 0;
-            off = (size_t)P.lds_cts;
-        }
-    }
+    if (b->geo_lds) off = up16(off + (size_t)BERT_BOX_LDS * P.nbox);
     b->lds_bytes = off;
     P.lds_vel = (int32_t)up16(off);
     b->lds_vl_bytes = up16(off) + 32 * (size_t)P.n;
@@ -1869,6 +1901,8 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     // next to the particle kernels' layout; else 256-thread step and
     // 512-thread emission workgroups
     if (cfg->step_shape < 0 || cfg->step_shape > 1) throw Error(BTE_EINVAL, "step_shape must be 0 or 1");
+    // boxes in LDS (polygon kernels read the geometry globally)
+    b->geo_lds = !g->poly && (size_t)BERT_BOX_LDS * nbox <= BERT_GEO_LDS_BYTES;
     b->vl = !b->periodic && cfg->step_shape == 0;
     if (b->vl) {
         b->step_blocks = std::min(c->cu_count, BERT_MAXSEG - 512 - BERT_SRC_BLOCKS);
@@ -1876,6 +1910,13 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
         b->nsegs = b->step_blocks + b->emit_blocks + b->src_blocks;
         (void)make_params(b);  // the layout for these segments
         b->vl = b->lds_vl_bytes + 1024 <= c->lds_per_block;
+        if (!b->vl && b->geo_lds) {
+            // the velocity tables before the boxes where only one of them fits
+            b->geo_lds = false;
+            (void)make_params(b);
+            b->vl = b->lds_vl_bytes + 1024 <= c->lds_per_block;
+            b->geo_lds = !b->vl;
+        }
     }
     if (!b->vl) {
         b->step_blocks = std::min((b->periodic ? 3 : (b->p1 ? 5 : 4)) * c->cu_count, BERT_MAXSEG - 512 - BERT_SRC_BLOCKS);

@@ -177,6 +177,36 @@ __device__ __host__ inline int side_fast(const DevBox& B, int mask, double ex, d
                      : (side == 1 ? B.side_nbr[1] : (side == 2 ? B.side_nbr[2] : B.side_nbr[3]));
 }
 
+// Exit from a rectangle (box_exit) and the fast neighbour search (side_fast)
+// in one: time t, point (ex, ey), the side or, when the general search must
+// run, the mask of the sides. Returns the neighbour, SIDE_VOID or SIDE_MIXED.
+// Selects only: a lane's box and direction differ from its neighbours', so
+// branches would run one after the other.
+template <class Box>
+__device__ inline int rect_exit(const Box& b, double x, double y, double vx, double vy, double ivx, double ivy,
+                                double& t, double& ex, double& ey, int& aux) {
+    const bool px = vx > 0., py = vy > 0.;
+    const double bx = px ? b.xmax : b.xmin, by = py ? b.ymax : b.ymin;
+    double tx = vx == 0. ? 1e300 : (bx - x) * ivx, ty = vy == 0. ? 1e300 : (by - y) * ivy;
+    tx = tx < 0. ? 0. : tx;
+    ty = ty < 0. ? 0. : ty;
+    const bool xfirst = tx < ty, yfirst = ty < tx;  // neither: both sides at once
+    t = yfirst ? ty : tx;
+    ex = yfirst ? x + t * vx : bx;
+    ey = xfirst ? y + t * vy : by;
+    if (almost_equal(t, 0.)) t = 0.;
+    const bool in_y = (ey > b.ymin) & (ey < b.ymax), in_x = (ex > b.xmin) & (ex < b.xmax);
+    const bool clear = (xfirst & in_y & !almost_equal(vx, 0.)) | (yfirst & in_x & !almost_equal(vy, 0.));
+    const int nx = px ? b.side_nbr[3] : b.side_nbr[0], ny = py ? b.side_nbr[2] : b.side_nbr[1];
+    if (clear) {
+        aux = xfirst ? (px ? 3 : 0) : (py ? 2 : 1);
+        return xfirst ? nx : ny;
+    }
+    const int sx = px ? 3 : (vx < 0. ? 0 : 31), sy = py ? 2 : (vy < 0. ? 1 : 31);
+    aux = (yfirst ? 0 : 1 << sx) | (xfirst ? 0 : 1 << sy);
+    return SIDE_MIXED;
+}
+
 // Neighbour search at an exit point (RTA_MC2D.cpp:1130-1163): contacts c
 // whose closed box holds rnew or rnew + 1e-6 v/|v| with n_c.v > 0 and not
 // parallel. Returns the count; the first four ids are packed in ids (kept in

@@ -475,35 +475,6 @@ __device__ inline void rta_look(const RtaParams& P, const RtaGeo<GL>& G, RtaStat
     S.se = P.scat[(size_t)(TM == 3 ? G.run : S.run) * (uint32_t)P.n + S.sk];
 }
 
-// Exit from a rectangle (box_exit) and the fast neighbour search (side_fast)
-// in one: time t, point (ex, ey), the side or, when the general search must
-// run, the mask of the sides. Returns the neighbour, SIDE_VOID or SIDE_MIXED.
-// Selects only: a lane's box and direction differ from its neighbours', so
-// branches would run one after the other.
-__device__ inline int rect_exit(const RtaBox& b, double x, double y, double vx, double vy, double ivx, double ivy,
-                                double& t, double& ex, double& ey, int& aux) {
-    const bool px = vx > 0., py = vy > 0.;
-    const double bx = px ? b.xmax : b.xmin, by = py ? b.ymax : b.ymin;
-    double tx = vx == 0. ? 1e300 : (bx - x) * ivx, ty = vy == 0. ? 1e300 : (by - y) * ivy;
-    tx = tx < 0. ? 0. : tx;
-    ty = ty < 0. ? 0. : ty;
-    const bool xfirst = tx < ty, yfirst = ty < tx;  // neither: both sides at once
-    t = yfirst ? ty : tx;
-    ex = yfirst ? x + t * vx : bx;
-    ey = xfirst ? y + t * vy : by;
-    if (almost_equal(t, 0.)) t = 0.;
-    const bool in_y = (ey > b.ymin) & (ey < b.ymax), in_x = (ex > b.xmin) & (ex < b.xmax);
-    const bool clear = (xfirst & in_y & !almost_equal(vx, 0.)) | (yfirst & in_x & !almost_equal(vy, 0.));
-    const int nx = px ? b.side_nbr[3] : b.side_nbr[0], ny = py ? b.side_nbr[2] : b.side_nbr[1];
-    if (clear) {
-        aux = xfirst ? (px ? 3 : 0) : (py ? 2 : 1);
-        return xfirst ? nx : ny;
-    }
-    const int sx = px ? 3 : (vx < 0. ? 0 : 31), sy = py ? 2 : (vy < 0. ? 1 : 31);
-    aux = (yfirst ? 0 : 1 << sx) | (xfirst ? 0 : 1 << sy);
-    return SIDE_MIXED;
-}
-
 // One event of evolparticle (RTA_MC2D.cpp:990-1386) for lanes in FRESH or FLY:
 // the flight draw of the history loop (2262-2288), the segment to the next
 // scattering or box side and its tally, the scattering or the crossing into
