@@ -46,6 +46,10 @@ struct BertParams {
     const DevBox* boxes;
     const DevContact* cts;
     const double4* cseg;     // contact segments (periodic translation)
+    // rectangles: periodic boxes, their targets' contacts, the periodic box per box
+    const DevPer* per;
+    const DevCross* tcross;
+    const int32_t* box_per;
     const double2* ptrans;   // periodic translation per box
     const uint2* palias;     // propagator alias per slot, ncol x ncol column-major
     const int32_t* box_pslot; // propagator slot per box (nslots > 1)
@@ -92,7 +96,8 @@ struct BertParams {
     int32_t nslots;          // propagator slots (box temperatures)
     int32_t lds_props;       // properties from per-workgroup box sums (nbox <= BERT_LDS_BOXES)
     // dynamic LDS layout of the particle kernels (byte offsets)
-    int32_t lds_pre, lds_eb, lds_sbox, lds_boxes, lds_vel;
+    int32_t lds_pre, lds_eb, lds_sbox, lds_boxes, lds_per, lds_tc, lds_vel;
+    int32_t nper, ntc;       // periodic boxes, contacts of their targets
     int32_t eb_lds;          // wall counters in LDS (nsd <= BERT_EB_LDS)
 };
 
@@ -113,25 +118,37 @@ __device__ inline void seed_stream(Pcg32& r, uint64_t key, uint64_t pid) {
 #define BERT_GEO_LDS_BYTES 49152
 extern __shared__ __align__(16) unsigned char bert_dyn[];
 
-// The boxes of the crossing loop: in LDS (GL) 80 bytes apart, else the global
-// records. Every lane reads its own box, and a stride of 20 banks starts 16
-// consecutive boxes at 16 different 16-byte groups, where the records' 64
-// bytes put them on four.
+// The boxes of the crossing loop and the tables of the periodic translation:
+// in LDS (GL), else in global memory. Every lane reads its own box, and the
+// LDS stride of 80 bytes (20 banks) starts 16 consecutive boxes at 16
+// different 16-byte groups, where the records' 64 bytes put them on four. The
+// LDS record of a periodic box holds its index among the periodic boxes in tgt.
 #define BERT_BOX_LDS 80
 template <bool GL>
 struct BertBoxes {
     const unsigned char* p;
+    const DevPer* per;
+    const DevCross* tcross;
     __device__ inline const DevBox& operator[](int i) const {
         return *reinterpret_cast<const DevBox*>(p + (size_t)i * (GL ? BERT_BOX_LDS : sizeof(DevBox)));
     }
 };
-template <bool GL>
+template <bool PER, bool GL>
 __device__ inline BertBoxes<GL> geo_stage(const BertParams& P) {
-    if (!GL) return BertBoxes<GL>{reinterpret_cast<const unsigned char*>(P.boxes)};
+    if (!GL) return BertBoxes<GL>{reinterpret_cast<const unsigned char*>(P.boxes), P.per, P.tcross};
     unsigned char* gb = bert_dyn + P.lds_boxes;
-    for (int i = threadIdx.x; i < P.nbox; i += blockDim.x)
-        *reinterpret_cast<DevBox*>(gb + (size_t)i * BERT_BOX_LDS) = P.boxes[i];
-    return BertBoxes<GL>{gb};
+    for (int i = threadIdx.x; i < P.nbox; i += blockDim.x) {
+        DevBox b = P.boxes[i];
+        if (PER) b.tgt = P.box_per[i];
+        *reinterpret_cast<DevBox*>(gb + (size_t)i * BERT_BOX_LDS) = b;
+    }
+    DevPer* per = reinterpret_cast<DevPer*>(bert_dyn + P.lds_per);
+    DevCross* tc = reinterpret_cast<DevCross*>(bert_dyn + P.lds_tc);
+    if (PER) {
+        for (int i = threadIdx.x; i < P.nper; i += blockDim.x) per[i] = P.per[i];
+        for (int i = threadIdx.x; i < P.ntc; i += blockDim.x) tc[i] = P.tcross[i];
+    }
+    return BertBoxes<GL>{gb, per, tc};
 }
 
 // The kernel's parameters (its first argument) for code off the main path,
@@ -155,28 +172,32 @@ __device__ inline void wall_hit(const BertParams& P, bool lds, int32_t* Eg, int 
     }
 }
 
-// What advect meets rarely, for the lanes that met it: a periodic box
-// (mask 0), or an exit through the sides of mask that needs the general
-// neighbour search. Returns 1 to fly on for dt, 0 when the particle has ended.
-template <bool PER, bool POLY>
+// A periodic box, for the lanes (flying) that met one; every lane of the wave
+// calls. Returns false when the particle has ended.
+template <bool POLY, bool GL>
+__device__ inline bool advect_translate(const BertBoxes<GL>& boxes, bool want, double& x, double& y, int& box, double vx,
+                                        double vy, Pcg32& rng) {
+    const BertParams& P = bert_cold_params();
+    int nb = -1;
+    // translate and continue the flight (beyondRTA_MC2d.cpp:729-737)
+    if constexpr (POLY) {
+        if (want) nb = translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng);
+    } else {
+        const int pi = want ? (GL ? boxes[box].tgt : P.box_per[box]) : -1;
+        nb = translate_rect_wave(want, boxes.per, boxes.tcross, pi, x, y, vx, vy, rng);
+    }
+    if (!want) return true;
+    box = nb;
+    if (nb < 0) atomicOr(P.flags + 3, 1u);
+    return nb >= 0;
+}
+
+// An exit through the sides of mask that needs the general neighbour search,
+// for the lanes that met one. Returns 1 to fly on, 0 when the particle has ended.
+template <bool POLY>
 __device__ inline int advect_slow(bool eb_lds, int32_t* Eg, double& x, double& y, int& box, int sign, double vx,
                                   double vy, int mask, Pcg32& rng) {
     const BertParams& P = bert_cold_params();
-    if (mask == 0) {
-        if (!PER) {  // the host launches PER whenever a box is periodic
-            atomicOr(P.flags + 3, 1u);
-            return 0;
-        }
-        // translate and continue the flight (beyondRTA_MC2d.cpp:729-737)
-        const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng)
-                            : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, box, x, y, vx, vy, rng);
-        if (nb < 0) {
-            atomicOr(P.flags + 3, 1u);
-            return 0;
-        }
-        box = nb;
-        return 1;
-    }
     const DevBox B = P.boxes[box];
     const int2 sr = POLY ? P.srange[box] : make_int2(4 * box, 4);
     Ids4 pb{};
@@ -218,12 +239,65 @@ __device__ inline int advect_slow(bool eb_lds, int32_t* Eg, double& x, double& y
     return 1;
 }
 
-// evolparticle (beyondRTA_MC2d.cpp:708-970): ballistic advection by dt
-// through box crossings; a void side adds the particle sign to that side's
-// Eborder and ends the particle. Returns false if the particle ended.
-// The inner loop crosses sides shared with one box; a lane that meets a
-// periodic box or an exit that needs the general search waits at its end, so
-// that the long code of those cases runs once for all of them.
+// One stretch of evolparticle (beyondRTA_MC2d.cpp:708-970): crossings of sides
+// shared with one box, until the particle arrives (ADV_ARRIVED), ends in a
+// reservoir or at a void side, whose Eborder takes its sign (ADV_ENDED), or
+// meets a periodic box (ADV_PERIODIC) or an exit through the sides of mask
+// that needs the general search (ADV_SEARCH).
+enum { ADV_ENDED = 0, ADV_ARRIVED = 1, ADV_PERIODIC = 2, ADV_SEARCH = 3 };
+template <bool POLY, bool GL>
+__device__ inline int advect_cross(const BertParams& P, const BertBoxes<GL>& boxes, bool eb_lds, int32_t* Eg, double& x,
+                                   double& y, int& box, int sign, double vx, double vy, double ivx, double ivy,
+                                   double& dt, int& mask, int& it) {
+    for (;;) {
+        if (++it > 4096) {
+            atomicOr(P.flags + 2, 1u);
+            return ADV_ENDED;
+        }
+        const DevBox B = boxes[box];
+        if (B.kind != 0) return B.kind == 1 ? ADV_ENDED : ADV_PERIODIC;  // reservoir: deleted
+        double nx = x + dt * vx, ny = y + dt * vy;
+        int2 sr = make_int2(4 * box, 4);
+        if constexpr (POLY) sr = P.srange[box];
+        const bool inside = POLY ? poly_inside(P.sides, sr, nx, ny)
+                                 : (nx >= B.xmin) & (nx <= B.xmax) & (ny >= B.ymin) & (ny <= B.ymax);
+        if (inside) {
+            x = nx;
+            y = ny;
+            return ADV_ARRIVED;
+        }
+        double tf;
+        int aux, fast;
+        if constexpr (POLY) {
+            int m;
+            tf = poly_exit(P.sides, sr, x, y, vx, vy, m, nx, ny);
+            fast = poly_side_fast(P.sides, sr, m, nx, ny, vx, vy, aux);
+            if (fast == SIDE_MIXED) aux = m;
+        } else {
+            fast = rect_exit(B, x, y, vx, vy, ivx, ivy, tf, nx, ny, aux);
+        }
+        dt -= tf;
+        if (almost_equal(dt, 0.)) dt = 0.;
+        if (fast == SIDE_VOID) {
+            wall_hit(P, eb_lds, Eg, sr.x + aux, sign);
+            return ADV_ENDED;
+        }
+        x = nx;
+        y = ny;
+        if (fast < 0) {
+            mask = aux;
+            return ADV_SEARCH;
+        }
+        box = fast;
+        if (dt == 0.) return ADV_ARRIVED;
+    }
+}
+
+// evolparticle: ballistic advection by dt through box crossings, called by
+// every lane of the wave; returns whether the particle (alive) arrives.
+// A lane that meets a periodic box or an exit that needs the general search
+// waits at the end of the crossing loop, so that the long code of those cases
+// runs once for all of them.
 // With the exit test in selects, the boxes at a conflict-free stride and the
 // rare cases' parameters out of the loop's scalar registers (95 instead of 165
 // lane reads of spilled ones in the kernel) the step kernel takes 144.6 us
@@ -232,60 +306,37 @@ __device__ inline int advect_slow(bool eb_lds, int32_t* Eg, double& x, double& y
 // kernels use the instantiation without it, which needs fewer registers per
 // lane. POLY: convex polygon boxes (the geometry from the side tables).
 template <bool PER, bool POLY, bool GL>
-__device__ inline bool advect(const BertParams& P, const BertBoxes<GL>& boxes, bool eb_lds, int32_t* Eg, double& x,
-                              double& y, int& box, int sign, double vx, double vy, double ivx, double ivy,
+__device__ inline bool advect(const BertParams& P, const BertBoxes<GL>& boxes, bool alive, bool eb_lds, int32_t* Eg,
+                              double& x, double& y, int& box, int sign, double vx, double vy, double ivx, double ivy,
                               double dt, Pcg32& rng) {
-    for (int it = 0;;) {
-        int mask = -1;
-        for (;; it++) {
-            if (it >= 4096) {
-                atomicOr(P.flags + 2, 1u);
+    int it = 0, mask = 0;
+    if constexpr (!PER) {
+        if (!alive) return false;
+        for (;;) {
+            const int st = advect_cross<POLY, GL>(P, boxes, eb_lds, Eg, x, y, box, sign, vx, vy, ivx, ivy, dt, mask, it);
+            if (st <= ADV_ARRIVED) return st == ADV_ARRIVED;
+            if (st == ADV_PERIODIC) {  // the host launches PER whenever a box is periodic
+                atomicOr(P.flags + 3, 1u);
                 return false;
             }
-            const DevBox B = boxes[box];
-            if (B.kind != 0) {
-                if (B.kind == 1) return false;  // reservoir: deleted
-                mask = 0;
-                break;
-            }
-            double nx = x + dt * vx, ny = y + dt * vy;
-            int2 sr = make_int2(4 * box, 4);
-            if constexpr (POLY) sr = P.srange[box];
-            const bool inside = POLY ? poly_inside(P.sides, sr, nx, ny)
-                                     : (nx >= B.xmin) & (nx <= B.xmax) & (ny >= B.ymin) & (ny <= B.ymax);
-            if (inside) {
-                x = nx;
-                y = ny;
-                return true;
-            }
-            double tf;
-            int aux, fast;
-            if constexpr (POLY) {
-                int m;
-                tf = poly_exit(P.sides, sr, x, y, vx, vy, m, nx, ny);
-                fast = poly_side_fast(P.sides, sr, m, nx, ny, vx, vy, aux);
-                if (fast == SIDE_MIXED) aux = m;
-            } else {
-                fast = rect_exit(B, x, y, vx, vy, ivx, ivy, tf, nx, ny, aux);
-            }
-            dt -= tf;
-            if (almost_equal(dt, 0.)) dt = 0.;
-            if (fast == SIDE_VOID) {
-                wall_hit(P, eb_lds, Eg, sr.x + aux, sign);
-                return false;
-            }
-            x = nx;
-            y = ny;
-            if (fast < 0) {
-                mask = aux;
-                break;
-            }
-            box = fast;
+            if (!advect_slow<POLY>(eb_lds, Eg, x, y, box, sign, vx, vy, mask, rng)) return false;
             if (dt == 0.) return true;
         }
-        if (!advect_slow<PER, POLY>(eb_lds, Eg, x, y, box, sign, vx, vy, mask, rng)) return false;
-        if (mask != 0 && dt == 0.) return true;
-        it++;
+    } else {
+        // the wave stays together for the translation
+        int st = alive ? ADV_SEARCH : ADV_ENDED;
+        for (;;) {
+            if (st > ADV_ARRIVED)
+                st = advect_cross<POLY, GL>(P, boxes, eb_lds, Eg, x, y, box, sign, vx, vy, ivx, ivy, dt, mask, it);
+            if (__ballot(st > ADV_ARRIVED) == 0ULL) return st == ADV_ARRIVED;
+            if (__ballot(st == ADV_PERIODIC)) {
+                if (!advect_translate<POLY, GL>(boxes, st == ADV_PERIODIC, x, y, box, vx, vy, rng)) st = ADV_ENDED;
+            }
+            if (st == ADV_SEARCH) {
+                if (!advect_slow<POLY>(eb_lds, Eg, x, y, box, sign, vx, vy, mask, rng)) st = ADV_ENDED;
+                else if (dt == 0.) st = ADV_ARRIVED;
+            }
+        }
     }
 }
 
@@ -606,15 +657,17 @@ __device__ inline void box_lds_flush(const BertParams& P, int myseg) {
 // stay resident per CU
 // VL: one 1024-thread workgroup per CU with the mode velocities and their
 // inverses (32 B per mode) copied into LDS after the shared layout, so the
-// per-particle table reads are LDS reads; otherwise 256-thread workgroups,
-// five per CU for the P1 kernels, reading the tables from global memory.
+// per-particle table reads are LDS reads; otherwise 256-thread workgroups
+// reading the tables from global memory: five per CU for the P1 kernels, three
+// with periodic boxes (the bound keeps 170 registers, which would leave two,
+// at 168), four else.
 template <bool GL, bool PER, bool P1, bool POLY, bool VL = false>
-__global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) void bert_step_kernel(
+__global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : (PER ? 3 : (P1 ? 5 : 4))) void bert_step_kernel(
     BertParams P, uint32_t step, int cur, int cancel_prev, int hist) {
     __shared__ uint32_t tsum[16];
     __shared__ uint32_t lcount;
     uint32_t* pre = (uint32_t*)(bert_dyn + P.lds_pre);
-    const BertBoxes<GL> boxes = geo_stage<GL>(P);
+    const BertBoxes<GL> boxes = geo_stage<PER, GL>(P);
     const double2* vtab = P.vel;
     const double2* ivtab = P.ivel;
     if constexpr (VL) {
@@ -656,6 +709,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) v
         bool alive = false;
         Pcg32 rng;
         Pick0 f0{0u, 0u, make_uint2(0u, 0u)};
+        double2 v = make_double2(0., 0.), iv = v;
         if (valid) {
             while (sg < P.nsegs - 1 && i >= pre[sg]) sg++;
             const uint32_t off = i - (sg > 0 ? pre[sg - 1] : 0u);
@@ -689,12 +743,13 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : ((P1 && !PER) ? 5 : 1)) v
             if (alive) {
                 seed_stream(rng, skey, p.pid);
                 if (nslots_of<P1>(P) == 1) f0 = first_pick<P1>(P, rng, mode, 0);
-                const double2 v = vtab[mode];
-                const double2 iv = ivtab[mode];
-                alive = advect<PER, POLY, GL>(P, boxes, P.eb_lds != 0, Eg, p.x, p.y, box, sign, v.x, v.y, iv.x, iv.y, P.dt, rng);
-                if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, box);
+                v = vtab[mode];
+                iv = ivtab[mode];
             }
         }
+        alive = advect<PER, POLY, GL>(P, boxes, alive, P.eb_lds != 0, Eg, p.x, p.y, box, sign, v.x, v.y, iv.x, iv.y,
+                                      P.dt, rng);
+        if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, box);
         scatter_out<P1>(P, H, sbox, vtab, rng, f0, alive, mode, sign, box, p.x, p.y, p.pid, step, &lcount, myseg);
         done += alive ? 1 : 0;
     }
@@ -966,7 +1021,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
     const int myseg = P.seg_emit0 + blockIdx.x;
     uint32_t* segout = P.seg + (size_t)(cur ^ 1) * P.nsegs;
     if (threadIdx.x == 0) lcount = 0;
-    const BertBoxes<GL> boxes = geo_stage<GL>(P);
+    const BertBoxes<GL> boxes = geo_stage<PER, GL>(P);
     const double2* vtab = P.vel;
     const double2* ivtab = P.ivel;
     if constexpr (VL) {
@@ -997,7 +1052,8 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
         Pcg32 rng;
         Pick0 f0{0u, 0u, make_uint2(0u, 0u)};
         int mode = 0, bx = 0, sign = 1;
-        double x = 0, y = 0;
+        double x = 0, y = 0, rdt = 0;
+        double2 v = make_double2(0., 0.), iv = v;
         bool alive = false;
         uint64_t pid = 0;
         if (valid) {
@@ -1041,13 +1097,13 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
             double t = rng.uniform();
             x = p1x + t * ndx;
             y = p1y + t * ndy;
-            const double2 v = vtab[mode];
-            const double2 iv = ivtab[mode];
-            double rdt = P.dt * rng.uniform();
+            v = vtab[mode];
+            iv = ivtab[mode];
+            rdt = P.dt * rng.uniform();
             if (nslots_of<P1>(P) == 1) f0 = first_pick<P1>(P, rng, mode, 0);
-            alive = advect<PER, POLY, GL>(P, boxes, P.eb_lds != 0, Eg, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
-            if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, bx);
         }
+        alive = advect<PER, POLY, GL>(P, boxes, valid, P.eb_lds != 0, Eg, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
+        if (nslots_of<P1>(P) > 1 && alive) f0 = first_pick<P1>(P, rng, mode, bx);
         scatter_out<P1>(P, H, sbox, vtab, rng, f0, alive, mode, sign, bx, x, y, pid, step, &lcount, myseg);
         done += alive ? 1 : 0;
     }
@@ -1075,7 +1131,9 @@ struct BertSource {
     int32_t area, pad;
 };
 #define BERT_SRC_BLOCKS 256
-template <bool PER, bool POLY>
+// particles per step and part: one round of a workgroup's 256 threads
+#define BERT_SRC_PART 256.0
+template <bool GL, bool PER, bool POLY>
 __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const BertSource* src, int nparts_all,
                                                           const uint2* stab, uint32_t step, int cur, int hist) {
     __shared__ uint32_t lcount;
@@ -1083,10 +1141,10 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
     uint32_t* segout = P.seg + (size_t)(cur ^ 1) * P.nsegs;
     if (threadIdx.x == 0) lcount = 0;
     double* sbox = box_lds_begin(P);
+    const BertBoxes<GL> boxes = geo_stage<PER, GL>(P);
     __syncthreads();
     int32_t* Eb = P.Eb + (size_t)(step & 1) * P.nsd;
     unsigned long long* H = hist ? P.H + (size_t)cur * P.nbox * P.n : nullptr;
-    const BertBoxes<false> boxes{reinterpret_cast<const unsigned char*>(P.boxes)};
     unsigned long long done = 0;
     const int j0 = (int)((int64_t)nparts_all * blockIdx.x / gridDim.x);
     const int j1 = (int)((int64_t)nparts_all * (blockIdx.x + 1) / gridDim.x);
@@ -1107,7 +1165,8 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
             Pcg32 rng;
             Pick0 f0{0u, 0u, make_uint2(0u, 0u)};
             int mode = 0, bx = S.box, sign = S.sign;
-            double x = 0, y = 0;
+            double x = 0, y = 0, rdt = 0;
+            double2 v = make_double2(0., 0.), iv = v;
             bool alive = false;
             uint64_t pid = mix64(P.seed ^ ((uint64_t)step << 40) ^ ((uint64_t)S.src << 20) ^ (uint64_t)k ^ 0x15a0ULL);
             if (valid) {
@@ -1149,13 +1208,13 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
                 bool ngf;
                 mode = (int)alias_pick(stab + S.tab, (uint32_t)P.n, rng, ngf);
                 if (S.area) sign = ngf ? -1 : 1;
-                const double2 v = P.vel[mode];
-                const double2 iv = P.ivel[mode];
-                double rdt = P.dt * rng.uniform();
+                v = P.vel[mode];
+                iv = P.ivel[mode];
+                rdt = P.dt * rng.uniform();
                 if (nslots_of<false>(P) == 1) f0 = first_pick<false>(P, rng, mode, 0);
-                alive = advect<PER, POLY, false>(P, boxes, false, Eb, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
-                if (nslots_of<false>(P) > 1 && alive) f0 = first_pick<false>(P, rng, mode, bx);
             }
+            alive = advect<PER, POLY, GL>(P, boxes, valid, false, Eb, x, y, bx, sign, v.x, v.y, iv.x, iv.y, rdt, rng);
+            if (nslots_of<false>(P) > 1 && alive) f0 = first_pick<false>(P, rng, mode, bx);
             scatter_out<false>(P, H, sbox, P.vel, rng, f0, alive, mode, sign, bx, x, y, pid, step, &lcount, myseg);
             done += alive ? 1 : 0;
         }
@@ -1361,6 +1420,13 @@ static const EmitKernel emit_kernel_poly_tab[2][2] = {
     {bert_emit_kernel<false, false, false, true>, bert_emit_kernel<false, false, true, true>},
     {bert_emit_kernel<false, true, false, true>, bert_emit_kernel<false, true, true, true>}};
 
+using SourceKernel = void (*)(BertParams, const BertSource*, int, const uint2*, uint32_t, int, int);
+static const SourceKernel source_kernel_tab[2][2] = {
+    {bert_source_kernel<false, false, false>, bert_source_kernel<false, true, false>},
+    {bert_source_kernel<true, false, false>, bert_source_kernel<true, true, false>}};
+static const SourceKernel source_kernel_poly_tab[2] = {bert_source_kernel<false, false, true>,
+                                                       bert_source_kernel<false, true, true>};
+
 struct Bert {
     Ctx* ctx = nullptr;
     const Modes* m = nullptr;
@@ -1519,6 +1585,11 @@ static BertParams make_params(Bert* b) {
     P.boxes = b->g->d_boxes.p;
     P.cts = b->g->d_contacts.p;
     P.cseg = b->g->d_cseg.p;
+    P.per = b->g->d_per.p;
+    P.tcross = b->g->d_tcross.p;
+    P.box_per = b->g->d_box_per.p;
+    P.nper = (int32_t)b->g->per.size();
+    P.ntc = (int32_t)b->g->tcross.size();
     P.ptrans = b->g->d_ptrans.p;
     P.sides = b->g->d_sides.p;
     P.srange = b->g->d_srange.p;
@@ -1583,6 +1654,10 @@ static BertParams make_params(Bert* b) {
     if (P.lds_props) off = up16(off + sizeof(double) * 3 * (size_t)P.nbox);
     P.lds_boxes = (int32_t)off;
     if (b->geo_lds) off = up16(off + (size_t)BERT_BOX_LDS * P.nbox);
+    P.lds_per = (int32_t)off;
+    if (b->geo_lds && b->periodic) off += sizeof(DevPer) * (size_t)P.nper;
+    P.lds_tc = (int32_t)off;
+    if (b->geo_lds && b->periodic) off += sizeof(DevCross) * (size_t)P.ntc;
     b->lds_bytes = off;
     P.lds_vel = (int32_t)up16(off);
     b->lds_vl_bytes = up16(off) + 32 * (size_t)P.n;
@@ -1811,7 +1886,7 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     b->ninit = (int)inits.size();
     // one buffer segment per writing workgroup: step, emission, sources
     // reservoir sources (Isothermal_walls): expected particles per step,
-    // split over workgroups of at most ~1024 particles each
+    // split into parts of at most 256 particles each
     std::vector<BertSource> srcs;
     std::vector<uint2> stab;
     double src_total = 0;
@@ -1825,7 +1900,7 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
             double spf = hc.length() * cfg->thickness / vuc;
             build_alias(pmf.data(), n, th.data(), al.data());
             const double expected = cfg->dt * spf * cum / (b->Eeff * m->nq);
-            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / 1024.0)));
+            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / BERT_SRC_PART)));
             const int src = (int)(stab.size() / n);
             for (int part = 0; part < nparts; part++)
                 srcs.push_back(BertSource{hc.p1x, hc.p1y, hc.p2x - hc.p1x, hc.p2y - hc.p1y, expected, hc.box,
@@ -1867,7 +1942,7 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
             const double cumulsum = kB * acc;
             build_alias(pmf.data(), n, th.data(), al.data());
             const double expected = cfg->dt * (bx.area() * cfg->thickness / vuc) * cumulsum / (b->Eeff * m->nq);
-            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / 1024.0)));
+            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / BERT_SRC_PART)));
             const int src = (int)(stab.size() / n);
             for (int part = 0; part < nparts; part++)
                 srcs.push_back(BertSource{bx.xmin, bx.ymin, bx.xmax - bx.xmin, bx.ymax - bx.ymin, expected, i, 1,
@@ -1902,7 +1977,8 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     // 512-thread emission workgroups
     if (cfg->step_shape < 0 || cfg->step_shape > 1) throw Error(BTE_EINVAL, "step_shape must be 0 or 1");
     // boxes in LDS (polygon kernels read the geometry globally)
-    b->geo_lds = !g->poly && (size_t)BERT_BOX_LDS * nbox <= BERT_GEO_LDS_BYTES;
+    b->geo_lds = !g->poly && (size_t)BERT_BOX_LDS * nbox + sizeof(DevPer) * g->per.size() +
+                                     sizeof(DevCross) * g->tcross.size() <= BERT_GEO_LDS_BYTES;
     b->vl = !b->periodic && cfg->step_shape == 0;
     if (b->vl) {
         b->step_blocks = std::min(c->cu_count, BERT_MAXSEG - 512 - BERT_SRC_BLOCKS);
@@ -2203,8 +2279,7 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
                            s, P, (uint32_t)istep, cur, cancel_prev, hist);
         if (timed) HIPCHECK(hipEventRecord(b->kev[2 * istep + 1], s));
         if (b->nsrc)
-            hipLaunchKernelGGL(b->g->poly ? (b->periodic ? bert_source_kernel<true, true> : bert_source_kernel<false, true>)
-                                          : (b->periodic ? bert_source_kernel<true, false> : bert_source_kernel<false, false>),
+            hipLaunchKernelGGL(b->g->poly ? source_kernel_poly_tab[b->periodic] : source_kernel_tab[b->geo_lds][b->periodic],
                                dim3(b->src_blocks),
                                dim3(256), b->lds_bytes, s, P, b->d_src.p, b->nsrc, b->d_src_tab.p, (uint32_t)istep,
                                cur, hist);

@@ -581,6 +581,28 @@ static void rect_contacts(Geom* g) {
 // their contact ranges and side neighbours, contact segments, and the sides
 // (rectangles: left, bottom, top, right; polygons: hull edges) with the ids
 // of their outward normals.
+// the periodic boxes' records and their targets' contacts (asynchronous; the
+// vectors stay with the geometry)
+static void upload_periodic(Geom* g) {
+    const int nbox = (int)g->dboxes.size();
+    g->per.clear();
+    g->tcross.clear();
+    g->box_per.assign(nbox, -1);
+    for (int i = 0; i < nbox; i++) {
+        const DevBox& d = g->dboxes[i];
+        if (d.kind != 2 || d.tgt < 0) continue;
+        const DevBox& t = g->dboxes[d.tgt];
+        const int t0 = (int)g->tcross.size();
+        g->tcross.insert(g->tcross.end(), g->cross.begin() + t.c0, g->cross.begin() + t.c1);
+        g->box_per[i] = (int32_t)g->per.size();
+        g->per.push_back(DevPer{t.xmin, t.xmax, t.ymin, t.ymax, g->ptrans[i], t0, (int)g->tcross.size(), d.tgt, 0});
+    }
+    hipStream_t s = g->ctx->stream;
+    g->d_per.upload(g->per.empty() ? std::vector<DevPer>(1) : g->per, s);
+    g->d_tcross.upload(g->tcross.empty() ? std::vector<DevCross>(1) : g->tcross, s);
+    g->d_box_per.upload(g->box_per, s);
+}
+
 static void finish_geom(Geom* g) {
     const int nbox = (int)g->boxes.size();
     for (int i = 0; i < nbox; i++)
@@ -614,6 +636,10 @@ static void finish_geom(Geom* g) {
             const double ux = L > 0 ? (hc.p2x - hc.p1x) / L : 0., uy = L > 0 ? (hc.p2y - hc.p1y) / L : 0.;
             g->cseg.push_back(make_double4(hc.p1x - 1.0e-6 * ux, hc.p1y - 1.0e-6 * uy, hc.p2x + 1.0e-6 * ux,
                                            hc.p2y + 1.0e-6 * uy));
+            const double4 sg = g->cseg.back();
+            const RectBox& nb = g->boxes[hc.box];
+            g->cross.push_back(DevCross{nb.xmin, nb.xmax, nb.ymin, nb.ymax, sg.x, sg.y, sg.z, sg.w, hc.box,
+                                        nb.kind == 0 ? 1 : 0, {0, 0}});
         }
         d.c1 = (int32_t)g->dcontacts.size();
         d.tgt = -1;
@@ -670,7 +696,9 @@ static void finish_geom(Geom* g) {
     g->d_boxes.upload(g->dboxes, c->stream);
     g->d_contacts.upload(g->dcontacts.empty() ? std::vector<DevContact>(1) : g->dcontacts, c->stream);
     g->d_cseg.upload(g->cseg.empty() ? std::vector<double4>(1) : g->cseg, c->stream);
+    g->d_cross.upload(g->cross.empty() ? std::vector<DevCross>(1) : g->cross, c->stream);
     g->d_ptrans.upload(g->ptrans, c->stream);
+    upload_periodic(g);
     g->d_sides.upload(g->sides, c->stream);
     g->d_srange.upload(g->srange, c->stream);
     HIPCHECK(hipStreamSynchronize(c->stream));
@@ -788,6 +816,7 @@ int bte_geom_set_periodic(bte_geom* gg, int box, int target, double tx, double t
     HIPCHECK(hipSetDevice(g->ctx->device));
     g->d_boxes.upload(g->dboxes, g->ctx->stream);
     g->d_ptrans.upload(g->ptrans, g->ctx->stream);
+    upload_periodic(g);
     HIPCHECK(hipStreamSynchronize(g->ctx->stream));
     BTE_GUARD_END
 }

@@ -71,6 +71,7 @@ struct RtaParams {
     const DevBox* boxes;
     const DevContact* cts;
     const double4* cseg;    // contact segments (periodic translation)
+    const DevCross* cross;  // contacts as translate_rect reads them
     const double2* ptrans;  // periodic translation per box
     // polygon geometries (POLY kernels): sides, side range and centre per box
     const DevSide* sides;
@@ -577,7 +578,7 @@ __device__ inline void rta_slow(const RtaGeo<GL>& G, RtaState& S, RtaCounts& C) 
         // periodic box: translate, keep the remaining flight (RTA_MC2D.cpp:1034-1043)
         const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, abox, S.x, S.y,
                                              vx, vy, S.rng)
-                            : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, abox, S.x, S.y, vx, vy, S.rng);
+                            : translate_rect(P.boxes, P.cross, P.ptrans, abox, S.x, S.y, vx, vy, S.rng);
         if (nb < 0) {
             atomicAdd(P.counters + 5, 1ULL);
             S.st = RTA_DEAD;
@@ -1206,6 +1207,7 @@ struct RtaBatch {
     DevBuf<DevBox> d_boxes;
     DevBuf<DevContact> d_cts;
     DevBuf<double4> d_cseg;
+    DevBuf<DevCross> d_cross;
     DevBuf<double2> d_ptrans;
     DevBuf<double> d_timegrid, d_tally, d_dgz;
     DevBuf<RtaRunDev> d_runs, d_trial_runs;
@@ -1355,6 +1357,7 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
     P.boxes = b->d_boxes.p;
     P.cts = b->d_cts.p;
     P.cseg = b->d_cseg.p;
+    P.cross = b->d_cross.p;
     P.ptrans = b->d_ptrans.p;
     P.sides = b->d_sides.p;
     P.srange = b->d_srange.p;
@@ -1527,6 +1530,7 @@ static void batch_create(RtaBatch* b) {
     std::vector<DevBox> boxes;
     std::vector<DevContact> cts;
     std::vector<double4> cseg;
+    std::vector<DevCross> cross;
     std::vector<double2> ptrans;
     std::vector<uint64_t> lrow_cell;
     std::vector<RtaBox> rboxes;
@@ -1628,6 +1632,10 @@ static void batch_create(RtaBatch* b) {
             cts.push_back(ct);
         }
         cseg.insert(cseg.end(), g->cseg.begin(), g->cseg.end());
+        for (auto q : g->cross) {
+            q.box += bo;
+            cross.push_back(q);
+        }
         b->cells += (uint64_t)nb * nt;
         b->run_lrows.push_back((int32_t)b->lrows - b->run_lrow0.back());
         // BE_derivative sampler at the run temperature (sampling.cpp:47-68)
@@ -1677,6 +1685,7 @@ static void batch_create(RtaBatch* b) {
     }
     b->d_cts.upload(cts.empty() ? std::vector<DevContact>(1) : cts, s);
     b->d_cseg.upload(cseg.empty() ? std::vector<double4>(1) : cseg, s);
+    b->d_cross.upload(cross.empty() ? std::vector<DevCross>(1) : cross, s);
     b->d_ptrans.upload(ptrans, s);
     b->d_lrow_cell.upload(lrow_cell.empty() ? std::vector<uint64_t>(1) : lrow_cell, s);
     // arrays of the FP32 tallies: gz, jx, jy, then one per side that some run
@@ -2352,6 +2361,7 @@ struct RtaSteadyParams {
     const DevBox* boxes;
     const DevContact* cts;
     const double4* cseg;
+    const DevCross* cross;
     const double2* ptrans;
     const DevSide* sides;     // polygon geometries: sides, side range and centre per box
     const int2* srange;
@@ -2498,7 +2508,7 @@ __global__ __launch_bounds__(256) void rta_steady_flight_kernel(RtaSteadyParams 
                 if (B.kind == 2) {
                     const int nb = POLY ? translate_poly(P.boxes, P.sides, P.srange, P.cts, P.cseg, P.ptrans, box, x,
                                                          y, md.x, md.y, rng)
-                                        : translate_rect(P.boxes, P.cts, P.cseg, P.ptrans, box, x, y, md.x, md.y, rng);
+                                        : translate_rect(P.boxes, P.cross, P.ptrans, box, x, y, md.x, md.y, rng);
                     if (nb < 0) { badtrans++; break; }
                     box = nb;
                     continue;
@@ -2775,6 +2785,7 @@ extern "C" int bte_rta_steady_run(bte_ctx* ctx, const bte_modes* mm, const bte_g
     P.boxes = g->d_boxes.p;
     P.cts = g->d_contacts.p;
     P.cseg = g->d_cseg.p;
+    P.cross = g->d_cross.p;
     P.ptrans = g->d_ptrans.p;
     P.sides = g->d_sides.p;
     P.srange = g->d_srange.p;

@@ -118,6 +118,12 @@ struct Geom {
     std::vector<DevBox> dboxes;
     std::vector<DevContact> dcontacts;
     std::vector<double4> cseg;     // per contact: shared segment extended by 1e-6
+    std::vector<DevCross> cross;   // per contact: the neighbour and that segment
+    // periodic boxes of rectangle geometries: their records, the contacts of
+    // their targets and the record of each box (-1: none)
+    std::vector<DevPer> per;
+    std::vector<DevCross> tcross;
+    std::vector<int32_t> box_per;
     std::vector<double2> ptrans;   // per box: periodic translation (0 otherwise)
     // sides of every box (rectangles: left, bottom, top, right at 4 i ..
     // 4 i + 3), their ranges per box and the distinct outward normals
@@ -128,6 +134,9 @@ struct Geom {
     DevBuf<DevBox> d_boxes;
     DevBuf<DevContact> d_contacts;
     DevBuf<double4> d_cseg;
+    DevBuf<DevCross> d_cross, d_tcross;
+    DevBuf<DevPer> d_per;
+    DevBuf<int32_t> d_box_per;
     DevBuf<double2> d_ptrans;
     DevBuf<DevSide> d_sides;
     DevBuf<int2> d_srange;
