@@ -519,6 +519,23 @@ __device__ inline int seg_search(const uint32_t* pre, int nsegs, uint32_t i) {
     return l;
 }
 
+// first segment at or after s with pre > i (the last one when there is none).
+// Mostly it is s or the next one; where many segments in a row are empty (the
+// emission workgroups' of a geometry without walls: 512 of them between the
+// step and the source workgroups') a search replaces the walk, which alone
+// kept one wave of the step kernel busy for 30 us.
+__device__ inline int seg_from(const uint32_t* pre, int nsegs, int s, uint32_t i) {
+    if (s >= nsegs - 1 || i < pre[s]) return s;
+    s++;
+    if (s >= nsegs - 1 || i < pre[s]) return s;
+    int l = s + 1, h = nsegs - 1;
+    while (l < h) {
+        const int mid = (l + h) >> 1;
+        if (pre[mid] <= i) l = mid + 1; else h = mid;
+    }
+    return l;
+}
+
 // wave-wide exclusive prefix sum of c; one LDS atomic on the workgroup's
 // segment counter gives the wave's base. Returns this lane's slot.
 __device__ inline uint64_t wave_reserve(uint32_t* lds_count, int myseg, uint32_t segcap, int c,
@@ -702,7 +719,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : (PER ? 3 : (P1 ? 5 : 4)))
         const uint32_t i = base + threadIdx.x;
         const bool valid = i < hi;
         const uint32_t wfirst = base + (threadIdx.x & ~63u);
-        while (sgw < P.nsegs - 1 && wfirst >= pre[sgw]) sgw++;
+        sgw = seg_from(pre, P.nsegs, sgw, wfirst);
         int sg = sgw;
         BPart p{};
         int box = 0, sign = 1, mode = 0;
@@ -711,7 +728,7 @@ __global__ __launch_bounds__(VL ? 1024 : 256, VL ? 1 : (PER ? 3 : (P1 ? 5 : 4)))
         Pick0 f0{0u, 0u, make_uint2(0u, 0u)};
         double2 v = make_double2(0., 0.), iv = v;
         if (valid) {
-            while (sg < P.nsegs - 1 && i >= pre[sg]) sg++;
+            sg = seg_from(pre, P.nsegs, sgw, i);
             const uint32_t off = i - (sg > 0 ? pre[sg - 1] : 0u);
             p = P.pin[(uint64_t)sg * P.segcap + off];
             box = (int)(p.boxsign >> 1);
@@ -1048,7 +1065,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
         const uint32_t k = base + threadIdx.x;
         const bool valid = k < hi;
         const uint32_t wfirst = base + (threadIdx.x & ~63u);
-        while (bw < nb4 - 1 && wfirst >= pre[bw]) bw++;
+        bw = seg_from(pre, nb4, bw, wfirst);
         Pcg32 rng;
         Pick0 f0{0u, 0u, make_uint2(0u, 0u)};
         int mode = 0, bx = 0, sign = 1;
@@ -1058,8 +1075,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
         uint64_t pid = 0;
         if (valid) {
             // side b holds indices [pre[b-1], pre[b])
-            int b = bw;
-            while (b < nb4 - 1 && k >= pre[b]) b++;
+            const int b = seg_from(pre, nb4, bw, k);
             const uint32_t j = k - (b > 0 ? pre[b - 1] : 0u);
             bx = POLY ? P.side_box[b] : b >> 2;
             const int side = b & 3;

@@ -415,8 +415,8 @@ struct __align__(16) DevPer {
 // that rounding could grow). The lanes then test what is left, one or two
 // contacts each, all at once. The candidates are taken in the contacts' order,
 // so the choice and its draw are those of translate_rect. Bar of 41 bins, 9e4
-// particles: step kernel 73 -> 52 us (30 us of them one wave's walk over empty
-// buffer segments), source kernel (2000 particles) 138 -> 12 us.
+// particles: step kernel 73 -> 22 us (52 us before the walk of one wave over empty
+// buffer segments became a search), source kernel (2000 particles) 138 -> 12 us.
 template <class Rng>
 __device__ inline int translate_rect_wave(bool want, const DevPer* per, const DevCross* cross, int pi, double& x,
                                           double& y, double vx, double vy, Rng& rng) {

@@ -597,10 +597,11 @@ static void upload_periodic(Geom* g) {
         g->box_per[i] = (int32_t)g->per.size();
         g->per.push_back(DevPer{t.xmin, t.xmax, t.ymin, t.ymax, g->ptrans[i], t0, (int)g->tcross.size(), d.tgt, 0});
     }
+    if (g->per.empty()) return;
     hipStream_t s = g->ctx->stream;
-    g->d_per.upload(g->per.empty() ? std::vector<DevPer>(1) : g->per, s);
-    g->d_tcross.upload(g->tcross.empty() ? std::vector<DevCross>(1) : g->tcross, s);
-    g->d_box_per.upload(g->box_per, s);
+    g->d_per.upload(g->per.data(), g->per.size(), s);
+    g->d_tcross.upload(g->tcross.data(), g->tcross.size(), s);
+    g->d_box_per.upload(g->box_per.data(), g->box_per.size(), s);
 }
 
 static void finish_geom(Geom* g) {

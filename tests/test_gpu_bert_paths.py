@@ -34,3 +34,42 @@ def test_launch_shapes_agree(pkg, ctx, nb, rows, n):
     assert (a["npart"] + a["pending"] == a["npart"][0]).all() and a["npart"][0] > 0
     scale = np.abs(c["props"]).max(axis=(0, 1))
     np.testing.assert_allclose(a["props"] / scale, c["props"] / scale, rtol=0, atol=1e-10)
+
+
+def _periodic_bar(nb, extra, width=30.0, dx=10.0):
+    """nb boxes periodic in y between a 302 K and a 300 K reservoir, and
+    `extra` bars of the same kind without a temperature difference far away"""
+    rect, kind, teq, per = [], [], [], {}
+    for e in range(1 + extra):
+        y0, L, b0 = 1000.0 * e, nb * dx, len(rect)
+        rect += [[k * dx, (k + 1) * dx, y0, y0 + width] for k in range(nb)]
+        rect += [[0.0, L, y0 - 2.0, y0], [0.0, L, y0 + width, y0 + width + 2.0]]
+        rect += [[-dx, 0.0, y0, y0 + width], [L, L + dx, y0, y0 + width]]
+        kind += [0] * nb + [2, 2, 1, 1]
+        teq += [300.0] * (nb + 2) + [302.0 if e == 0 else 300.0, 300.0]
+        per.update({b0 + nb: (b0 + nb + 1, 0.0, width), b0 + nb + 1: (b0 + nb, 0.0, -width)})
+    return np.array(rect), np.array(kind, np.int32), np.array(teq), per
+
+
+@pytest.mark.parametrize("nb,extra", [(12, 20), (70, 3), (150, 1)])
+def test_periodic_tables_in_lds_and_in_global_memory(pkg, ctx, nb, extra):
+    """A bar alone (its boxes and periodic tables in LDS; past 64 contacts the
+    search takes several rounds) and with others that push the tables past
+    48 KB: the bar's histories are the same."""
+    W = pkg.workloads
+    mat = W.material(80, seed=5)
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    kw = dict(thickness=1.0, dt=4.0, maxtime=76.0, max_steps=20, rta=True, seed=3)
+    out = []
+    Ed = -1.0
+    for e in (0, extra):
+        rect, kind, teq, per = _periodic_bar(nb, e)
+        geom = pkg.Geometry(ctx, rect, kind, teq, periodic=per)
+        b = pkg.BertRun(ctx, modes, geom, None, Ed=Ed, Efactor=400, Tmax=302.0, Tmin=300.0, **kw)
+        out.append(b.execute())
+        Ed = out[0]["Eeff"]
+        b.close()
+    a, c = out
+    assert np.array_equal(a["npart"], c["npart"]) and a["npart"][-1] > 1000
+    scale = np.abs(a["props"]).max(axis=(0, 1))
+    np.testing.assert_allclose(c["props"][:, :nb] / scale, a["props"][:, :nb] / scale, rtol=0, atol=1e-10)
