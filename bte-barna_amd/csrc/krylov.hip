@@ -264,13 +264,79 @@ struct Basis {
 };
 __device__ inline size_t il(size_t x) { return 2 * (x & ~(size_t)7) + (x & 7); }
 
-// c = exp(H_i) e_1 for every column: one wave per column, H in LDS.
-// Scaling and squaring (the method of Eigen's MatrixExponential, which the
-// reference's build_P calls): with ||H/2^s||_1 <= 1/2 each factor
-// exp(H/2^s) is a Taylor polynomial of degree <= 24. When 2^s <= m the
-// factor is applied 2^s times to the vector; otherwise E = exp(H/2^s) is
-// formed column by column and squared s times, and c is its first column
-// (cost O(s m^3) instead of O(2^s m^2) for large norms).
+// c = exp(H_i) e_1 for every column. Scaling (the method of Eigen's
+// MatrixExponential, which the reference's build_P calls, scales and squares):
+// with ||H/2^s||_1 <= 1 the factor exp(H/2^s) is a Taylor polynomial of degree
+// KR_TAYLOR (1/21! < 2e-20), applied 2^s times to the vector
+// (kr_expm_e1_vec). Norms that need more than KR_MAX_APPLY applications are
+// left to kr_expm_e1_sq, where E = exp(H/2^s) with ||H/2^s||_1 <= 1/2 is formed
+// column by column and squared s times, and c is its first column (cost
+// O(s m^3) instead of O(2^s m^2)).
+#define KR_TAYLOR 20
+#define KR_MAX_APPLY 64
+
+// the scaling of column H_i: s with ||H_i / 2^s||_1 <= theta, -1 when H_i is
+// not finite; cs: the 1-norm
+__device__ inline int kr_scaling(double cs, double theta) {
+    if (!(cs < 1.0e300)) return -1;
+    return cs > theta ? (int)ceil(log2(cs / theta)) : 0;
+}
+
+// ML lanes per column (64 / ML columns per wave, m <= ML): lane l keeps row l
+// of the scaled H in registers and the vector passes through LDS, two doubles
+// per broadcast read; the number of terms is fixed, so no term waits for a
+// reduction. Bound by the chain of 2^s KR_TAYLOR products of m terms: 4096
+// columns of m = 30 and norms near 10 took 1360 us with H in LDS, one column
+// per wave and a maximum over the wave after each term (and, as 2^s > m, by
+// squaring), now 120 us.
+template <int ML>
+__global__ __launch_bounds__(64) void kr_expm_e1_vec(const double* __restrict__ H, double* __restrict__ C, int m,
+                                                     int N) {
+    constexpr int NC = 64 / ML;
+    __shared__ __align__(16) double vec[NC][ML];
+    const int l = threadIdx.x % ML, g = threadIdx.x / ML;
+    const int i = blockIdx.x * NC + g;
+    const bool on = i < N && l < m;
+    const double* Hi = H + (size_t)min(i, N - 1) * m * m;  // column-major
+    double cs = 0.;
+    if (on)
+        for (int r = 0; r < m; r++) cs += fabs(Hi[r + l * m]);
+    for (int d = ML / 2; d > 0; d >>= 1) cs = fmax(cs, __shfl_xor(cs, d, 64));
+    const int s = kr_scaling(cs, 1.0);
+    if (s < 0 && on) C[(size_t)i * m + l] = __builtin_nan("");  // a non-finite Hessenberg matrix yields NaN
+    const bool here = s >= 0 && s < 31 && (1 << s) <= KR_MAX_APPLY;
+    const double sc = here ? ldexp(1.0, -s) : 0.;
+    double row[ML];
+#pragma unroll
+    for (int c = 0; c < ML; c++) row[c] = (on && c < m && here) ? Hi[l + c * m] * sc : 0.;
+    double v = l == 0 ? 1.0 : 0.0;
+    int reps = here ? 1 << s : 0;  // the column's own; the wave runs the larger count
+    int most = reps;
+    for (int d = 32; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
+    const double2* x = reinterpret_cast<const double2*>(vec[g]);
+    for (int rp = 0; rp < most; rp++) {
+        double acc = v, term = v;
+        for (int k = 1; k <= KR_TAYLOR; k++) {
+            vec[g][l] = term;
+            __syncthreads();
+            double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
+#pragma unroll
+            for (int c = 0; c < ML / 2; c += 2) {
+                const double2 p = x[c], q = x[c + 1];
+                a0 = fma(row[2 * c], p.x, a0);
+                a1 = fma(row[2 * c + 1], p.y, a1);
+                a2 = fma(row[2 * c + 2], q.x, a2);
+                a3 = fma(row[2 * c + 3], q.y, a3);
+            }
+            term = ((a0 + a1) + (a2 + a3)) / (double)k;
+            acc += term;
+            __syncthreads();
+        }
+        if (rp < reps) v = acc;
+    }
+    if (on && here) C[(size_t)i * m + l] = v;
+}
+
 __device__ inline void kr_taylor_apply(const double* Hs, double* v, double* t, int m, int l) {
     double acc = l < m ? v[l] : 0.;
     double term = acc;
@@ -292,40 +358,28 @@ __device__ inline void kr_taylor_apply(const double* Hs, double* v, double* t, i
     __syncthreads();
 }
 
-__global__ __launch_bounds__(64) void kr_expm_e1(const double* __restrict__ H, double* __restrict__ C,
-                                                 int m) {
+// one wave per column, H in LDS; columns that kr_expm_e1_vec has done are passed over
+__global__ __launch_bounds__(64) void kr_expm_e1_sq(const double* __restrict__ H, double* __restrict__ C,
+                                                    int m) {
     extern __shared__ double sh[];
     double* Hs = sh;            // m*m
     double* v = sh + m * m;     // m
     double* t = v + m;          // m
-    double* E = t + m;          // m*m (squaring path)
-    double* W = E + m * m;      // m*m (squaring path)
+    double* E = t + m;          // m*m
+    double* W = E + m * m;      // m*m
     const int i = blockIdx.x, l = threadIdx.x;
     const double* Hi = H + (size_t)i * m * m;
-    for (int q = l; q < m * m; q += 64) Hs[q] = Hi[q];
-    __syncthreads();
     // 1-norm
     double cs = 0;
     if (l < m)
-        for (int r = 0; r < m; r++) cs += fabs(Hs[r + l * m]);
+        for (int r = 0; r < m; r++) cs += fabs(Hi[r + l * m]);
     for (int d = 32; d > 0; d >>= 1) cs = fmax(cs, __shfl_xor(cs, d, 64));
-    // a non-finite Hessenberg matrix yields NaN
-    if (!(cs < 1.0e300)) {
-        if (l < m) C[(size_t)i * m + l] = __builtin_nan("");
-        return;
-    }
-    int s = 0;
-    if (cs > 0.5) s = (int)ceil(log2(cs / 0.5));
+    const int s1 = kr_scaling(cs, 1.0);
+    if (s1 < 0 || (s1 < 31 && (1 << s1) <= KR_MAX_APPLY)) return;
+    const int s = kr_scaling(cs, 0.5);
     const double sc = ldexp(1.0, -s);
-    for (int q = l; q < m * m; q += 64) Hs[q] *= sc;
+    for (int q = l; q < m * m; q += 64) Hs[q] = Hi[q] * sc;
     __syncthreads();
-    if (s < 31 && (1L << s) <= m) {
-        if (l < m) v[l] = l == 0 ? 1.0 : 0.0;
-        __syncthreads();
-        for (long rp = 0; rp < (1L << s); rp++) kr_taylor_apply(Hs, v, t, m, l);
-        if (l < m) C[(size_t)i * m + l] = v[l];
-        return;
-    }
     for (int j = 0; j < m; j++) {
         if (l < m) v[l] = l == j ? 1.0 : 0.0;
         __syncthreads();
@@ -897,9 +951,12 @@ extern "C" int bte_krylov_build(bte_ctx* ctx, int N, const double* B, double dt,
     }
     {
         const size_t lds = (size_t)(3 * m * m + 2 * m) * sizeof(double);
-        HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&kr_expm_e1),
+        HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&kr_expm_e1_sq),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kr_expm_e1, dim3(N), dim3(64), lds, s, dH.p, dC.p, m);
+        if (m <= 16) hipLaunchKernelGGL(kr_expm_e1_vec<16>, dim3((N + 3) / 4), dim3(64), 0, s, dH.p, dC.p, m, N);
+        else if (m <= 32) hipLaunchKernelGGL(kr_expm_e1_vec<32>, dim3((N + 1) / 2), dim3(64), 0, s, dH.p, dC.p, m, N);
+        else hipLaunchKernelGGL(kr_expm_e1_vec<64>, dim3(N), dim3(64), 0, s, dH.p, dC.p, m, N);
+        hipLaunchKernelGGL(kr_expm_e1_sq, dim3(N), dim3(64), lds, s, dH.p, dC.p, m);
     }
     HIPCHECK(hipGetLastError());
     if (vec) {
