@@ -2,11 +2,17 @@
 // synthetic inputs, alias tables and the small host-side physics used to
 // build device tables.
 #include "runtime.hpp"
+#include "staging.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <numeric>
 #include <limits>
+#include <atomic>
+#include <exception>
+#include <system_error>
+#include <sys/mman.h>
+#include <unistd.h>
 
 namespace bte {
 
@@ -236,6 +242,132 @@ double Spline::eval(double x) const {
     if (idx >= a.size()) idx--;
     double dx = x - x0[idx];
     return a[idx] + dx * (b[idx] + dx * (c[idx] + d[idx] * dx));
+}
+
+// ---- large copies through pinned chunks (staging.hpp) ----
+
+// f(0) .. f(n - 1), each in a thread of its own as far as there are threads;
+// f takes its work from a shared counter, so any number of them does it all
+template <class F>
+static void on_threads(int n, F f) {
+    std::vector<std::exception_ptr> err(n);
+    auto one = [&](int t) {
+        try {
+            f(t);
+        } catch (...) {
+            err[t] = std::current_exception();
+        }
+    };
+    {
+        std::vector<StageThread> th(n - 1);
+        try {
+            for (int t = 1; t < n; t++) th[t - 1].t = std::thread(one, t);
+        } catch (const std::system_error&) {
+        }
+        one(0);
+    }
+    for (auto& e : err)
+        if (e) std::rethrow_exception(e);
+}
+
+Staging::~Staging() {
+    if (bg.t.joinable()) bg.t.join();
+    if (!mine) return;
+    (void)hipStreamSynchronize(c->stream);  // copies may still read the chunks
+    c->chunks.busy.store(false);
+}
+
+bool Staging::ready(const void* user, size_t bytes) {
+    if (bytes < STAGE_MIN) return false;
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, user) != hipSuccess)
+        (void)hipGetLastError();  // memory that the runtime does not know
+    else if (at.type != hipMemoryTypeUnregistered)
+        return false;
+    if (!mine && c->chunks.busy.exchange(true)) return false;
+    mine = true;
+    StageChunks& sc = c->chunks;
+    if (!sc.pin && hipHostMalloc((void**)&sc.pin, BYTES, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        sc.pin = nullptr;
+        return false;
+    }
+    while (sc.ev.size() < (size_t)THREADS * SLOTS) {
+        hipEvent_t e;
+        HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        sc.ev.push_back(e);
+    }
+    return true;
+}
+
+void Staging::upload(void* dst, const void* src, size_t bytes) {
+    if (!ready(src, bytes)) {
+        HIPCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        return;
+    }
+    const size_t nc = (bytes + CHUNK - 1) / CHUNK;
+    std::atomic<size_t> next{0};
+    on_threads(THREADS, [&](int t) {
+        HIPCHECK(hipSetDevice(c->device));
+        for (int q = 0;; q = (q + 1) % SLOTS) {
+            const size_t k = next.fetch_add(1);
+            if (k >= nc) return;
+            const int slot = t * SLOTS + q;
+            char* buf = c->chunks.pin + (size_t)slot * CHUNK;
+            const size_t off = k * CHUNK, len = std::min(CHUNK, bytes - off);
+            HIPCHECK(hipEventSynchronize(c->chunks.ev[slot]));  // of the copy before; at once if there was none
+            memcpy(buf, (const char*)src + off, len);
+            HIPCHECK(hipMemcpyAsync((char*)dst + off, buf, len, hipMemcpyHostToDevice, c->stream));
+            HIPCHECK(hipEventRecord(c->chunks.ev[slot], c->stream));
+        }
+    });
+}
+
+void Staging::prefault(void* dst, size_t bytes) {
+#ifdef MADV_POPULATE_WRITE
+    if (!ready(dst, bytes)) return;
+    try {
+        bg.t = std::thread([=] {
+            const uintptr_t pg = (uintptr_t)sysconf(_SC_PAGESIZE), b = ((uintptr_t)dst + pg - 1) / pg * pg,
+                            e = ((uintptr_t)dst + bytes) / pg * pg;
+            // in parts, so that no part holds the memory map for long
+            for (uintptr_t a = b; a < e; a += CHUNK)
+                if (madvise((void*)a, std::min((size_t)(e - a), CHUNK), MADV_POPULATE_WRITE) != 0) return;
+        });
+    } catch (const std::system_error&) {
+    }
+#endif
+}
+
+void Staging::download(void* dst, const void* src, size_t bytes) {
+    if (bg.t.joinable()) bg.t.join();
+    if (!ready(dst, bytes)) {
+        HIPCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+        return;
+    }
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    const size_t nc = (bytes + CHUNK - 1) / CHUNK;
+    std::atomic<size_t> next{0};
+    on_threads(THREADS, [&](int t) {
+        HIPCHECK(hipSetDevice(c->device));
+        size_t k[SLOTS];
+        auto start = [&](int q) {
+            k[q] = next.fetch_add(1);
+            if (k[q] >= nc) return;
+            const int slot = t * SLOTS + q;
+            HIPCHECK(hipMemcpyAsync(c->chunks.pin + (size_t)slot * CHUNK, (const char*)src + k[q] * CHUNK,
+                                    std::min(CHUNK, bytes - k[q] * CHUNK), hipMemcpyDeviceToHost, c->stream));
+            HIPCHECK(hipEventRecord(c->chunks.ev[slot], c->stream));
+        };
+        for (int q = 0; q < SLOTS; q++) start(q);
+        for (int q = 0; k[q] < nc; q = (q + 1) % SLOTS) {
+            const int slot = t * SLOTS + q;
+            HIPCHECK(hipEventSynchronize(c->chunks.ev[slot]));
+            memcpy((char*)dst + k[q] * CHUNK, c->chunks.pin + (size_t)slot * CHUNK, std::min(CHUNK, bytes - k[q] * CHUNK));
+            start(q);
+        }
+    });
 }
 
 }  // namespace bte

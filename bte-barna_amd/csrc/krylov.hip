@@ -11,6 +11,7 @@
 // energy projection (collision_operator.cpp:786-807 applied to P: columns
 // sum to one).
 #include "runtime.hpp"
+#include "staging.hpp"
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 #include <hip/hip_bf16.h>
@@ -852,7 +853,9 @@ extern "C" int bte_krylov_build(bte_ctx* ctx, int N, const double* B, double dt,
     DevBuf<double> dV64;
     DevBuf<__hip_bfloat16> dAil, dVil;
     DevBuf<int> dClosed;
-    dB.upload(B, NN, s);
+    Staging st(c);
+    dB.alloc(NN);
+    st.upload(dB.p, B, NN * sizeof(double));
     Basis V{nullptr, nullptr, nullptr, nullptr, prec, N, (size_t)N};
     // BF16: N padded to the product kernel's 256 with zero rows and columns
     const int Np = prec == 2 ? (N + gk::TM - 1) / gk::TM * gk::TM : N;
@@ -912,6 +915,7 @@ extern "C" int bte_krylov_build(bte_ctx* ctx, int N, const double* B, double dt,
     for (auto& e : eg.ev) HIPCHECK(hipEventCreate(&e));
     const hipEvent_t e0 = eg.ev[0], e1 = eg.ev[1];
     HIPCHECK(hipEventRecord(e0, s));
+    st.prefault(P, NN * sizeof(double));
     int gemms = 0;
     const bool vec = N % 8 == 0;  // vector Gram-Schmidt and combine kernels
     const double one = 1.0, zero = 0.0;
@@ -970,7 +974,7 @@ extern "C" int bte_krylov_build(bte_ctx* ctx, int N, const double* B, double dt,
     }
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(e1, s));
-    HIPCHECK(hipMemcpyAsync(P, dP.p, NN * sizeof(double), hipMemcpyDeviceToHost, s));
+    st.download(P, dP.p, NN * sizeof(double));
     std::vector<double> err(N);
     std::vector<int> closed(N);
     HIPCHECK(hipMemcpyAsync(err.data(), dErr.p, N * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1052,7 +1056,9 @@ extern "C" int bte_expm(bte_ctx* ctx, int N, const double* A, double t, double* 
     const int sq = norm1 > theta13 ? (int)std::ceil(std::log2(norm1 / theta13)) : 0;
     DevBuf<double> X, A2, A4, A6, T, U, V;
     DevBuf<rocblas_int> piv, info;
-    X.upload(A, nn, s);
+    Staging st(c);
+    X.alloc(nn);
+    st.upload(X.p, A, nn * sizeof(double));
     A2.alloc(nn); A4.alloc(nn); A6.alloc(nn); T.alloc(nn); U.alloc(nn); V.alloc(nn);
     piv.alloc(N); info.alloc(1);
     const int gb = 4 * c->cu_count;
@@ -1060,6 +1066,7 @@ extern "C" int bte_expm(bte_ctx* ctx, int N, const double* A, double t, double* 
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));
     HIPCHECK(hipEventRecord(e0, s));
+    st.prefault(E, nn * sizeof(double));
     hipLaunchKernelGGL(ex_scale_kernel, dim3(gb), dim3(256), 0, s, X.p, std::ldexp(t, -sq), nn);
     rocblas_handle hb = (rocblas_handle)blas_handle(c);
     const double one = 1.0, zero = 0.0;
@@ -1091,7 +1098,7 @@ extern "C" int bte_expm(bte_ctx* ctx, int N, const double* A, double t, double* 
     }
     HIPCHECK(hipEventRecord(e1, s));
     rocblas_int inf = 0;
-    HIPCHECK(hipMemcpyAsync(E, cur, nn * sizeof(double), hipMemcpyDeviceToHost, s));
+    st.download(E, cur, nn * sizeof(double));
     HIPCHECK(hipMemcpyAsync(&inf, info.p, sizeof(inf), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     float el = 0;

@@ -1,6 +1,7 @@
 // Host-side runtime objects behind the C ABI handles.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <string>
@@ -74,6 +75,17 @@ struct DevBuf {
     }
 };
 
+// Pinned chunks of large copies (staging.hpp)
+struct StageChunks {
+    char* pin = nullptr;
+    std::vector<hipEvent_t> ev;  // one per chunk
+    std::atomic<bool> busy{false};
+    ~StageChunks() {
+        for (auto e : ev) (void)hipEventDestroy(e);
+        if (pin) (void)hipHostFree(pin);
+    }
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -82,6 +94,8 @@ struct Ctx {
     // BLAS handle kept for the context's lifetime (created on first use)
     void* blas = nullptr;
     void (*blas_free)(void*) = nullptr;
+    // made by the first large copy, kept for the context's lifetime
+    StageChunks chunks;
 };
 
 struct Modes {

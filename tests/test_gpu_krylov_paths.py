@@ -1,4 +1,7 @@
 """Routes of the Krylov build around the edges of its kernels."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -25,3 +28,45 @@ def test_small_exponentials(pkg, ctx, m, dt):
     d = np.abs(Pg - Po).max()
     print(f"m={m} dt={dt}: {d:.2e} of {np.abs(Po).max():.2e}", flush=True)
     assert d < 1e-10 * max(1.0, np.abs(Po).max())
+
+
+def _build(pkg, ctx, B, P, m):
+    dp = C.POINTER(C.c_double)
+    rep = pkg.KrylovReport()
+    pkg.check(pkg.lib().bte_krylov_build(ctx.h, len(B), C.cast(B.ctypes.data, dp), 0.5, m, pkg.PREC["bf16"], 1,
+                                         C.cast(P.ctypes.data, dp), C.byref(rep)))
+
+
+@pytest.mark.parametrize("n", [1447, 1449, 1536])
+def test_large_copies(pkg, ctx, n):
+    """Operators on both sides of 16 MB, above which pageable memory goes
+    through pinned chunks of 4 MB by two threads (N = 1449: the last chunk
+    holds 20 kB, N = 1536: half of it is used); pinned memory is copied the
+    plain way. The same bits arrive at an output that starts in the middle of a
+    page, its neighbours stay as they were, and two threads that share the
+    context get the same."""
+    hip = C.CDLL("libamdhip64.so.7")  # the one that the library has loaded
+
+    def pinned():
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), C.c_size_t(8 * n * n), 0) == 0
+        return p, np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), (n, n))
+
+    rng = np.random.default_rng(3)
+    B = rng.standard_normal((n, n)) / n
+    (hb, pb), (hp, pp) = pinned(), pinned()
+    pb[:] = B
+    _build(pkg, ctx, pb, pp, 3)
+    want = pp.copy()
+    assert hip.hipHostFree(hb) == 0 and hip.hipHostFree(hp) == 0
+    assert np.isfinite(want).all()
+    bufs = [np.full(n * n + 40, 7.0) for _ in range(2)]
+    out = [b[17:17 + n * n].reshape(n, n) for b in bufs]
+    th = [threading.Thread(target=_build, args=(pkg, ctx, B, o, 3)) for o in out]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for b, o in zip(bufs, out):
+        assert np.array_equal(o, want)
+        assert (b[:17] == 7.0).all() and (b[17 + n * n:] == 7.0).all()
