@@ -8,6 +8,7 @@
 //   evolparticle (transient)    990-1386  -> rta_fly(), rta_slow()
 //   history loop                2228-2317 -> rta_histories()
 //   post-processing             2326-2435 -> rta_postprocess()
+#include "flight_log.hpp"
 #include "runtime.hpp"
 #include <algorithm>
 #include <chrono>
@@ -49,8 +50,9 @@ struct RtaRunRows {
 // new mode costs one line (velocity, inverse velocity, rate and the range of
 // its diffuse-bounce table) instead of one line in each of three arrays.
 struct __align__(64) RtaMode {
-    double vx, vy, ivx, ivy, w;     // inverses are 0 where the component is 0
-    int32_t lo, len, base, pad[3];  // Lambert table: first partner, partners, offset
+    double vx, vy, ivx, ivy;       // inverses are 0 where the component is 0
+    double w, iw;                  // rate and 1 / w
+    int32_t lo, len, base, pad;    // Lambert table: first partner, partners, offset
 };
 static_assert(sizeof(RtaMode) == 64, "one mode record is half a 128-byte line");
 
@@ -125,8 +127,11 @@ struct RtaParams {
 #define RTA_NCOPY 8
 // the XCD (XCC) this wave runs on, from the hardware register HW_REG_XCC_ID
 
-// Boxes, polygon sides and the time grid of the history kernels: in LDS (GL)
-// when they take at most RTA_GEO_LDS bytes, else in global memory. Every
+static __device__ const LogEntry rta_log_table[FLIGHT_LOG_N] = FLIGHT_LOG_TABLE;
+
+// Boxes, polygon sides and the time grid of the history kernels: in LDS (GL),
+// behind the table of the flight logarithm, when they take at most
+// RTA_GEO_LDS bytes, else in global memory. Every
 // lane of a wave reads its own box, side and time bin, and such a scattered
 // load occupies the vector memory pipe for one cycle per lane: with the
 // geometry, the grid and the mode record read from global memory for every
@@ -142,16 +147,17 @@ struct RtaGeo {
     const unsigned char* box;
     const DevSide* side;
     const double* grid;
+    const LogEntry* log;
     int32_t bo;      // tally mode 3: first box of the run (staged indices are local)
     int32_t run;     // tally mode 3: the run of every lane, and its rate factor
-    double wscale;
+    double wscale, iws;  // and 1 / wscale
     __device__ inline RtaBox at(int i) const {
         return *reinterpret_cast<const RtaBox*>(box + (size_t)i * (GL ? RTA_BOX_LDS : sizeof(RtaBox)));
     }
 };
 
-// Copies nb boxes from bo on and ns sides from so on (with local indices) and
-// the time grid into LDS. The caller synchronises.
+// Copy nb boxes from bo on and ns sides from so on (with local indices), and
+// the time grid and the logarithm's table, into LDS. The caller synchronises.
 template <bool POLY>
 __device__ inline void rta_stage_boxes(const RtaParams& P, unsigned char* lds, int bo, int nb, int so, int ns, int lrow0) {
     for (int i = threadIdx.x; i < nb; i += blockDim.x) {
@@ -160,7 +166,7 @@ __device__ inline void rta_stage_boxes(const RtaParams& P, unsigned char* lds, i
             if (b.side_nbr[k] >= 0) b.side_nbr[k] -= bo;
         b.lrow -= lrow0;
         b.s0 -= so;
-        *reinterpret_cast<RtaBox*>(lds + (size_t)i * RTA_BOX_LDS) = b;
+        *reinterpret_cast<RtaBox*>(lds + FLIGHT_LOG_BYTES + (size_t)i * RTA_BOX_LDS) = b;
     }
     if constexpr (POLY) {
         DevSide* S = reinterpret_cast<DevSide*>(lds + P.geo_side);
@@ -172,6 +178,8 @@ __device__ inline void rta_stage_boxes(const RtaParams& P, unsigned char* lds, i
     }
 }
 __device__ inline void rta_stage_grid(const RtaParams& P, unsigned char* lds) {
+    LogEntry* t = reinterpret_cast<LogEntry*>(lds);
+    for (int i = threadIdx.x; i < FLIGHT_LOG_N; i += blockDim.x) t[i] = rta_log_table[i];
     double* g = reinterpret_cast<double*>(lds + P.geo_grid);
     for (int i = threadIdx.x; i <= P.nt; i += blockDim.x) g[i] = P.timegrid[i];
 }
@@ -263,7 +271,7 @@ struct RtaState {
     uint32_t sk, su, budget;
     int mode, box, still, bin, st, aux;  // aux: side (WALL) or side mask (MIXED)
     int run;                   // modes 0 to 2: the lane's run and its rate factor
-    double wscale;
+    double wscale, iws;        // and 1 / wscale
     int sign, ballistic, gmask;
     float score[4];
 };
@@ -433,6 +441,7 @@ __device__ inline void rta_start(const RtaGeo<GL>& G, RtaState& S, uint64_t pid)
     if (TM != 3) S.run = find_run(P, pid);
     const RtaRunDev& R = P.runs[TM == 3 ? G.run : S.run];
     S.wscale = R.wscale;
+    S.iws = 1.0 / S.wscale;
     S.rng.seed(R.seed, pid - R.first);
     S.ballistic = R.ballistic;
     S.gmask = R.gmask;
@@ -500,15 +509,21 @@ __device__ inline void rta_fly(const RtaParams& P, const RtaGeo<GL>& G, const Rt
         }
         const RtaMode* M = P.rmodes + S.mode;
         const double2 v = make_double2(M->vx, M->vy), iv = make_double2(M->ivx, M->ivy);
-        const double w = M->w;
+        const double w = M->w, iw = M->iw;
         const double u = 1.0 - S.rng.uniform();
         rta_look<TM>(P, G, S);
         S.vx = v.x;
         S.vy = v.y;
         S.ivx = iv.x;
         S.ivy = iv.y;
-        S.dtrem = -log(u) / (w * (TM == 3 ? G.wscale : S.wscale));
-        if (S.t + S.dtrem > P.maxtime) S.dtrem = P.maxtime - S.t + 1.0e-8;
+        // -log u / (w wscale): the quotient from the reciprocal, corrected by
+        // its remainder (Markstein), which rounds as the division does
+        const double a = -flight_log(G.log, u);
+        const double den = w * (TM == 3 ? G.wscale : S.wscale), rec = iw * (TM == 3 ? G.iws : S.iws);
+        const double q = a * rec;
+        S.dtrem = fma(fma(-q, den, a), rec, q);
+        // also where a rate whose reciprocal overflows has left no number
+        if (!(S.t + S.dtrem <= P.maxtime)) S.dtrem = P.maxtime - S.t + 1.0e-8;
         if (almost_equal(S.dtrem, 0.)) {
             S.still++;
             return;
@@ -765,7 +780,10 @@ __device__ inline void rta_mail_read(const RtaParams& P, const RtaGeo<GL>& G, co
         S.score[2] = __int_as_float(lo(w[11 * 64]));
         S.score[3] = __int_as_float(hi(w[11 * 64]));
     }
-    if (TM != 3) S.wscale = P.runs[S.run].wscale;
+    if (TM != 3) {
+        S.wscale = P.runs[S.run].wscale;
+        S.iws = 1.0 / S.wscale;
+    }
     // of the flight under way: the mode's velocity and the look-ahead
     const RtaMode* M = P.rmodes + S.mode;
     S.vx = M->vx;
@@ -951,7 +969,7 @@ struct RtaTake {
 
 // One launch follows the histories of all runs of a batch; ids of all runs
 // form one range, so a batch of runs of any sizes fills the GPU.
-// Bound by VALU issue while ids last (a pass is about 400 vector
+// Bound by VALU issue while ids last (a pass was about 400 vector
 // instructions, three waves per SIMD) and by the latency of a pass times the
 // passes of the longest history after that. 1 um x 200 nm, 100 bins, 200 time
 // bins, 3000 modes, 1e6 particles: 16.2 ms with geometry, grid and mode
@@ -959,7 +977,8 @@ struct RtaTake {
 // wave and segment; 15 of 64 lanes active), 10.7 ms with the geometry in LDS,
 // the mode in registers and the rare paths deferred, 7.0 ms with histories
 // changing waves, 6.2 ms with the exit test in selects, the segment's bins
-// found once and the rare paths' parameters read where they are used.
+// found once and the rare paths' parameters read where they are used, 5.65 ms
+// with the flight drawn by table and reciprocal (some 330 vector instructions).
 template <bool GRAD, int TMK, bool POLY, bool GL>
 __global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams P) {
     constexpr bool D = GRAD && TMK == 0;
@@ -969,10 +988,12 @@ __global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams 
     if constexpr (GL) {
         rta_stage_boxes<POLY>(P, rta_lds, 0, P.nboxes, 0, P.nsides, 0);
         rta_stage_grid(P, rta_lds);
-        G.box = rta_lds;
+        G.box = rta_lds + FLIGHT_LOG_BYTES;
+        G.log = reinterpret_cast<const LogEntry*>(rta_lds);
         G.side = reinterpret_cast<const DevSide*>(rta_lds + P.geo_side);
         G.grid = reinterpret_cast<const double*>(rta_lds + P.geo_grid);
     } else {
+        G.log = rta_log_table;
         G.box = reinterpret_cast<const unsigned char*>(P.rboxes);
         G.side = P.sides;
         G.grid = P.timegrid;
@@ -1019,8 +1040,8 @@ __global__ __launch_bounds__(TMK ? 768 : 512) void rta_history_kernel(RtaParams 
 // runs would not hold a single time bin.
 // The wait for the longest history (2900 passes against 160 on average for
 // 1 um over 5 ns) is paid once per run that a workgroup follows: 16 runs of
-// 3e4 to 1e6 particles take 17.3 ms, against 28.6 ms with the ids in items of
-// 4096 or more, each of which ended with that wait.
+// 3e4 to 1e6 particles took 17.3 ms (15.8 ms now, see flight_log.hpp), against 28.6 ms with the
+// ids in items of 4096 or more, each of which ended with that wait.
 
 // The run a workgroup turns to, by its first wave: the first_run entry, then
 // the run with the most particles left per workgroup on it, where those fill
@@ -1079,14 +1100,17 @@ __global__ __launch_bounds__(768) void rta_history_runs_kernel(RtaParams P) {
         G.bo = I.box0;
         G.run = run;
         G.wscale = P.runs[run].wscale;
+        G.iws = 1.0 / G.wscale;
         if constexpr (GL) {
             rta_stage_boxes<POLY>(P, rta_lds, I.box0, I.nbox, I.side0, I.nsides, (int)lrow0);
-            G.box = rta_lds;
+            G.box = rta_lds + FLIGHT_LOG_BYTES;
+            G.log = reinterpret_cast<const LogEntry*>(rta_lds);
             G.side = reinterpret_cast<const DevSide*>(rta_lds + P.geo_side);
             G.grid = reinterpret_cast<const double*>(rta_lds + P.geo_grid);
         } else {
             // global boxes keep the batch's indices
             G.bo = 0;
+            G.log = rta_log_table;
             G.box = reinterpret_cast<const unsigned char*>(P.rboxes);
             G.side = P.sides;
             G.grid = P.timegrid;
@@ -1398,7 +1422,9 @@ static RtaParams batch_params(RtaBatch* b, const RtaRunDev* runs, uint64_t total
 }
 
 // LDS of a workgroup of the history kernels: the geometry and the time grid
-// when they take at most RTA_GEO_LDS bytes (see RtaGeo), then the tallies.
+// when they take at most RTA_GEO_LDS bytes (see RtaGeo), then the tallies. (The
+// 2 KB of the logarithm's table beside such a geometry, at most 256 boxes,
+// never take a time bin's last room.)
 struct RtaLds {
     bool gl = false;
     int32_t side = 0, grid = 0, geo = 0;  // byte offsets: sides, grid, tallies
@@ -1409,9 +1435,9 @@ struct RtaLds {
 static RtaLds rta_lds_layout(int nboxes, int nsides, int nt) {
     RtaLds L;
     auto up16 = [](size_t v) { return (v + 15) & ~(size_t)15; };
-    const size_t side = (size_t)RTA_BOX_LDS * nboxes, grid = up16(side + sizeof(DevSide) * (size_t)nsides);
+    const size_t side = FLIGHT_LOG_BYTES + (size_t)RTA_BOX_LDS * nboxes, grid = up16(side + sizeof(DevSide) * (size_t)nsides);
     const size_t geo = up16(grid + sizeof(double) * ((size_t)nt + 1));
-    L.gl = geo <= RTA_GEO_LDS;
+    L.gl = geo <= FLIGHT_LOG_BYTES + RTA_GEO_LDS;
     if (L.gl) {
         L.side = (int32_t)side;
         L.grid = (int32_t)grid;
@@ -1708,7 +1734,7 @@ static void batch_create(RtaBatch* b) {
     std::vector<RtaMode> rm(n);
     for (int i = 0; i < n; i++)
         rm[i] = RtaMode{m->vx[i], m->vy[i], m->vx[i] != 0. ? 1.0 / m->vx[i] : 0., m->vy[i] != 0. ? 1.0 / m->vy[i] : 0.,
-                        m->w[i], info[i].x, info[i].y, info[i].z, {0, 0, 0}};
+                        m->w[i], 1.0 / m->w[i], info[i].x, info[i].y, info[i].z, 0};
     b->d_rmodes.upload(rm, s);
     b->d_lam_tab.upload(ltab, s);
     b->d_perm.upload(perm, s);

@@ -126,3 +126,23 @@ def test_runs_shared_among_workgroups(pkg, ctx, nruns):
         for g, r in zip(got, ref):
             _same(g, r)
     b.close()
+
+
+@pytest.mark.parametrize("tally", ["fp64", "fp64-lds-runs"])
+def test_modes_without_scattering(pkg, ctx, tally):
+    """A rate below the smallest normal number, whose reciprocal overflows,
+    draws flights longer than any run: they end at maxtime, as with a rate so
+    small that no flight ends before it. (Rates of 0 are refused.)"""
+    m = pkg.workloads.material(200, seed=3, mirror=True)
+    geom = _ribbon(pkg, ctx, 12)
+    out = []
+    for w in (1e-30, 1e-310):
+        modes = pkg.ModeTable(ctx, m["omega"], m["vx"], m["vy"], np.full(200, w), m["V"], m["lattz"])
+        b = pkg.RtaBatch(ctx, modes, [dict(geom=geom, T0=300.0, nparticles=5000, seed=2)], tally=tally, **KW)
+        (r,), rep = b.execute()
+        b.close()
+        out.append((r, rep["events"], rep["crossings"]))
+    assert out[0][2] > 5000
+    for r, ev, cr in out[1:]:
+        assert (ev, cr) == out[0][1:]
+        _same(r, out[0][0])
