@@ -73,8 +73,9 @@ struct BertParams {
     uint32_t* seg;           // [2][nsegs] live count per buffer segment
     unsigned long long* H;   // [2][nbox][n] particle counts: positive | negative << 32
     double* pbox;            // [nsegs][nbox][3] per-workgroup (sum h, sum h vx, sum h vy)
+    const double* pbox_prev; // of the step before
     uint32_t* tickets;       // [nbox][n]
-    int32_t* Eb;             // [2][nsd]
+    int32_t* Eb;             // [2 + 3][nsd] wall hits (see wall_emit)
     double* props;           // [steps+1][nbox][3]
     int64_t* npart;          // [steps+1]
     int64_t* pending;        // [steps+1] signed wall counts awaiting re-emission
@@ -824,12 +825,137 @@ __device__ inline int block_max_scan_256(int v, int* wmax) {
     return v;
 }
 
+// The wall counters of a step: the hits of its step and source kernels
+// (two rows, by parity) and those of the emission before it (three rows, so
+// that the step after next can clear a row that nothing reads).
+__device__ inline int32_t* wall_emit(const BertParams& P, uint32_t step) { return P.Eb + (size_t)(2 + step % 3) * P.nsd; }
+
+// The i-th of n workgroups, dispatched round-robin over 8 XCDs, takes item
+// start(x) + i / 8 on XCD x = i % 8: each XCD gets a contiguous range.
+__device__ inline int xcd_major_index(int i, int n) {
+    const int x = i & 7, j = i >> 3;
+    int start = 0;
+    for (int y = 0; y < x; y++) start += (n - y + 7) >> 3;
+    return start + j;
+}
+
+// What bert_props works on: a step's histogram and segment counts (halves
+// hist and seg), its box sums and the row of the results.
+struct BertPropsArgs {
+    int32_t row;         // results' row, -1: none
+    uint32_t step;       // the step after it (its emission's wall hits are that step's)
+    int32_t hist, seg;
+    int32_t cancel;      // the step cancels
+    int32_t from_boxes;  // sums from the box sums, else from the histogram
+    int32_t clear;       // clear its histogram (1) and the tickets (2)
+};
+
+// calculate_prop (beyondRTA_MC2d.cpp:1535-1602) of one box by a workgroup of
+// 256 from a step's box sums or histogram, the post-cancellation particle
+// count and the wall hits pending for the next step. The next step's kernel
+// has read the histogram and used the tickets by then: both are cleared for
+// their next use. lds: 10 KB.
+__device__ inline void bert_props(const BertParams& P, const BertPropsArgs& A, const double* pbox, int box, void* lds) {
+    const int row = A.row;
+    unsigned long long* H = P.H + (size_t)A.hist * P.nbox * P.n + (size_t)box * P.n;
+    double(*red)[256] = reinterpret_cast<double(*)[256]>(lds);                        // [3][256]
+    long long(*redc)[256] = reinterpret_cast<long long(*)[256]>((double*)lds + 768);  // [2][256]
+    double s = 0, fx = 0, fy = 0;
+    long long cnt = 0, acnt = 0;
+    if (!A.from_boxes || A.cancel || A.clear) {
+        for (int k = threadIdx.x; k < P.n; k += blockDim.x) {
+            if (!A.from_boxes || A.cancel) {
+                const int h = h_net(H[k]);
+                if (h != 0) {
+                    const double2 v = P.vel[k];
+                    s += h;
+                    fx += h * v.x;
+                    fy += h * v.y;
+                    cnt += h;
+                    acnt += h < 0 ? -h : h;
+                }
+            }
+            if (A.clear & 1) H[k] = 0;
+            if (A.clear & 2) P.tickets[(size_t)box * P.n + k] = 0;
+        }
+    }
+    if (A.from_boxes) {
+        // fixed summation order over the writing workgroups
+        s = fx = fy = 0.;
+        for (int g = threadIdx.x; g < P.nsegs; g += blockDim.x) {
+            const double* q = pbox + ((size_t)g * P.nbox + box) * 3;
+            s += q[0];
+            fx += q[1];
+            fy += q[2];
+        }
+    }
+    red[0][threadIdx.x] = s;
+    red[1][threadIdx.x] = fx;
+    red[2][threadIdx.x] = fy;
+    redc[0][threadIdx.x] = cnt;
+    redc[1][threadIdx.x] = acnt;
+    __syncthreads();
+    for (int d = 128; d > 0; d >>= 1) {
+        if (threadIdx.x < d) {
+            for (int q = 0; q < 3; q++) red[q][threadIdx.x] += red[q][threadIdx.x + d];
+            redc[0][threadIdx.x] += redc[0][threadIdx.x + d];
+            redc[1][threadIdx.x] += redc[1][threadIdx.x + d];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const DevBox B = P.boxes[box];
+        double vol = P.box_area[box] * P.thickness;
+        bool skip = B.kind != 0;
+        double* o = P.props + ((size_t)row * P.nbox + box) * 3;
+        o[0] = skip ? 0. : P.Eeff / vol * 1.0e27 * red[0][0];
+        o[1] = skip ? 0. : P.Eeff / vol * 1.0e30 * red[1][0];
+        o[2] = skip ? 0. : P.Eeff / vol * 1.0e30 * red[2][0];
+        // particles left after this step: sum |h| over regular boxes when
+        // the step cancels, else every particle written this step
+        if (A.cancel && !skip) atomicAdd((unsigned long long*)(P.npart + row), (unsigned long long)redc[1][0]);
+        const int2 sr = P.srange[box];
+        const int32_t* E = wall_emit(P, A.step) + sr.x;
+        long long pend = 0;
+        for (int k = 0; k < sr.y; k++) pend += E[k];
+        if (pend) atomicAdd((unsigned long long*)(P.pending + row), (unsigned long long)pend);
+    }
+    if (box == 0 && !A.cancel) {
+        // live particles written in the step
+        __syncthreads();
+        const uint32_t* segw = P.seg + (size_t)A.seg * P.nsegs;
+        long long c = 0;
+        for (int k = threadIdx.x; k < P.nsegs; k += blockDim.x) c += min(segw[k], P.segcap);
+        redc[0][threadIdx.x] = c;
+        __syncthreads();
+        for (int d = 128; d > 0; d >>= 1) {
+            if (threadIdx.x < d) redc[0][threadIdx.x] += redc[0][threadIdx.x + d];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) P.npart[row] = (int64_t)redc[0][0];
+    }
+}
+
+// The properties alone: of the initial particles and of the last step.
+__global__ __launch_bounds__(256) void bert_props_kernel(BertParams P, BertPropsArgs A) {
+    __shared__ double red[1280];
+    bert_props(P, A, P.pbox, xcd_major_index((int)blockIdx.x, (int)gridDim.x), red);
+}
+
 #define BERT_WCDF_PER 8
 // Adiabatic diffuse walls (beyondRTA_MC2d.cpp:281-435), phase 1: one
 // workgroup per (box, side) with a nonzero Eborder computes the border
 // temperature from the J(T) spline and the emission cumulative of
 // Isothermal_wall_distribution(Tborder, Teq, -n) (sampling.cpp:189-269).
-__global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_t step) {
+// The workgroups past the sides compute the properties of the step before
+// (A.row >= 0), one box each: both are short chains of dependent loads on a
+// few hundred workgroups, and as a launch of their own the properties took
+// 7 us of a step's 81 (1e6 particles in 50 boxes; 75 us now).
+// Workgroups go to the 8 XCDs round-robin; consecutive boxes are given to
+// workgroups on the same XCD, so the cache lines of pbox rows (a 128-B line
+// holds the sums of five neighbouring boxes) are fetched once into that XCD's
+// L2 instead of once per box.
+__global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_t step, BertPropsArgs A) {
     __shared__ double wtot[4];
     __shared__ int kcarry[4];
     // register path: the weight of every mode, then its guide key
@@ -837,6 +963,10 @@ __global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_
     __shared__ int skey[256 * BERT_WCDF_PER];
     __shared__ int grun[BERT_GUIDE];  // mode starting the run of keys at each guide entry, else 0
     const int b = blockIdx.x;  // side
+    if (b >= P.nsd) {
+        bert_props(P, A, P.pbox_prev, xcd_major_index(b - P.nsd, P.nbox), spm);
+        return;
+    }
     const int n = P.n;
     const bool regs = n <= 256 * BERT_WCDF_PER;
     // The kernel is a chain of dependent loads (side -> box -> spline ->
@@ -854,17 +984,21 @@ __global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_
     }
     const int box = P.side_box[b];
     int32_t* Eb = P.Eb + (size_t)(step & 1) * P.nsd;
-    const int E = Eb[b];
+    const int E = Eb[b] + wall_emit(P, step)[b];
     const int si = P.side_spl[b];
     if (E == 0 || si < 0) {
         if (threadIdx.x == 0) {
             P.wcount[b] = 0;
             Eb[b] = 0;
+            wall_emit(P, step + 2)[b] = 0;
         }
         return;
     }
     __syncthreads();
-    if (threadIdx.x == 0) Eb[b] = 0;
+    if (threadIdx.x == 0) {
+        Eb[b] = 0;
+        wall_emit(P, step + 2)[b] = 0;
+    }
     const DevSide sd = P.sides[b];
     const double Teq = P.box_Teq[box];
     const double* beq = P.beq + (size_t)P.box_beq[box] * n;
@@ -1059,7 +1193,7 @@ __global__ __launch_bounds__(VL ? 1024 : BERT_EMIT_THREADS) void bert_emit_kerne
         vtab = sv;
         ivtab = sv + P.n;
     }
-    int32_t* Eg = P.Eb + (size_t)((step + 1) & 1) * nb4;
+    int32_t* Eg = wall_emit(P, step + 1);
     eb_lds_begin(P, nb4);
     double* sbox = box_lds_begin(P);
     const uint32_t total = seg_prefix(P.wcount, nb4, 0xffffffffu, pre, tsum);  // ends with a barrier
@@ -1244,112 +1378,6 @@ __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const Be
     }
     seg_close(P, segout, myseg, &lcount, &ldone, done);
     box_lds_flush(P, myseg);
-}
-
-// The i-th of n workgroups, dispatched round-robin over 8 XCDs, takes item
-// start(x) + i / 8 on XCD x = i % 8: each XCD gets a contiguous range.
-__device__ inline int xcd_major_index(int i, int n) {
-    const int x = i & 7, j = i >> 3;
-    int start = 0;
-    for (int y = 0; y < x; y++) start += (n - y + 7) >> 3;
-    return start + j;
-}
-
-// calculate_prop (beyondRTA_MC2d.cpp:1535-1602) from the step's box sums
-// (from_boxes) or its histogram, the post-cancellation particle count, and
-// buffer recycling for the next step (clear_old: the previous step wrote its
-// histogram, which the step kernel has now consumed).
-__global__ __launch_bounds__(256) void bert_props_kernel(BertParams P, int row, int cur, int cancel_now,
-                                                         int clear_tickets, int ebn, int from_boxes,
-                                                         int clear_old) {
-    // Workgroups go to the 8 XCDs round-robin; consecutive boxes are given
-    // to workgroups on the same XCD, so the cache lines of pbox rows (a
-    // 128-B line holds the sums of five neighbouring boxes) are fetched
-    // once into that XCD's L2 instead of once per box.
-    const int box = xcd_major_index((int)blockIdx.x, (int)gridDim.x);
-    const unsigned long long* H = P.H + (size_t)cur * P.nbox * P.n + (size_t)box * P.n;
-    unsigned long long* Hold = P.H + (size_t)(cur ^ 1) * P.nbox * P.n + (size_t)box * P.n;
-    __shared__ double red[3][256];
-    __shared__ long long redc[2][256];
-    double s = 0, fx = 0, fy = 0;
-    long long cnt = 0, acnt = 0;
-    if (!from_boxes || cancel_now || clear_old || clear_tickets) {
-        for (int k = threadIdx.x; k < P.n; k += blockDim.x) {
-            if (!from_boxes || cancel_now) {
-                const int h = h_net(H[k]);
-                if (h != 0) {
-                    const double2 v = P.vel[k];
-                    s += h;
-                    fx += h * v.x;
-                    fy += h * v.y;
-                    cnt += h;
-                    acnt += h < 0 ? -h : h;
-                }
-            }
-            if (clear_old) Hold[k] = 0;
-            if (clear_tickets) P.tickets[(size_t)box * P.n + k] = 0;
-        }
-    }
-    if (from_boxes) {
-        // fixed summation order over the writing workgroups
-        s = fx = fy = 0.;
-        for (int g = threadIdx.x; g < P.nsegs; g += blockDim.x) {
-            const double* q = P.pbox + ((size_t)g * P.nbox + box) * 3;
-            s += q[0];
-            fx += q[1];
-            fy += q[2];
-        }
-    }
-    red[0][threadIdx.x] = s;
-    red[1][threadIdx.x] = fx;
-    red[2][threadIdx.x] = fy;
-    redc[0][threadIdx.x] = cnt;
-    redc[1][threadIdx.x] = acnt;
-    __syncthreads();
-    for (int d = 128; d > 0; d >>= 1) {
-        if (threadIdx.x < d) {
-            for (int q = 0; q < 3; q++) red[q][threadIdx.x] += red[q][threadIdx.x + d];
-            redc[0][threadIdx.x] += redc[0][threadIdx.x + d];
-            redc[1][threadIdx.x] += redc[1][threadIdx.x + d];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const DevBox B = P.boxes[box];
-        double vol = P.box_area[box] * P.thickness;
-        bool skip = B.kind != 0;
-        double* o = P.props + ((size_t)row * P.nbox + box) * 3;
-        o[0] = skip ? 0. : P.Eeff / vol * 1.0e27 * red[0][0];
-        o[1] = skip ? 0. : P.Eeff / vol * 1.0e30 * red[1][0];
-        o[2] = skip ? 0. : P.Eeff / vol * 1.0e30 * red[2][0];
-        // particles left after this step: sum |h| over regular boxes when
-        // the step cancels, else every particle written this step
-        if (cancel_now && !skip)
-            atomicAdd((unsigned long long*)(P.npart + row), (unsigned long long)redc[1][0]);
-        const int2 sr = P.srange[box];
-        const int32_t* E = P.Eb + (size_t)ebn * P.nsd + sr.x;
-        long long pend = 0;
-        for (int k = 0; k < sr.y; k++) pend += E[k];
-        if (pend) atomicAdd((unsigned long long*)(P.pending + row), (unsigned long long)pend);
-    }
-    if (box == 0) {
-        // live particles written this step; recycle the input counters
-        __syncthreads();
-        uint32_t* segin = P.seg + (size_t)cur * P.nsegs;
-        const uint32_t* segw = P.seg + (size_t)(cur ^ 1) * P.nsegs;
-        long long c = 0;
-        for (int k = threadIdx.x; k < P.nsegs; k += blockDim.x) {
-            c += min(segw[k], P.segcap);
-            segin[k] = 0;
-        }
-        redc[0][threadIdx.x] = c;
-        __syncthreads();
-        for (int d = 128; d > 0; d >>= 1) {
-            if (threadIdx.x < d) redc[0][threadIdx.x] += redc[0][threadIdx.x + d];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0 && !cancel_now) P.npart[row] = (int64_t)redc[0][0];
-    }
 }
 
 // initial particles: histogram into H[cur] (properties row 0)
@@ -2059,8 +2087,8 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     b->d_stats.alloc((size_t)b->nsegs);
     b->d_H.alloc((size_t)2 * nbox * n);
     b->d_tickets.alloc((size_t)nbox * n);
-    if (nbox <= BERT_LDS_BOXES) b->d_pbox.alloc((size_t)b->nsegs * nbox * 3);
-    b->d_Eb.alloc((size_t)2 * g->sides.size());
+    if (nbox <= BERT_LDS_BOXES) b->d_pbox.alloc((size_t)2 * b->nsegs * nbox * 3);
+    b->d_Eb.alloc((size_t)5 * g->sides.size());
     b->d_props.alloc((size_t)(b->max_steps + 1) * nbox * 3);
     b->d_npart.alloc((size_t)(b->max_steps + 1));
     b->d_pending.alloc((size_t)(b->max_steps + 1));
@@ -2236,7 +2264,7 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
     BPart* buf[2] = {b->d_parts.p, b->d_parts.p + b->cap};
     HIPCHECK(hipMemsetAsync(b->d_H.p, 0, (size_t)2 * nbox * n * sizeof(unsigned long long), s));
     HIPCHECK(hipMemsetAsync(b->d_tickets.p, 0, (size_t)nbox * n * sizeof(uint32_t), s));
-    HIPCHECK(hipMemsetAsync(b->d_Eb.p, 0, (size_t)2 * b->g->sides.size() * sizeof(int32_t), s));
+    HIPCHECK(hipMemsetAsync(b->d_Eb.p, 0, (size_t)5 * b->g->sides.size() * sizeof(int32_t), s));
     HIPCHECK(hipMemsetAsync(b->d_flags.p, 0, 4 * sizeof(uint32_t), s));
     HIPCHECK(hipMemsetAsync(b->d_stats.p, 0, (size_t)b->nsegs * sizeof(unsigned long long), s));
     HIPCHECK(hipMemsetAsync(b->d_npart.p, 0, (size_t)(b->max_steps + 1) * sizeof(int64_t), s));
@@ -2255,13 +2283,9 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
     // row 0: properties of the initial particles
     hipLaunchKernelGGL(bert_hist_kernel, dim3(c->cu_count * 4), dim3(256), 0, s, P, 0);
     HIPCHECK(hipGetLastError());
-    // props of H[0] into row 0; the kernel clears H[1] and the input segment
-    // counters; restore them afterwards because the initial particles are
-    // the first step's input
-    hipLaunchKernelGGL(bert_props_kernel, dim3(nbox), dim3(256), 0, s, P, 0, 0, 0, 0, 0, 0, 1);
+    // their properties into row 0; H[0] is clear again afterwards
+    hipLaunchKernelGGL(bert_props_kernel, dim3(nbox), dim3(256), 0, s, P, BertPropsArgs{0, 0u, 0, 0, 0, 0, 1});
     HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(b->d_seg.p, c0.data(), c0.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    HIPCHECK(hipMemsetAsync(b->d_H.p, 0, (size_t)nbox * n * sizeof(unsigned long long), s));
     HIPCHECK(hipMemcpyAsync(b->d_npart.p, &b->n0, sizeof(int64_t), hipMemcpyHostToDevice, s));
     HIPCHECK(hipStreamSynchronize(s));
     const int step_blocks = b->step_blocks;
@@ -2282,11 +2306,19 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
     auto t0 = std::chrono::steady_clock::now();
     HIPCHECK(hipEventRecord(b->ev0, s));
     int istep = 0;
-    int prev_hist = 0;
+    // a step's properties are computed beside the next step's wall
+    // distributions, those of the last one after the loop
+    BertPropsArgs props_of{-1, 0u, 0, 0, 0, 0, 0};
+    const unsigned nsd = (unsigned)b->g->sides.size();
+    const size_t pbox_half = (size_t)b->nsegs * nbox * 3;
     for (; istep < b->max_steps; istep++) {
         const int cur = istep & 1;
         P.pin = buf[cur];
         P.pout = buf[cur ^ 1];
+        if (P.lds_props) {
+            P.pbox = b->d_pbox.p + cur * pbox_half;
+            P.pbox_prev = b->d_pbox.p + (cur ^ 1) * pbox_half;
+        }
         const int cancel_prev = istep > 0 && ((istep - 1) % pc == 0);
         const int cancel_now = (istep % pc == 0);
         // the (box, mode) histogram is built only where a cancellation or a
@@ -2305,18 +2337,18 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
                                dim3(b->src_blocks),
                                dim3(256), b->lds_bytes, s, P, b->d_src.p, b->nsrc, b->d_src_tab.p, (uint32_t)istep,
                                cur, hist);
-        hipLaunchKernelGGL(bert_wallcdf_kernel, dim3((unsigned)b->g->sides.size()), dim3(256), 0, s, P, (uint32_t)istep);
+        hipLaunchKernelGGL(bert_wallcdf_kernel, dim3(nsd + (props_of.row >= 0 ? (unsigned)nbox : 0u)), dim3(256), 0, s, P,
+                           (uint32_t)istep, props_of);
         hipLaunchKernelGGL(emit_k, dim3(emit_blocks), dim3(b->vl ? 1024 : BERT_EMIT_THREADS),
                            b->vl ? b->lds_vl_bytes : b->lds_bytes, s, P, (uint32_t)istep, cur, hist);
-        // H of this step lives in H[cur]; H[cur^1] (previous step) is cleared
-        // after the step kernel used it for cancellation
-        hipLaunchKernelGGL(bert_props_kernel, dim3(nbox), dim3(256), 0, s, P, istep + 1, cur, cancel_now,
-                           cancel_now, (istep + 1) & 1, P.lds_props, prev_hist);
-        prev_hist = hist;
+        // H of this step lives in H[cur] until the next step's kernel has used
+        // it for the cancellation, its segments in seg[cur ^ 1]
+        props_of = BertPropsArgs{istep + 1, (uint32_t)istep + 1u, cur, cur ^ 1, cancel_now, P.lds_props,
+                                 (hist ? 1 : 0) | (cancel_now ? 2 : 0)};
         HIPCHECK(hipGetLastError());
         if (cb) {
             // the histogram of this step is in H[cur] until the next step's
-            // props kernel clears it
+            // wall kernel clears it
             HIPCHECK(hipMemcpyAsync(b->hH64.data(), b->d_H.p + (size_t)cur * nbox * n,
                                     (size_t)nbox * n * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
             HIPCHECK(hipStreamSynchronize(s));
@@ -2327,6 +2359,10 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
                 break;
             }
         }
+    }
+    if (props_of.row >= 0) {
+        hipLaunchKernelGGL(bert_props_kernel, dim3(nbox), dim3(256), 0, s, P, props_of);
+        HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipEventRecord(b->ev1, s));
     HIPCHECK(hipStreamSynchronize(s));

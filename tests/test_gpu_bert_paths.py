@@ -73,3 +73,47 @@ def test_periodic_tables_in_lds_and_in_global_memory(pkg, ctx, nb, extra):
     assert np.array_equal(a["npart"], c["npart"]) and a["npart"][-1] > 1000
     scale = np.abs(a["props"]).max(axis=(0, 1))
     np.testing.assert_allclose(c["props"][:, :nb] / scale, a["props"][:, :nb] / scale, rtol=0, atol=1e-10)
+
+
+@pytest.mark.parametrize("pc", [1, 2, 4])
+@pytest.mark.parametrize("steps", [1, 2, 9])
+def test_properties_of_each_step(pkg, ctx, pc, steps):
+    """A step's properties, particle count and pending wall hits are taken
+    while the next step runs (the last step's afterwards), from box sums or,
+    where it cancels, the histogram. The frames of a second run hold that
+    histogram after each step: its net sum times the energy per particle and
+    volume is the first property, and its net counts those left where the
+    step cancels. A third run, which its callback stops, has the same rows up
+    to there."""
+    W = pkg.workloads
+    mat = W.material(60, seed=5)
+    rect, kind, teq, _ = W.ribbon(60.0, 5.0, 6, 300.0, reservoirs=(302.0, 300.0))  # narrow: emitted particles reach the other side
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    geom = pkg.Geometry(ctx, rect, kind, teq)
+    kw = dict(thickness=1.0, dt=4.0, maxtime=4.0 * (steps - 1), max_steps=steps, rta=True, Efactor=4000, Tmax=302.0,
+              Tmin=300.0, seed=3, pcancel_each=pc)
+
+    def run(cb=None):
+        b = pkg.BertRun(ctx, modes, geom, None, **kw)
+        r = b.execute() if cb is None else b.execute(cb)
+        b.close()
+        return r
+
+    frames = []
+    a = run()
+    c = run(lambda s, t, e, H: frames.append((e, H)) and False)
+    assert len(frames) == steps == len(a["npart"]) - 1
+    for key in ("npart", "pending"):
+        assert np.array_equal(a[key], c[key]), key
+    np.testing.assert_allclose(a["props"], c["props"], rtol=1e-10, atol=1e-10 * np.abs(a["props"]).max())
+    area = (rect[:, 1] - rect[:, 0]) * (rect[:, 3] - rect[:, 2])
+    reg = np.asarray(kind) == 0
+    assert a["npart"][-1] > 0 and (steps < 9 or a["pending"][1:].any())
+    for s, (e, H) in enumerate(frames):
+        want = e / area * 1.0e27 * H.sum(1)
+        np.testing.assert_allclose(a["props"][s + 1, reg, 0], want[reg], rtol=1e-12, atol=0)
+        if s % pc == 0:
+            assert a["npart"][s + 1] == np.abs(H[reg]).sum()
+    stop = run(lambda s, t, e, H: s == steps // 2)
+    assert np.array_equal(stop["npart"][:steps // 2 + 2], a["npart"][:steps // 2 + 2])
+    assert np.array_equal(stop["pending"][:steps // 2 + 2], a["pending"][:steps // 2 + 2])
