@@ -146,3 +146,31 @@ def test_modes_without_scattering(pkg, ctx, tally):
     for r, ev, cr in out[1:]:
         assert (ev, cr) == out[0][1:]
         _same(r, out[0][0])
+
+
+# events and crossings with the tables made on the host, one mode after the other
+@pytest.mark.parametrize("n,sigma,own,want", [(300, 2.0, False, (60479, 21616)), (300, 2.0, True, (61429, 22044)),
+                                              (2200, 1e3, False, (68168, 24881))])
+def test_lambert_tables(pkg, ctx, n, sigma, own, want):
+    """The diffuse-bounce tables of every mode and side normal, with one width
+    or one per mode; windows of all 2200 modes make more entries than one pass takes."""
+    m = pkg.workloads.material(n, seed=5)
+    rect, kind, teq, _ = pkg.workloads.ribbon(60.0, 5.0, 6, 300.0, reservoirs=(302.0, 300.0))
+    modes = pkg.ModeTable(ctx, m["omega"], m["vx"], m["vy"], m["w"], m["V"], m["lattz"])
+    if own:
+        modes.set_sigma(np.random.default_rng(1).uniform(0.5, 3.0, n))
+    b = pkg.RtaBatch(ctx, modes, [dict(geom=pkg.Geometry(ctx, rect, kind, teq), T0=300.0, nparticles=4000, seed=2)],
+                     thickness=1.0, dt=10.0, maxtime=400.0, sigma_bounce=sigma)
+    _, rep = b.execute()
+    b.close()
+    assert (rep["events"], rep["crossings"]) == want
+
+
+def test_lambert_window_without_partner(pkg, ctx):
+    """A width so small that a mode's window holds the mode alone: the first
+    one that can reach a side is named."""
+    m = pkg.workloads.material(200, seed=5)
+    modes = pkg.ModeTable(ctx, m["omega"], m["vx"], m["vy"], m["w"], m["V"], m["lattz"])
+    with pytest.raises(pkg.BteError, match="mode 0 has no diffuse partner within the Lambert window"):
+        pkg.RtaBatch(ctx, modes, [dict(geom=_ribbon(pkg, ctx, 6), T0=300.0, nparticles=100, seed=2)],
+                     **dict(KW, sigma_bounce=1e-9))
