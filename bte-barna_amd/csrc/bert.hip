@@ -11,11 +11,13 @@
 //   bert_wallcdf_kernel adiabatic_diffuse_walls (281-435), part 1: per box
 //                      side the border temperature from the J(T) spline and
 //                      the emission cumulative distribution
+//                      of step s, and in workgroups of its own calculate_prop
+//                      (1535-1602) of every box and the post-cancel particle
+//                      count of step s-1 (those of the last step by
+//                      bert_props_kernel)
 //   bert_emit_kernel   part 2: all |Eborder| re-emissions as one balanced
 //                      index space: placed, advected U*dt, scattered,
 //                      histogrammed
-//   bert_props_kernel  calculate_prop (1535-1602) for every box, post-cancel
-//                      particle count, buffer recycling
 // Particle state is 32 bytes (x, y f64; mode; box|sign; 64-bit id). The
 // random stream of a particle in a step is PCG32 seeded from (seed, id,
 // step), so a particle's fate does not depend on where it sits in the buffer.
@@ -301,7 +303,7 @@ __device__ inline int advect_cross(const BertParams& P, const BertBoxes<GL>& box
 // runs once for all of them.
 // With the exit test in selects, the boxes at a conflict-free stride and the
 // rare cases' parameters out of the loop's scalar registers (95 instead of 165
-// lane reads of spilled ones in the kernel) the step kernel takes 144.6 us
+// lane reads of spilled ones in the kernel) the step kernel takes 140 us
 // instead of 152 at 3.3e6 particle-steps.
 // PER compiles in the periodic translation; without periodic boxes the
 // kernels use the instantiation without it, which needs fewer registers per
