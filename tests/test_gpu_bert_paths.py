@@ -117,3 +117,30 @@ def test_properties_of_each_step(pkg, ctx, pc, steps):
     stop = run(lambda s, t, e, H: s == steps // 2)
     assert np.array_equal(stop["npart"][:steps // 2 + 2], a["npart"][:steps // 2 + 2])
     assert np.array_equal(stop["pending"][:steps // 2 + 2], a["pending"][:steps // 2 + 2])
+
+
+@pytest.mark.parametrize("nb", [1, 3, 8, 33])
+def test_wall_workgroups_cover_every_side(pkg, ctx, nb):
+    """Sides are dealt to the wall workgroups by fours, in polygon geometries
+    of 4 nb + 3 sides (one box a triangle, so that their number is no multiple
+    of four) as in nb + 1 rectangles: with adiabatic walls all around, every
+    particle that hits one comes out of it again, none is lost over the run."""
+    W = pkg.workloads
+    mat = W.material(60, seed=5)
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    for tri in (False, True):
+        rect = np.array([[k * 10.0, (k + 1) * 10.0, 0.0, 12.0] for k in range(nb + 1)])
+        polys = [np.array([[r[0], r[2]], [r[1], r[2]], [r[1], r[3]], [r[0], r[3]]]) for r in rect]
+        if tri:
+            x = nb * 10.0
+            polys[nb] = np.array([[x, 0.0], [x + 9.0, 6.0], [x, 12.0]])
+        teq = np.full(nb + 1, 300.0)
+        tin = teq.copy()
+        tin[0] = 304.0
+        geom = pkg.Geometry(ctx, rect, np.zeros(nb + 1, np.int32), teq, tin, polys=polys if tri else None)
+        b = pkg.BertRun(ctx, modes, geom, None, thickness=1.0, dt=4.0, maxtime=36.0, max_steps=10, rta=True,
+                        Efactor=20000, Tmax=304.0, Tmin=300.0, seed=3)
+        r = b.execute()
+        b.close()
+        assert r["npart"][0] > 5000
+        assert (r["npart"] + r["pending"] == r["npart"][0]).all(), (tri, r["npart"], r["pending"])
