@@ -335,11 +335,12 @@ typedef struct {
     uint64_t step_kernel_particle_steps; /* the part done by the main step kernel */
     int64_t max_particles;
     double loop_ms;           /* wall time of the step loop (device-synchronised) */
-    double step_kernel_ms;    /* device time of the timed step-kernel launches, summed */
+    double step_kernel_ms;    /* step_kernel_timed times their mean device time (each place of the
+                               * cancellation cycle with the same weight) */
     int step_kernel_launches;
-    /* launches bracketed by events: one in pcancel_each, rotating through
-     * the cancellation cycle so every step type is sampled equally (an
-     * event pair costs about 11 us of idle device time per step) */
+    /* launches bracketed by events: one in every fourth cancellation cycle
+     * (of pcancel_each steps), at each place of the cycle in turn (an event
+     * pair costs about 11 us of idle device time) */
     int step_kernel_timed;
     int step_threads;         /* threads per step-kernel workgroup: 1024 with the
                                  mode velocities in LDS, else 256 */
