@@ -22,6 +22,7 @@
 // random stream of a particle in a step is PCG32 seeded from (seed, id,
 // step), so a particle's fate does not depend on where it sits in the buffer.
 #include "runtime.hpp"
+#include "wall_hits.hpp"
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -993,21 +994,12 @@ __global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_
         }
     }
     const int box = P.side_box[b];
-    int32_t* Eb = P.Eb + (size_t)(step & 1) * P.nsd;
-    const int E = Eb[b] + wall_emit(P, step)[b];
     const int si = P.side_spl[b];
-    if (E == 0 || si < 0) {
-        if (threadIdx.x == 0) {
-            P.wcount[b] = 0;
-            Eb[b] = 0;
-            wall_emit(P, step + 2)[b] = 0;
-        }
+    const int E = take_wall_hits(P.Eb + (size_t)(step & 1) * P.nsd + b, wall_emit(P, step) + b,
+                                 wall_emit(P, step + 2) + b, threadIdx.x == 0, [] { __syncthreads(); });
+    if (E == 0 || si < 0) {  // uniform over the workgroup
+        if (threadIdx.x == 0) P.wcount[b] = 0;
         return;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        Eb[b] = 0;
-        wall_emit(P, step + 2)[b] = 0;
     }
     const DevSide sd = P.sides[b];
     const double Teq = P.box_Teq[box];

@@ -144,3 +144,28 @@ def test_wall_workgroups_cover_every_side(pkg, ctx, nb):
         b.close()
         assert r["npart"][0] > 5000
         assert (r["npart"] + r["pending"] == r["npart"][0]).all(), (tri, r["npart"], r["pending"])
+
+
+@pytest.mark.parametrize("nb,seed", [(2, 1), (6, 1), (6, 2)])
+def test_wall_hits_that_cancel(pkg, ctx, nb, seed):
+    """Few particles of both signs between adiabatic walls 5 nm apart: the
+    hits of a side from the step and from the emission before often cancel.
+    Every step keeps the signed particle count: those in the boxes (the first
+    property is their net count times the energy per particle and volume) and
+    the hits that wait for their emission."""
+    W = pkg.workloads
+    mat = W.material(60, seed=5)
+    L = 10.0
+    rect = np.array([[k * L, (k + 1) * L, r * 8.0, r * 8.0 + 5.0] for r in range(2) for k in range(nb)])
+    teq = np.full(2 * nb, 300.0)
+    tin = np.repeat([303.0, 297.0], nb)
+    tin[1::2] = 600.0 - tin[1::2]  # hot and cold boxes in turn, opposite in the second row
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    geom = pkg.Geometry(ctx, rect, np.zeros(2 * nb, np.int32), teq, tin)
+    b = pkg.BertRun(ctx, modes, geom, None, thickness=1.0, dt=4.0, maxtime=4.0 * 399, max_steps=400, rta=True,
+                    Efactor=40, Tmax=303.0, Tmin=297.0, seed=seed, pcancel_each=1000)
+    r = b.execute()
+    b.close()
+    net = r["props"][:, :, 0].sum(1) * (L * 5.0) / (r["Eeff"] * 1.0e27) + r["pending"]
+    assert r["npart"][0] > 20 and r["pending"].any()
+    np.testing.assert_allclose(net, round(net[0]), rtol=0, atol=1e-6)
