@@ -1290,8 +1290,17 @@ struct BertSource {
     int32_t area, pad;
 };
 #define BERT_SRC_BLOCKS 256
-// particles per step and part: one round of a workgroup's 256 threads
+// Expected particles per step and part (a source above 256 parts takes 256
+// larger ones): one round of a workgroup's 256 threads, or four rounds where
+// buffer segments are scarce. Each part up to BERT_SRC_BLOCKS gets a workgroup
+// and a segment, and all segments have the same size, so up to 256 more of them
+// shrink the step workgroups' segments in a capacity that the caller gave, and
+// enlarge the buffers that are sized for many initial particles (more than
+// BERT_STEADY / 2), beside whose step kernel the source kernel's time is small.
 #define BERT_SRC_PART 256.0
+#define BERT_SRC_PART_WIDE 1024.0
+// population that the automatic buffers hold with sources: 0.7 x 2^25
+#define BERT_STEADY ((uint64_t)(0.7 * (1ull << 25)))
 template <bool GL, bool PER, bool POLY>
 __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const BertSource* src, int nparts_all,
                                                           const uint2* stab, uint32_t step, int cur, int hist) {
@@ -1937,8 +1946,11 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     b->n0 = total;
     b->ninit = (int)inits.size();
     // one buffer segment per writing workgroup: step, emission, sources
-    // reservoir sources (Isothermal_walls): expected particles per step,
-    // split into parts of at most 256 particles each
+    // reservoir sources (Isothermal_walls): expected particles per step, split into parts
+    const double src_part = cfg->capacity || 2 * total > BERT_STEADY ? BERT_SRC_PART_WIDE : BERT_SRC_PART;
+    const auto source_parts = [src_part](double expected) {
+        return (int)std::min(256.0, std::max(1.0, std::ceil(expected / src_part)));
+    };
     std::vector<BertSource> srcs;
     std::vector<uint2> stab;
     double src_total = 0;
@@ -1952,7 +1964,7 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
             double spf = hc.length() * cfg->thickness / vuc;
             build_alias(pmf.data(), n, th.data(), al.data());
             const double expected = cfg->dt * spf * cum / (b->Eeff * m->nq);
-            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / BERT_SRC_PART)));
+            const int nparts = source_parts(expected);
             const int src = (int)(stab.size() / n);
             for (int part = 0; part < nparts; part++)
                 srcs.push_back(BertSource{hc.p1x, hc.p1y, hc.p2x - hc.p1x, hc.p2y - hc.p1y, expected, hc.box,
@@ -1994,7 +2006,7 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
             const double cumulsum = kB * acc;
             build_alias(pmf.data(), n, th.data(), al.data());
             const double expected = cfg->dt * (bx.area() * cfg->thickness / vuc) * cumulsum / (b->Eeff * m->nq);
-            const int nparts = (int)std::min(256.0, std::max(1.0, std::ceil(expected / BERT_SRC_PART)));
+            const int nparts = source_parts(expected);
             const int src = (int)(stab.size() / n);
             for (int part = 0; part < nparts; part++)
                 srcs.push_back(BertSource{bx.xmin, bx.ymin, bx.xmax - bx.xmin, bx.ymax - bx.ymin, expected, i, 1,
@@ -2064,8 +2076,8 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
         src_wg_max = std::max(src_wg_max, e);
     }
     // (every step workgroup's segment takes twice its share of the initial
-    // particles; with sources, its share of a steady population of 0.7 x 2^25)
-    const uint64_t seg_step = std::max<uint64_t>(2 * total, src_total > 0 ? (uint64_t)(0.7 * (1ull << 25)) : 0ull) /
+    // particles; with sources, its share of a steady population of BERT_STEADY)
+    const uint64_t seg_step = std::max<uint64_t>(2 * total, src_total > 0 ? BERT_STEADY : 0ull) /
                                   (uint64_t)b->step_blocks + 4096;
     b->cap = cfg->capacity ? cfg->capacity
                            : std::max<uint64_t>({1ull << 22, 3 * total, src_total > 0 ? (1ull << 25) : 0ull,

@@ -295,7 +295,9 @@ typedef struct {
     int rta;           /* <RTA/> */
     int pcancel_each;  /* cancellation period (4 in the reference) */
     uint64_t seed;
-    uint64_t capacity; /* particle buffer capacity; 0 = automatic */
+    uint64_t capacity; /* particle buffer capacity, in equal segments per writing workgroup
+                        * (sources: one per 1024 expected particles per step, one at least and
+                        * 256 at most); 0 = automatic */
     /* gradient sources (source_term_gradient, beyondRTA_MC2d.cpp:597-676):
      * 0 = per-box gradients from calculate_gradientT (the default),
      * 1 = <gradient x y> [K/nm] in every regular box */

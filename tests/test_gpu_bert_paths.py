@@ -169,3 +169,32 @@ def test_wall_hits_that_cancel(pkg, ctx, nb, seed):
     net = r["props"][:, :, 0].sum(1) * (L * 5.0) / (r["Eeff"] * 1.0e27) + r["pending"]
     assert r["npart"][0] > 20 and r["pending"].any()
     np.testing.assert_allclose(net, round(net[0]), rtol=0, atol=1e-6)
+
+
+def test_a_given_capacity_holds_with_a_large_source(pkg, ctx):
+    """A source of about 1e5 particles per step beside 2e6 initial ones, in a
+    given capacity: with a source segment for every 1024 particles (98 beside
+    256 of the step kernel and 256 of the emission) a segment of 0.95 of the
+    step workgroups' share of the initial particles is enough, as 15 percent
+    of them leave or wait at a wall in the first step; with one for every 256
+    (256 at most) it would be 0.75. The histories are those of the automatic
+    capacity."""
+    W = pkg.workloads
+    mat = W.material(60, seed=5)
+    rect, kind, teq, _ = W.ribbon(100.0, 200.0, 5, 300.0, reservoirs=(302.0, 300.0))
+    tin = np.where(np.asarray(kind) == 0, 302.0, teq)
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    geom = pkg.Geometry(ctx, rect, kind, teq, tin)
+
+    def run(**kw):
+        b = pkg.BertRun(ctx, modes, geom, None, thickness=1.0, dt=4.0, maxtime=8.0, rta=True, Efactor=400000,
+                        Tmax=302.0, Tmin=300.0, seed=3, pcancel_each=1000, **kw)
+        r = b.execute()
+        b.close()
+        return r
+
+    a = run()
+    n0 = int(a["npart"][0])
+    assert n0 > 1900000 and a["npart"].max() == n0 and a["step_threads"] == 1024
+    c = run(capacity=int(0.95 * n0 / 256 * (256 + 256 + 98)))
+    assert np.array_equal(a["npart"], c["npart"]) and np.array_equal(a["pending"], c["pending"])
