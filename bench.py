@@ -472,8 +472,9 @@ def main():
     log(f"timed {args.steps} runs in {elapsed:.3f} s")
     events = sum(o["particle_steps"] for o in outs)
     value = events / elapsed
-    # HIP events bracket one step-kernel launch in four (every step type of
-    # the cancellation cycle equally); the bytes are averaged over all
+    # HIP events bracket one step-kernel launch in 16 (one in every fourth
+    # cancellation cycle, each step type in turn, of equal weight in the
+    # mean); the bytes are averaged over all
     k_ms = sum(o["step_kernel_ms"] for o in outs)
     k_timed = sum(o["step_kernel_timed"] for o in outs)
     k_launch = sum(o["step_kernel_launches"] for o in outs)

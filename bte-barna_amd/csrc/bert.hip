@@ -2266,13 +2266,15 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
 }
 
 // The launches of the step kernel that carry an event pair: one in every
-// fourth cancellation cycle, at each place of the cycle in turn. A record
+// `every`-th cancellation cycle, at each place of the cycle in turn. A record
 // between two kernels leaves the device idle for about 5.6 us on both sides:
 // with one in every cycle, 80 steps of a periodic bar took 3.80 ms and 100 steps of
-// 1e6 particles 7.49 ms, now 3.71 and 7.38 ms.
-static bool timed_step(int istep, int pc) {
+// 1e6 particles 7.49 ms, with one in every fourth 3.71 and 7.38 ms. A run whose
+// cycles would not reach every place that way has them closer together.
+static int timed_every(int steps, int pc) { return std::min(4, std::max(1, steps / pc / pc)); }
+static bool timed_step(int istep, int pc, int every) {
     const int cycle = istep / pc;
-    return cycle % 4 == 0 && istep % pc == cycle / 4 % pc;
+    return cycle % every == 0 && istep % pc == cycle / every % pc;
 }
 
 int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pending, bte_frame_cb cb,
@@ -2316,7 +2318,7 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
     const int emit_blocks = b->emit_blocks;
     // one propagator table and no RTA scattering: the P1 particle kernels
     const int p1 = (!b->cfg.rta && P.nslots == 1) ? 1 : 0;
-    const int pc = b->cfg.pcancel_each;
+    const int pc = b->cfg.pcancel_each, every = timed_every(b->max_steps, pc);
     StepKernel step_k = b->g->poly ? step_kernel_poly_tab[b->periodic][p1] : step_kernel_tab[b->geo_lds][b->periodic][p1];
     EmitKernel emit_k = b->g->poly ? emit_kernel_poly_tab[b->periodic][p1] : emit_kernel_tab[b->geo_lds][b->periodic][p1];
     if (b->vl) {
@@ -2348,7 +2350,7 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
         // the (box, mode) histogram is built only where a cancellation or a
         // frame reads it; properties come from the box sums otherwise
         const int hist = cancel_now || cb != nullptr || !P.lds_props;
-        const bool timed = timed_step(istep, pc);
+        const bool timed = timed_step(istep, pc, every);
         if (timed) HIPCHECK(hipEventRecord(b->kev[2 * istep], s));
         hipLaunchKernelGGL(step_k, dim3(step_blocks), dim3(b->vl ? 1024 : 256), b->vl ? b->lds_vl_bytes : b->lds_bytes,
                            s, P, (uint32_t)istep, cur, cancel_prev, hist);
@@ -2397,7 +2399,7 @@ int bte_bert_execute(bte_bert* bb, double* props, int64_t* npart, int64_t* pendi
     std::vector<int> place_n(nplace, 0);
     int ktimed = 0, places = 0;
     for (int i = 0; i < istep; i++) {
-        if (!timed_step(i, pc)) continue;
+        if (!timed_step(i, pc, every)) continue;
         float e = 0;
         HIPCHECK(hipEventElapsedTime(&e, b->kev[2 * i], b->kev[2 * i + 1]));
         place_ms[i % pc] += e;

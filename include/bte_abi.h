@@ -338,11 +338,13 @@ typedef struct {
     int64_t max_particles;
     double loop_ms;           /* wall time of the step loop (device-synchronised) */
     double step_kernel_ms;    /* step_kernel_timed times their mean device time (each place of the
-                               * cancellation cycle with the same weight) */
+                               * cancellation cycle that was timed with the same weight) */
     int step_kernel_launches;
-    /* launches bracketed by events: one in every fourth cancellation cycle
-     * (of pcancel_each steps), at each place of the cycle in turn (an event
-     * pair costs about 11 us of idle device time) */
+    /* launches bracketed by events, at each place of the cancellation cycle
+     * (of pcancel_each steps) in turn: one in every fourth cycle, or in every
+     * third to every one where the steps are fewer than 4 pcancel_each^2 (an
+     * event pair costs about 11 us of idle device time); with fewer steps
+     * than pcancel_each^2 the last places are not timed */
     int step_kernel_timed;
     int step_threads;         /* threads per step-kernel workgroup: 1024 with the
                                  mode velocities in LDS, else 256 */

@@ -198,3 +198,20 @@ def test_a_given_capacity_holds_with_a_large_source(pkg, ctx):
     assert n0 > 1900000 and a["npart"].max() == n0 and a["step_threads"] == 1024
     c = run(capacity=int(0.95 * n0 / 256 * (256 + 256 + 98)))
     assert np.array_equal(a["npart"], c["npart"]) and np.array_equal(a["pending"], c["pending"])
+
+
+@pytest.mark.parametrize("pc,steps,timed", [(4, 16, 4), (4, 15, 3), (4, 100, 7), (1, 9, 3), (2, 8, 2), (6, 36, 6)])
+def test_timed_steps_reach_every_place_of_the_cycle(pkg, ctx, pc, steps, timed):
+    """One launch in every fourth cancellation cycle is timed, at each place
+    of the cycle in turn, and more closely together where the run has fewer
+    than 4 pc^2 steps: from pc^2 steps on, every place has its launch."""
+    W = pkg.workloads
+    mat = W.material(60, seed=5)
+    rect, kind, teq, tin = W.ribbon(60.0, 30.0, 6, 300.0, Tinit_first=302.0)
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    geom = pkg.Geometry(ctx, rect, kind, teq, tin)
+    b = pkg.BertRun(ctx, modes, geom, None, thickness=1.0, dt=4.0, maxtime=4.0 * (steps - 1), max_steps=steps,
+                    rta=True, Efactor=4000, Tmax=302.0, Tmin=300.0, seed=3, pcancel_each=pc)
+    r = b.execute()
+    b.close()
+    assert r["nsteps"] == steps and r["step_kernel_timed"] == timed and r["step_kernel_ms"] > 0
