@@ -2050,10 +2050,11 @@ static void batch_set_tally(RtaBatch* b, int mode) {
                                         " bytes of LDS for one time bin, the device has " +
                                         std::to_string(b->ctx->lds_per_block) + " per workgroup");
         allow_lds(rta_kernel(2, false, b->poly, L.gl), b->ctx->lds_per_block);
-        // two 768-thread workgroups per CU when two blocks fit its LDS (small
-        // geometries), else one
+        // one 768-thread workgroup per CU, also where two blocks fit its LDS:
+        // the kernels' 139 registers leave each SIMD three waves, so a second
+        // one would begin when the first has ended and the ids are gone
         b->block = 768;
-        b->blocks = b->ctx->cu_count * (2 * L.bytes <= b->ctx->lds_per_block ? 2 : 1);
+        b->blocks = b->ctx->cu_count;
         const size_t np = (size_t)b->blocks * 3 * b->lrows * L.lbins;
         if (b->d_part.n < np) b->d_part.alloc(np);  // kept: a captured graph holds its address
     } else if (mode == 1) {

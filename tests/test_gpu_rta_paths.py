@@ -174,3 +174,18 @@ def test_lambert_window_without_partner(pkg, ctx):
     with pytest.raises(pkg.BteError, match="mode 0 has no diffuse partner within the Lambert window"):
         pkg.RtaBatch(ctx, modes, [dict(geom=_ribbon(pkg, ctx, 6), T0=300.0, nparticles=100, seed=2)],
                      **dict(KW, sigma_bounce=1e-9))
+
+
+@pytest.mark.parametrize("nb", [8, 249])
+def test_fp64_lds_tallies_launch_what_runs_at_a_time(pkg, ctx, nb):
+    """One 768-thread workgroup per CU, whether one tally block or two fit its
+    LDS (the device atomics' launch is eight 256-thread workgroups per CU)."""
+    run = dict(geom=_ribbon(pkg, ctx, nb), T0=300.0, nparticles=30000, seed=5)
+    reps = []
+    for tally in ("fp64", "fp64-lds"):
+        b = pkg.RtaBatch(ctx, _modes(pkg, ctx), [run], tally=tally, **KW)
+        reps.append(b.execute()[1])
+        b.close()
+    assert reps[0]["block"] == 256 and reps[1]["block"] == 768
+    assert reps[1]["blocks"] == reps[0]["blocks"] // 8
+    assert reps[1]["events"] == reps[0]["events"]
