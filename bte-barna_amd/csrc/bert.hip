@@ -1167,7 +1167,9 @@ __global__ __launch_bounds__(256) void bert_wallcdf_kernel(BertParams P, uint32_
 // advected U*dt, scattered and histogrammed. 512-thread workgroups (two per
 // CU) keep four waves per SIMD resident with one output segment per
 // workgroup: 256-thread ones left two (and more segments slow the step
-// kernel's segment walk).
+// kernel's segment walk). With periodic boxes the kernels take 142 to 171
+// registers (119 with polygons under P1): one workgroup per CU runs at a time,
+// the others follow.
 #define BERT_EMIT_MAXB 4096
 #define BERT_EMIT_THREADS 512
 // VL: as in the step kernel, one 1024-thread workgroup per CU with the mode
@@ -1301,6 +1303,8 @@ struct BertSource {
 #define BERT_SRC_PART_WIDE 1024.0
 // population that the automatic buffers hold with sources: 0.7 x 2^25
 #define BERT_STEADY ((uint64_t)(0.7 * (1ull << 25)))
+// At most one source workgroup per CU runs, one wave per SIMD: the 118 to 178
+// registers of the instantiations limit nothing.
 template <bool GL, bool PER, bool POLY>
 __global__ __launch_bounds__(256) void bert_source_kernel(BertParams P, const BertSource* src, int nparts_all,
                                                           const uint2* stab, uint32_t step, int cur, int hist) {
