@@ -2045,8 +2045,9 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
     // 512-thread emission workgroups
     if (cfg->step_shape < 0 || cfg->step_shape > 1) throw Error(BTE_EINVAL, "step_shape must be 0 or 1");
     // boxes in LDS (polygon kernels read the geometry globally)
-    b->geo_lds = !g->poly && (size_t)BERT_BOX_LDS * nbox + sizeof(DevPer) * g->per.size() +
-                                     sizeof(DevCross) * g->tcross.size() <= BERT_GEO_LDS_BYTES;
+    const bool boxes_fit = !g->poly && (size_t)BERT_BOX_LDS * nbox + sizeof(DevPer) * g->per.size() +
+                                               sizeof(DevCross) * g->tcross.size() <= BERT_GEO_LDS_BYTES;
+    b->geo_lds = boxes_fit;
     b->vl = !b->periodic && cfg->step_shape == 0;
     if (b->vl) {
         b->step_blocks = std::min(c->cu_count, BERT_MAXSEG - 512 - BERT_SRC_BLOCKS);
@@ -2060,6 +2061,17 @@ int bte_bert_create(bte_ctx* ctx, const bte_modes* mm, const bte_geom* gg, const
             (void)make_params(b);
             b->vl = b->lds_vl_bytes + 1024 <= c->lds_per_block;
             b->geo_lds = !b->vl;
+        }
+        // A VL workgroup's segment takes 1/256 of the particles in 512 or more
+        // segments, a 256-thread one's 1/1024 or 1/1280 in 1536 or 1792: up to
+        // 2 against 1.4 times the particles. In a capacity that the caller
+        // gives, the tables displace no boxes beyond their padding in LDS.
+        const size_t unpadded = sizeof(DevBox) * (size_t)nbox;
+        if (b->vl && !b->geo_lds && cfg->capacity && !g->poly &&
+            unpadded + sizeof(DevContact) * g->dcontacts.size() <= BERT_GEO_LDS_BYTES &&
+            b->lds_vl_bytes + unpadded + 1024 > c->lds_per_block) {
+            b->vl = false;
+            b->geo_lds = boxes_fit;
         }
     }
     if (!b->vl) {

@@ -215,3 +215,32 @@ def test_timed_steps_reach_every_place_of_the_cycle(pkg, ctx, pc, steps, timed):
     r = b.execute()
     b.close()
     assert r["nsteps"] == steps and r["step_kernel_timed"] == timed and r["step_kernel_ms"] > 0
+
+
+@pytest.mark.parametrize("nmodes,threads", [(400, 1024), (4500, 256)])
+def test_a_given_capacity_holds_where_velocities_displace_boxes(pkg, ctx, nmodes, threads):
+    """4500 modes and 200 boxes do not fit the LDS together. The velocity
+    tables alone would, in workgroups whose segments (256 beside 256 of the
+    emission) need twice the particles as capacity; those of 256 threads
+    (1024 beside 512) need 1.5 times, and a capacity of 1.65 times the
+    particles is enough as a tenth of them wait at a wall. 400 modes fit beside
+    the boxes, and 2.1 times the particles are given."""
+    W = pkg.workloads
+    mat = W.material(nmodes, seed=5)
+    rect = np.array([[k * 10.0, (k + 1) * 10.0, r * 200.0, r * 200.0 + 100.0] for r in range(4) for k in range(50)])
+    modes = pkg.ModeTable(ctx, mat["omega"], mat["vx"], mat["vy"], mat["w"], mat["V"], mat["lattz"])
+    geom = pkg.Geometry(ctx, rect, np.zeros(200, np.int32), np.full(200, 300.0), np.full(200, 302.0))
+
+    def run(**kw):
+        b = pkg.BertRun(ctx, modes, geom, None, thickness=1.0, dt=4.0, maxtime=8.0, rta=True, Efactor=5000,
+                        Tmax=302.0, Tmin=300.0, seed=3, pcancel_each=1000, **kw)
+        r = b.execute()
+        b.close()
+        return r
+
+    a = run()
+    n0 = int(a["npart"][0])
+    assert n0 > 900000 and a["step_threads"] == 1024
+    c = run(capacity=int((2.1 if threads == 1024 else 1.65) * n0))
+    assert c["step_threads"] == threads
+    assert np.array_equal(a["npart"], c["npart"]) and np.array_equal(a["pending"], c["pending"])
