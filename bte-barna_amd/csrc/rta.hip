@@ -1300,7 +1300,7 @@ struct RtaLambert {
     const double *omega, *vx, *vy;
     const double2* normals;
     const double* e;    // per pair from mode i0 on: the pdf's exponential, 0 outside the cut
-    const double* pre;  // its factor 1 / (sigma sqrt(2 pi)) with per-mode sigma, else null
+    const double* pre;  // its factor 1 / (sigma sqrt(2 pi)), 0 outside the cut, with per-mode sigma, else null
     double* q;          // scratch: scaled weights and the two stacks, per entry
     int32_t* list;
     uint2* tab;
@@ -1449,7 +1449,8 @@ static void build_lambert(const Modes& m, double sigma, const std::vector<double
                 const bool ok = !almost_equal(0., m.omega[f]) && d <= nsig * sig;
                 e.push_back(ok ? std::exp(-0.5 * d * d / (sig * sig)) : 0.);
                 // the pdf's 1 / (sig sqrt(2 pi)) differs between pairs only with per-mode sigma
-                if (own) pre.push_back(1.0 / (sig * rt2pi));
+                // (a pair of weight 0 may have width 0)
+                if (own) pre.push_back(ok ? 1.0 / (sig * rt2pi) : 0.);
             }
             part += nn * info[i1].y;
         }

@@ -189,3 +189,27 @@ def test_fp64_lds_tallies_launch_what_runs_at_a_time(pkg, ctx, nb):
     assert reps[0]["block"] == 256 and reps[1]["block"] == 768
     assert reps[1]["blocks"] == reps[0]["blocks"] // 8
     assert reps[1]["events"] == reps[0]["events"]
+
+
+def test_diffuse_partners_without_broadening_or_frequency(pkg, ctx):
+    """Three of eight modes at zero frequency and with a per-mode broadening
+    of 0 (a quarter of the modes: the broadening's floor is 0 too). They are
+    nobody's diffuse partner, so the width of their pairs, 0, enters no
+    table, and the other five scatter at the walls as without them."""
+    omega = np.array([0.0, 0.0, 0.0, 10.0, 10.0, 10.1, 10.1, 10.2])
+    v = np.array([[1.0, 0.5], [-1.0, 0.5], [0.5, -1.0], [2.0, 2.0], [-2.0, -2.0], [2.0, -2.0], [-2.0, 2.0], [1.0, 1.5]])
+    modes = pkg.ModeTable(ctx, omega, v[:, 0], v[:, 1], np.full(8, 0.1), 1.0, 1.0)
+    modes.set_sigma(np.array([0.0] * 3 + [0.5] * 5))
+    five = pkg.ModeTable(ctx, omega[3:], v[3:, 0], v[3:, 1], np.full(5, 0.1), 1.0, 1.0)
+    five.set_sigma(np.full(5, 0.5))
+    out = []
+    for m in (modes, five):
+        run = pkg.RtaRun(ctx, m, _ribbon(pkg, ctx, 4, width=10.0), thickness=1.0, T0=300.0, dt=10.0, maxtime=100.0,
+                         nparticles=2000, seed=3)
+        out.append(run.execute())
+        run.close()
+    for o in out:
+        assert o["events"] > 2000 and np.isfinite(o["T"]).all()
+    # a history has a few tens of events at most (10 scatterings and 20 walls
+    # on average for one that stays), so their number varies by less than its mean
+    assert abs(out[0]["events"] / out[1]["events"] - 1.0) < 5.0 * np.sqrt(2.0 / 2000)
